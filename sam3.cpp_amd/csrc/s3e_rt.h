@@ -29,6 +29,11 @@ struct s3e_ctx {
     // s3e_flash_attn_ext_f16's operand copies and key-split partials
     void *attn_ws = nullptr;
     size_t attn_ws_cap = 0;
+    // converted operands of s3e_mul_mat and s3e_flash_attn_ext (CallWs), held
+    // by one call at a time: both synchronise before they return
+    std::mutex call_mu;
+    void *call_ws = nullptr;
+    size_t call_ws_cap = 0;
     // the measurement kernels' output words (made at first use)
     uint32_t *probe_sink = nullptr;
     int64_t probe_sink_cap = 0;
@@ -57,6 +62,30 @@ int upload_weight(int device, int type, int64_t K, int64_t N, const uint8_t *src
                   int64_t npad = GEMM_BN);
 // f32 weights as the two fp16 planes of WK_F16X3, N padded to npad.
 int upload_weight_split(const float *src, int64_t K, int64_t N, Weight &w, int64_t npad);
+
+// Device memory for the converted operands of one call that synchronises
+// before it returns: the context's call workspace, grown when a call needs more
+// than every earlier one and freed with the context.  Above CALL_WS_MAX the
+// memory is the call's own, freed when it ends.  Allocating and freeing per
+// call (each hipFree waits for the device) and clearing the scale planes took
+// more than the kernels: at 5184 × 3072 × 1024 F16 105 → 69 µs a call, at
+// 7 × 1024 × 1024 Q4_0 28.6 → 21.4 µs, windowed f32 attention (9 × 16 × 576²)
+// 526 → 184 µs.  A second caller on the context waits for the
+// first call to end.
+constexpr size_t CALL_WS_MAX = (size_t)1 << 30;
+class CallWs {
+public:
+    explicit CallWs(s3e_ctx *ctx) : ctx_(ctx), lock_(ctx->call_mu) {}
+    ~CallWs() { if (own_) (void)hipFree(own_); }
+    CallWs(const CallWs &) = delete;
+    CallWs &operator=(const CallWs &) = delete;
+    hipError_t get(size_t bytes, void **out);
+
+private:
+    s3e_ctx *ctx_;
+    std::lock_guard<std::mutex> lock_;
+    void *own_ = nullptr;
+};
 
 // A tensor record as read from a model file.
 struct RawTensor {

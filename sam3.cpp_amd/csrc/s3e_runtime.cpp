@@ -316,6 +316,7 @@ extern "C" void s3e_ctx_destroy(s3e_ctx *ctx) {
     if (ctx->sm_dev) (void)hipFree(ctx->sm_dev);
     if (ctx->sk_part) (void)hipFree(ctx->sk_part);
     if (ctx->attn_ws) (void)hipFree(ctx->attn_ws);
+    if (ctx->call_ws) (void)hipFree(ctx->call_ws);
     if (ctx->probe_sink) (void)hipFree(ctx->probe_sink);
     delete ctx;
 }
@@ -487,6 +488,36 @@ hipError_t sk_workspace(s3e_ctx *ctx, int64_t parts) {
     return hipSuccess;
 }
 
+}  // namespace
+
+hipError_t s3e::CallWs::get(size_t bytes, void **out) {
+    *out = nullptr;
+    if (bytes > CALL_WS_MAX) {
+        const hipError_t e = hipMalloc(&own_, bytes);
+        if (e == hipSuccess) *out = own_;
+        else own_ = nullptr;
+        return e;
+    }
+    if (bytes > ctx_->call_ws_cap) {
+        // a call that failed half way may have left work behind
+        hipError_t e = hipStreamSynchronize(ctx_->stream);
+        if (e != hipSuccess) return e;
+        if (ctx_->call_ws) (void)hipFree(ctx_->call_ws);
+        ctx_->call_ws = nullptr;
+        ctx_->call_ws_cap = 0;
+        e = hipMalloc(&ctx_->call_ws, bytes);
+        if (e != hipSuccess) {
+            ctx_->call_ws = nullptr;
+            return e;
+        }
+        ctx_->call_ws_cap = bytes;
+    }
+    *out = ctx_->call_ws;
+    return hipSuccess;
+}
+
+namespace {
+
 hipError_t run_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const Act &a, int64_t M, const EpiArgs &ea) {
     const Weight &W = w->w;
     hipStream_t st = ctx->stream;
@@ -583,13 +614,27 @@ extern "C" int s3e_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const float *X, in
         HIP_TRY(launch_gemm(W, a, M, EPI_F32, ea, ctx->stream));
         return S3E_OK;
     }
-    ActBuf buf;
-    HIP_TRY(buf.alloc(std::max<int64_t>(M, 64), W.K, ctx->stream));
-    const Act a = buf.as(sm_eligible(W, M) ? ak : act_kind_gemm(W), W.K);
-    hipError_t e = launch_rows_quant(a.kind, X, M, W.K, a, ctx->stream);
+    // [values of X in the product's format][d][s (Q8_1)].  Rows past M of the
+    // values and scale planes are never written: they only reach output rows
+    // past M, which no kernel stores.
+    Act a;
+    a.kind = sm_eligible(W, M) ? ak : act_kind_gemm(W);
+    a.ld = W.K;
+    a.mp = round_up(M, ROW_PAD);
+    const bool f16 = a.kind == A_F16;
+    const size_t vb = (size_t)(a.mp * W.K) * (f16 ? 4 : 3) / 2;  // fp6 pairs take 1.5 bytes, Q8 codes 1
+    const size_t sb = f16 ? 0 : (size_t)(a.mp * (round_up(W.K, 128) / QK)) * 2;
+    CallWs ws(ctx);
+    void *base = nullptr;
+    hipError_t e = ws.get(vb + 2 * sb, &base);
+    if (e == hipSuccess) {
+        a.x = base;
+        a.d = (uint16_t *)((uint8_t *)base + vb);
+        a.s = (uint16_t *)((uint8_t *)base + vb + sb);
+        e = launch_rows_quant(a.kind, X, M, W.K, a, ctx->stream);
+    }
     if (e == hipSuccess) e = run_mul_mat(ctx, w, a, M, ea);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    buf.release();
     if (e != hipSuccess) { set_error("s3e_mul_mat: %s", hipGetErrorString(e)); return S3E_ERR_HIP; }
     return S3E_OK;
 } S3E_CATCH("s3e_mul_mat")
@@ -762,14 +807,14 @@ extern "C" int s3e_flash_attn_ext(s3e_ctx *ctx, const float *q, const int64_t q_
         const int64_t per = (ktiles + ns - 1) / ns;
         nsplit = (int)((ktiles + per - 1) / per);
     }
-    _Float16 *q16 = nullptr, *k16 = nullptr, *vt16 = nullptr;
-    float *part = nullptr;
-    hipError_t e = hipMalloc(&q16, qn * 2 * np);
-    if (e == hipSuccess) e = hipMalloc(&k16, kn * 2 * np);
-    if (e == hipSuccess) e = hipMalloc(&vt16, vn * 2 * np);
-    if (e == hipSuccess) e = hipMemsetAsync(vt16, 0, vn * 2 * np, ctx->stream);
     const size_t po = (size_t)nsplit * BH * Nq * hdp, pml = (size_t)nsplit * BH * Nq * 2;
-    if (e == hipSuccess && nsplit > 1) e = hipMalloc(&part, (po + pml) * 4);
+    // [Q][K][Vᵀ][partials]; every plane is a multiple of 128 bytes
+    CallWs ws(ctx);
+    void *base = nullptr;
+    hipError_t e = ws.get((qn + kn + vn) * 2 * np + (nsplit > 1 ? (po + pml) * 4 : 0), &base);
+    _Float16 *q16 = (_Float16 *)base, *k16 = q16 + qn * np, *vt16 = k16 + kn * np;
+    float *part = (float *)(vt16 + vn * np);
+    if (e == hipSuccess) e = hipMemsetAsync(vt16, 0, vn * 2 * np, ctx->stream);
     AttnArgs a;
     a.q = q16;
     a.k = k16;
@@ -802,10 +847,6 @@ extern "C" int s3e_flash_attn_ext(s3e_ctx *ctx, const float *q, const int64_t q_
         e = launch_attn(a, ctx->stream);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (q16) (void)hipFree(q16);
-    if (k16) (void)hipFree(k16);
-    if (vt16) (void)hipFree(vt16);
-    if (part) (void)hipFree(part);
     if (e != hipSuccess) { set_error("s3e_flash_attn_ext: %s", hipGetErrorString(e)); return S3E_ERR_HIP; }
     return S3E_OK;
 } S3E_CATCH("s3e_flash_attn_ext")
