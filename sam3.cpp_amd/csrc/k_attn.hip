@@ -15,10 +15,16 @@
 // registers straight into the B operand (fp16) with no data movement, and the
 // keys of each K=16 MFMA step are the ones that lane already holds; thanks to
 // the vt_slot order the matching Vᵀ A-operand is one 16-byte LDS read.
-// The VN variant (fp16 operands, head dims 64 / 128) reads V as ggml holds
-// it, [BH][Nkv][hd]: its tiles are laid out like K tiles, and each Vᵀ
-// A-operand is two LDS transpose loads (ds_read_b64_tr_b16), which hand every
-// lane one channel of four keys.
+// The VN variants (the flash_attn_ext entry points) read V as ggml holds it,
+// rows of keys: its tiles are laid out like K tiles, and each Vᵀ A-operand is
+// two LDS transpose loads (ds_read_b64_tr_b16), which hand every lane one
+// channel of four keys.  They take Q by strides, fp16 or f32 (converted once
+// per work-group, in registers), and K and V by strides too, so tensors that
+// already are fp16 are read where they lie: a head narrower than hd is padded
+// by chunk offsets past the buffer descriptor's record count, which load as
+// zeros.  Head dim 256 takes Q and K so, but V as Vᵀ: its one wave per SIMD
+// does not hide the two LDS instructions per operand (4096 queries × 28736
+// keys: 219 µs against 172 µs, more than the transposing pass).
 //
 // K and Vᵀ tiles of 32 keys stream through a 2-deep LDS ring filled by
 // buffer_load_dwordx4 ... lds (rows of 128 bytes, 16-byte chunks
@@ -137,11 +143,12 @@ __device__ __forceinline__ float sub_hi_half(float p, uint32_t h2) {
 
 // CROP: the windowed, cropped output mapping and narrower real heads
 // (a.wo, a.hd_out; the Hiera layouts), kept out of the plain variants.
-template <bool SPLIT, int HD, bool CROP, bool VN = false>
+// STR: Q and K (and V, VN) by strides.
+template <bool SPLIT, int HD, bool CROP, bool VN = false, bool STR = VN>
 __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_attn(AttnArgs a, int ldv) {
-    static_assert(!VN || (!SPLIT && HD <= 128), "natural V: fp16 operands, head dim 64 or 128");
     using G = AG<HD>;
     constexpr int NP = SPLIT ? 2 : 1;  // planes: hi (and lo)
+    static_assert(VN ? STR && HD <= 128 : !STR || HD == 256, "natural V at head dim 64 or 128, by strides");
     constexpr int KPL = G::KPL, VPL = G::VPL;
     constexpr int KBUF = NP * KPL, VBUF = NP * VPL;
     // K ring (2 tiles) then Vᵀ ring (2 tiles)
@@ -155,7 +162,48 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
     const bool qvalid = qi < a.Nq;
 
     v8h qf[NP][G::DS];
-    {
+    if constexpr (STR) {
+        const int64_t off = (int64_t)(bh / a.NH) * a.qs[2] + (int64_t)(bh % a.NH) * a.qs[1] +
+                            (int64_t)(qvalid ? qi : 0) * a.qs[0];
+        const int dr = a.hd_out > 0 ? a.hd_out : HD;
+#pragma unroll
+        for (int ds = 0; ds < G::DS; ds++) {
+            const int d0 = ds * 16 + lh * 8;
+            if (a.q32) {
+                // (the head dim is a multiple of 4: four channels are all real or all padding)
+                float x[8];
+#pragma unroll
+                for (int h4 = 0; h4 < 8; h4 += 4) {
+                    const float *src = a.q32 + off + d0 + h4;
+                    const bool in = qvalid && d0 + h4 < dr;
+                    if (a.q_vec) {
+                        const float4 f = in ? *(const float4 *)src : make_float4(0.f, 0.f, 0.f, 0.f);
+                        x[h4] = f.x; x[h4 + 1] = f.y; x[h4 + 2] = f.z; x[h4 + 3] = f.w;
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) x[h4 + i] = in ? src[i] : 0.f;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const _Float16 hv = to_half(x[i]);
+                    qf[0][ds][i] = hv;
+                    if constexpr (SPLIT) qf[NP - 1][ds][i] = (_Float16)(x[i] - (float)hv);
+                }
+            } else if constexpr (!SPLIT) {
+                const _Float16 *src = a.q + off + d0;
+                v8h z = {};
+                if (a.q_vec) {
+                    if (qvalid && d0 < dr) z = *(const v8h *)src;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; i++)
+                        if (qvalid && d0 + i < dr) z[i] = src[i];
+                }
+                qf[0][ds] = z;
+            }
+        }
+    } else {
         const int64_t off = (int64_t)bh * (a.q_hs > 0 ? a.q_hs : (int64_t)a.Nq * HD) + (int64_t)(qvalid ? qi : 0) * HD;
 #pragma unroll
         for (int pl = 0; pl < NP; pl++) {
@@ -175,7 +223,19 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
 #pragma unroll
         for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
 
-    const int64_t koff = (int64_t)bh * a.Nkv * HD, voff = (int64_t)bh * HD * ldv;
+    int64_t koff = (int64_t)bh * a.Nkv * HD, voff = (int64_t)bh * HD * ldv;
+    // bytes from one K (V) row to the next, and of a row's real channels
+    int k_rb = G::ROWK, v_rb = G::ROWK, real = G::ROWK;
+    if constexpr (STR) {
+        const int b = bh / a.NH, h = bh % a.NH;
+        koff = b * a.ks[2] + h * a.ks[1];
+        k_rb = (int)a.ks[0] * 2;
+        real = a.kv_d * 2;
+        if constexpr (VN) {
+            voff = b * a.vs[2] + h * a.vs[1];
+            v_rb = (int)a.vs[0] * 2;
+        }
+    }
     // key tiles of this work-group: all, or with nsplit > 1 the blockIdx.z-th
     // of nsplit consecutive ranges (each holds at least one tile)
     const int ntiles_all = (a.Nkv + KT - 1) / KT;
@@ -200,13 +260,17 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
             __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)nrec, 0x00020000);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, LDS_PTR(ldsp), 16, lane_off, 0, 0, 0);
     };
+    // STR: chunks past a row's real channels load zeros (the launcher keeps
+    // every tile's record count below this offset)
+    constexpr int PAST = 1 << 30;
     int k_lane[G::KRUNS], v_lane[G::VRUNS];
 #pragma unroll
     for (int j = 0; j < G::KRUNS; j++) {
         constexpr int RPR = 1024 / G::ROWK;      // rows per run
         constexpr int CPR = G::ROWK / 16;        // chunks per row
         const int r = RPR * (wave * G::KRUNS + j) + lane / CPR;
-        k_lane[j] = r * G::ROWK + (((lane % CPR) ^ swzk_hd<HD>(r)) << 4);
+        const int ch = ((lane % CPR) ^ swzk_hd<HD>(r)) << 4;
+        k_lane[j] = STR && ch >= real ? PAST : r * k_rb + ch;
     }
     int vn_lane[G::KRUNS];  // VN: V tiles as K tiles, own swizzle
 #pragma unroll
@@ -214,7 +278,8 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         constexpr int RPR = 1024 / G::ROWK;
         constexpr int CPR = G::ROWK / 16;
         const int r = RPR * (wave * G::KRUNS + j) + lane / CPR;
-        vn_lane[j] = r * G::ROWK + (((lane % CPR) ^ swzvn<HD>(r)) << 4);
+        const int ch = ((lane % CPR) ^ swzvn<HD>(r)) << 4;
+        vn_lane[j] = ch >= real ? PAST : r * v_rb + ch;
     }
     int v_row[G::VRUNS], v_ch[G::VRUNS];
 #pragma unroll
@@ -227,10 +292,10 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
     auto issue_k = [&](int tt) {
         uint8_t *L = Kring + (tt & 1) * KBUF;
         const int tile = t0 + tt;
-        const uint32_t nrec = (uint32_t)min(a.Nkv - tile * KT, KT) * G::ROWK;
+        const uint32_t nrec = (uint32_t)(min(a.Nkv - tile * KT, KT) - 1) * k_rb + real;
 #pragma unroll
         for (int pl = 0; pl < NP; pl++) {
-            const _Float16 *base = (pl == 0 ? a.k : a.k_lo) + koff + (int64_t)tile * KT * HD;
+            const _Float16 *base = (pl == 0 ? a.k : a.k_lo) + koff + (int64_t)tile * KT * (k_rb / 2);
 #pragma unroll
             for (int j = 0; j < G::KRUNS; j++) dma(base, nrec, L + pl * KPL + (wave * G::KRUNS + j) * 1024, k_lane[j]);
         }
@@ -240,10 +305,13 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         const int tile = t0 + tt;
         if constexpr (VN) {
             // rows past the keys read as zeros (their probabilities are 0)
-            const uint32_t nk = (uint32_t)min(a.Nkv - tile * KT, KT) * G::ROWK;
-            const _Float16 *base = a.v + koff + (int64_t)tile * KT * HD;
+            const uint32_t nk = (uint32_t)(min(a.Nkv - tile * KT, KT) - 1) * v_rb + real;
 #pragma unroll
-            for (int j = 0; j < G::KRUNS; j++) dma(base, nk, L + (wave * G::KRUNS + j) * 1024, vn_lane[j]);
+            for (int pl = 0; pl < NP; pl++) {
+                const _Float16 *base = (pl == 0 ? a.v : a.v_lo) + voff + (int64_t)tile * KT * (v_rb / 2);
+#pragma unroll
+                for (int j = 0; j < G::KRUNS; j++) dma(base, nk, L + pl * VPL + (wave * G::KRUNS + j) * 1024, vn_lane[j]);
+            }
             return;
         }
         const uint32_t nrec = (uint32_t)(HD * ldv - tile * KT) * 2;
@@ -299,8 +367,15 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
             for (int dt = 0; dt < G::DT; dt++)
 #pragma unroll
                 for (int jj = 0; jj < 2; jj++) {
-                    const v4h v0 = lds_tr16(L + tr_off(dt, jj, 0)), v1 = lds_tr16(L + tr_off(dt, jj, 1));
+                    const int o0 = tr_off(dt, jj, 0), o1 = tr_off(dt, jj, 1);
+                    const v4h v0 = lds_tr16(L + o0), v1 = lds_tr16(L + o1);
                     const v8h vh = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+                    if constexpr (SPLIT) {
+                        const v4h l0 = lds_tr16(L + VPL + o0), l1 = lds_tr16(L + VPL + o1);
+                        const v8h vl = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+                        o[dt] = mfma(vl, ph[jj], o[dt]);
+                        o[dt] = mfma(vh, pl[jj], o[dt]);
+                    }
                     o[dt] = mfma(vh, ph[jj], o[dt]);
                 }
             return;
@@ -668,14 +743,31 @@ hipError_t launch_attn(const AttnArgs &a, hipStream_t st) {
     if (a.out.kind == A_F16X2 && (!a.out.lo || a.out.ld % 4 != 0)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((a.Nq + QT - 1) / QT), (unsigned)a.BH, (unsigned)a.nsplit);
     const bool crop = a.wo > 0 || (a.hd_out > 0 && a.hd_out != hd);
+    if (a.kv_d != 0) {
+        // Q (fp16, or f32) and K by strides, and V where it is given by rows
+        const bool split = a.k_lo != nullptr;
+        if ((hd == 256) != (a.v == nullptr) || (hd == 256 && !a.vt) || (!a.q32 && !a.q)) return hipErrorInvalidValue;
+        if (split && (hd == 256 || !a.q32 || !a.v_lo)) return hipErrorInvalidValue;
+        if (a.kv_d < 0 || a.kv_d > hd || a.kv_d % 8 != 0) return hipErrorInvalidValue;
+        for (const int64_t *st3 : {a.ks, a.vs})
+            if (st3[0] < 0 || st3[0] > ATTN_MAX_ROW || st3[0] % 8 || st3[1] % 8 || st3[2] % 8) return hipErrorInvalidValue;
+        for (const void *ptr : {(const void *)a.k, (const void *)a.v, (const void *)a.k_lo, (const void *)a.v_lo})
+            if ((uintptr_t)ptr % 16 != 0) return hipErrorInvalidValue;
+    } else if (a.v || a.q32) {
+        return hipErrorInvalidValue;
+    }
     if (a.v) {
-        // natural V: fp16 operands, head dim 64 or 128
-        if (a.q_lo || a.k_lo || hd == 256) return hipErrorInvalidValue;
-        if (hd == 64 && !crop) hipLaunchKernelGGL((k_attn<false, 64, false, true>), grid, dim3(NTHR), 0, st, a, ldv);
+        if (a.k_lo) {
+            if (hd == 64 && !crop) hipLaunchKernelGGL((k_attn<true, 64, false, true>), grid, dim3(NTHR), 0, st, a, ldv);
+            else if (hd == 64) hipLaunchKernelGGL((k_attn<true, 64, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
+            else hipLaunchKernelGGL((k_attn<true, 128, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
+        } else if (hd == 64 && !crop) hipLaunchKernelGGL((k_attn<false, 64, false, true>), grid, dim3(NTHR), 0, st, a, ldv);
         else if (hd == 64) hipLaunchKernelGGL((k_attn<false, 64, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
         else hipLaunchKernelGGL((k_attn<false, 128, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
     } else if (hd == 256) {
-        hipLaunchKernelGGL((k_attn<false, 256, false>), grid, dim3(NTHR), 0, st, a, ldv);
+        // (the strided form costs the plain layouts 1.6 % of a memory-attention pass)
+        if (a.kv_d != 0) hipLaunchKernelGGL((k_attn<false, 256, false, false, true>), grid, dim3(NTHR), 0, st, a, ldv);
+        else hipLaunchKernelGGL((k_attn<false, 256, false>), grid, dim3(NTHR), 0, st, a, ldv);
     } else if (hd == 64 && !crop) {
         if (a.q_lo) hipLaunchKernelGGL((k_attn<true, 64, false>), grid, dim3(NTHR), 0, st, a, ldv);
         else hipLaunchKernelGGL((k_attn<false, 64, false>), grid, dim3(NTHR), 0, st, a, ldv);

@@ -418,67 +418,101 @@ __global__ void k_im2col(const float *__restrict__ chw, int img, int P, int64_t 
     }
 }
 
-// f32 strided Q/K/V (head dim D) → fp16 [BH][N][hdp] for Q and K,
-// [BH][hdp][ldt] for V (keys in vt_slot order), channels D..hdp−1 zero.
-// With lo != null the value is stored as the pair hi = fp16(v),
-// lo = fp16(v − hi) for split-precision attention.
-__global__ void k_attn_prep(const float *__restrict__ src, int64_t s1, int64_t s2, int64_t s3,
-                            int64_t N, int64_t nh, int64_t B, int D, int hdp, _Float16 *__restrict__ dst,
-                            _Float16 *__restrict__ lo, int64_t ldt, int transpose) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t total = B * nh * N * hdp;
-    if (idx >= total) return;
-    const int64_t d = idx % hdp;
-    const int64_t i = (idx / hdp) % N;
-    const int64_t h = (idx / (hdp * N)) % nh;
-    const int64_t b = idx / (hdp * N * nh);
-    const float v = d < D ? src[b * s3 + h * s2 + i * s1 + d] : 0.f;
-    const int64_t bh = b * nh + h;
-    const int64_t o = transpose ? (bh * hdp + d) * ldt + vt_slot(i) : (bh * N + i) * hdp + d;
-    const _Float16 hv = to_half(v);
-    dst[o] = hv;
-    if (lo) lo[o] = (_Float16)(v - (float)hv);
+// Strided K (blockIdx.z 0) and V (1) rows, f32 or fp16 with head dim D, to fp16
+// [BH][N][hdp], channels D..hdp−1 zero; f32 with lo planes as pairs hi =
+// fp16(v), lo = fp16(v − hi).  Bound by its traffic: one thread moves 8
+// channels (two or one 16-byte loads when VEC, 16-byte stores), blockIdx.y is
+// the (batch, head) pair, so no wide division.  K and V of 9 × 16 windows of
+// 576 tokens at head dim 64 with lo planes (85 MB): 17 µs (5 TB/s).  A thread
+// per element, Q converted too and V scattered into Vᵀ two bytes at a time
+// made the whole call 184 µs; it now takes 79, 50 of them the attention kernel.
+struct PrepRows {
+    const void *src[2];
+    int64_t s1[2], s2[2], s3[2];
+    _Float16 *hi[2], *lo[2];
+};
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void k_attn_prep(PrepRows p, int N, int nh, int D, int lg) {
+    const int z = blockIdx.z, bh = blockIdx.y;
+    if (!p.hi[z]) return;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t row = idx >> lg;
+    if (row >= N) return;
+    const int d0 = (int)(idx & ((1 << lg) - 1)) * 8;
+    const T *src = (const T *)p.src[z] + (int64_t)(bh / nh) * p.s3[z] + (int64_t)(bh % nh) * p.s2[z] + row * p.s1[z] + d0;
+    _Float16 h[8], l[8];
+    if constexpr (sizeof(T) == 2) {
+        if (VEC && d0 + 8 <= D) {
+            *(uint4 *)h = *(const uint4 *)src;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; i++) h[i] = d0 + i < D ? (_Float16)src[i] : (_Float16)0.f;
+        }
+    } else {
+        float x[8];
+#pragma unroll
+        for (int i = 0; i < 8; i += 4) {
+            // (D % 4 == 0: four channels are all real or all padding)
+            if (VEC && d0 + i < D) {
+                const float4 f = *(const float4 *)(src + i);
+                x[i] = f.x; x[i + 1] = f.y; x[i + 2] = f.z; x[i + 3] = f.w;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) x[i + j] = d0 + i < D ? (float)src[i + j] : 0.f;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            h[i] = to_half(x[i]);
+            l[i] = (_Float16)(x[i] - (float)h[i]);
+        }
+    }
+    const int64_t o = ((((int64_t)bh * N + row) << lg) << 3) + d0;
+    *(uint4 *)(p.hi[z] + o) = *(const uint4 *)h;
+    if (sizeof(T) == 4 && p.lo[z]) *(uint4 *)(p.lo[z] + o) = *(const uint4 *)l;
 }
 
-// fp16 strided rows (head dim D) → fp16 [BH][N][hdp], channels D..hdp−1 zero
-// (Q or K of s3e_flash_attn_ext_f16 when they are not already in that
-// layout).  One thread per output element.
-__global__ void k_attn_prep16(const _Float16 *__restrict__ src, int64_t s1, int64_t s2, int64_t s3, int64_t N,
-                              int64_t nh, int64_t B, int D, int hdp, _Float16 *__restrict__ dst) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= B * nh * N * hdp) return;
-    const int64_t d = idx % hdp, i = (idx / hdp) % N, h = (idx / (hdp * N)) % nh, b = idx / (hdp * N * nh);
-    dst[idx] = d < D ? src[b * s3 + h * s2 + i * s1 + d] : (_Float16)0.f;
-}
-
-// fp16 V (key j of head h of batch b at v[b*s3 + h*s2 + j*s1 + d]) → Vᵀ
-// [BH][hdp][ldv], keys in vt_slot order, zero past Nkv and for d ≥ D.  One
-// thread per 8 slots × 8 channels: it reads the 8 keys those slots hold (16
-// bytes of channels each; VEC: one 16-byte load per key, else element by
-// element) and writes the 8 channel rows' 16-byte runs, transposing in
-// registers.  Slots 8c .. 8c + 7 of a 16-key group hold keys {0-3, 8-11}
-// (c even) or {4-7, 12-15} (c odd) of it.
-template <bool VEC>
-__global__ __launch_bounds__(256) void k_vt16(const _Float16 *__restrict__ v, int64_t s1, int64_t s2, int64_t s3,
-                                              int64_t Nkv, int64_t nh, int D, int hdp, int64_t ldv,
-                                              _Float16 *__restrict__ vt, int64_t total) {
+// V of head dim 256 (key j of head h of batch b at v[b*s3 + h*s2 + j*s1 + d]) →
+// Vᵀ [BH][256][ldv] fp16, keys in vt_slot order, zero past Nkv.  One thread per
+// 8 slots × 8 channels: it reads the 8 keys those slots hold (VEC: 16-byte
+// loads; else element by element) and writes the 8 channel rows' 16-byte
+// runs, transposing in registers.  Slots 8c .. 8c + 7 of a 16-key group hold
+// keys {0-3, 8-11} (c even) or {4-7, 12-15} (c odd) of it.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void k_vt(const T *__restrict__ v, int64_t s1, int64_t s2, int64_t s3, int64_t Nkv,
+                                            int64_t nh, int64_t ldv, _Float16 *__restrict__ vt, int64_t total) {
+    constexpr int HD = 256, DCH = HD / 8;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= total) return;
-    const int dch = hdp / 8;
     const int64_t nsc = ldv / 8;
-    const int d0 = (int)(t % dch) * 8;
-    const int64_t sc = (t / dch) % nsc, bh = t / (dch * nsc);
-    const _Float16 *vb = v + (bh / nh) * s3 + (bh % nh) * s2;
+    const int d0 = (int)(t % DCH) * 8;
+    const int64_t sc = (t / DCH) % nsc, bh = t / (DCH * nsc);
+    const T *vb = v + (bh / nh) * s3 + (bh % nh) * s2;
     const int64_t kbase = (sc >> 1) * 16 + (sc & 1) * 4;
     _Float16 x[8][8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         const int64_t key = kbase + (i & 3) + (i >> 2) * 8;
-        if (VEC && key < Nkv && d0 + 8 <= D) {
-            *(uint4 *)x[i] = *(const uint4 *)(vb + key * s1 + d0);
-        } else {
+        const T *src = vb + key * s1 + d0;
+        if (key >= Nkv) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) x[i][j] = (key < Nkv && d0 + j < D) ? vb[key * s1 + d0 + j] : (_Float16)0.f;
+            for (int j = 0; j < 8; j++) x[i][j] = (_Float16)0.f;
+        } else if constexpr (sizeof(T) == 2) {
+            if (VEC) *(uint4 *)x[i] = *(const uint4 *)src;
+            else
+#pragma unroll
+                for (int j = 0; j < 8; j++) x[i][j] = src[j];
+        } else {
+            float f[8];
+            if (VEC) {
+                *(float4 *)f = *(const float4 *)src;
+                *(float4 *)(f + 4) = *(const float4 *)(src + 4);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; j++) f[j] = src[j];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[i][j] = to_half(f[j]);
         }
     }
 #pragma unroll
@@ -486,7 +520,7 @@ __global__ __launch_bounds__(256) void k_vt16(const _Float16 *__restrict__ v, in
         _Float16 run[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) run[i] = x[i][j];
-        *(uint4 *)(vt + (bh * hdp + d0 + j) * ldv + 8 * sc) = *(const uint4 *)run;
+        *(uint4 *)(vt + (bh * HD + d0 + j) * ldv + 8 * sc) = *(const uint4 *)run;
     }
 }
 
@@ -581,54 +615,58 @@ hipError_t launch_im2col(const float *chw, int img, int P, int64_t ldk, AKind ki
     return hipGetLastError();
 }
 
-hipError_t launch_attn_prep(const float *q, const int64_t q_nb[4], const float *k,
-                            const int64_t k_nb[4], const float *v, const int64_t v_nb[4],
-                            int64_t Nq, int64_t Nkv, int64_t nh, int64_t B, int D, int hdp, _Float16 *q16,
-                            _Float16 *k16, _Float16 *vt16, _Float16 *q_lo, _Float16 *k_lo,
-                            _Float16 *vt_lo, int64_t ldv, hipStream_t st) {
-    if (D <= 0 || D > hdp) return hipErrorInvalidValue;
-    const int64_t tq = B * nh * Nq * hdp, tk = B * nh * Nkv * hdp;
-    hipLaunchKernelGGL(k_attn_prep, dim3((unsigned)((tq + 255) / 256)), dim3(256), 0, st, q, q_nb[1],
-                       q_nb[2], q_nb[3], Nq, nh, B, D, hdp, q16, q_lo, (int64_t)0, 0);
-    hipLaunchKernelGGL(k_attn_prep, dim3((unsigned)((tk + 255) / 256)), dim3(256), 0, st, k, k_nb[1],
-                       k_nb[2], k_nb[3], Nkv, nh, B, D, hdp, k16, k_lo, (int64_t)0, 0);
-    hipLaunchKernelGGL(k_attn_prep, dim3((unsigned)((tk + 255) / 256)), dim3(256), 0, st, v, v_nb[1],
-                       v_nb[2], v_nb[3], Nkv, nh, B, D, hdp, vt16, vt_lo, ldv, 1);
+namespace {
+template <typename T>
+hipError_t attn_prep(PrepRows p, const int64_t *k_nb, const int64_t *v_nb, int64_t N, int64_t nh, int64_t B, int D,
+                     int hdp, hipStream_t st) {
+    if (D <= 0 || D > hdp || D % 4 != 0 || (hdp != 64 && hdp != 128 && hdp != 256) || B * nh > 65535) return hipErrorInvalidValue;
+    const int64_t *nb[2] = {k_nb, v_nb};
+    constexpr int64_t E = 16 / (int64_t)sizeof(T);  // elements of a 16-byte load
+    bool vec = true;
+    for (int z = 0; z < 2; z++) {
+        if (!p.hi[z]) continue;
+        p.s1[z] = nb[z][1];
+        p.s2[z] = nb[z][2];
+        p.s3[z] = nb[z][3];
+        vec = vec && (uintptr_t)p.src[z] % 16 == 0 && nb[z][1] % E == 0 && nb[z][2] % E == 0 && nb[z][3] % E == 0;
+    }
+    const int lg = hdp == 64 ? 3 : (hdp == 128 ? 4 : 5);
+    const dim3 grid((unsigned)(((N << lg) + 255) / 256), (unsigned)(B * nh), 2);
+    if (vec) hipLaunchKernelGGL((k_attn_prep<T, true>), grid, dim3(256), 0, st, p, (int)N, (int)nh, D, lg);
+    else hipLaunchKernelGGL((k_attn_prep<T, false>), grid, dim3(256), 0, st, p, (int)N, (int)nh, D, lg);
     return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_attn_prep(const float *k, const int64_t k_nb[4], const float *v, const int64_t v_nb[4], int64_t N,
+                            int64_t nh, int64_t B, int D, int hdp, _Float16 *k16, _Float16 *v16, _Float16 *k_lo,
+                            _Float16 *v_lo, hipStream_t st) {
+    const PrepRows p{{k, v}, {}, {}, {}, {k16, v16}, {k_lo, v_lo}};
+    return attn_prep<float>(p, k_nb, v_nb, N, nh, B, D, hdp, st);
 }
 
-hipError_t launch_attn_prep16(const _Float16 *q, const int64_t q_nb[4], const _Float16 *k, const int64_t k_nb[4],
-                              const _Float16 *v, const int64_t v_nb[4], int64_t Nq, int64_t Nkv, int64_t nh,
-                              int64_t B, int D, int hdp, _Float16 *q16, _Float16 *k16, _Float16 *v16,
-                              _Float16 *vt16, int64_t ldv, hipStream_t st) {
-    if (D <= 0 || D > hdp || hdp > 256 || (vt16 && (ldv % 16 != 0 || ldv < Nkv))) return hipErrorInvalidValue;
-    if (q16) {
-        const int64_t t = B * nh * Nq * hdp;
-        hipLaunchKernelGGL(k_attn_prep16, dim3((unsigned)((t + 255) / 256)), dim3(256), 0, st, q, q_nb[1], q_nb[2],
-                           q_nb[3], Nq, nh, B, D, hdp, q16);
-    }
-    if (k16) {
-        const int64_t t = B * nh * Nkv * hdp;
-        hipLaunchKernelGGL(k_attn_prep16, dim3((unsigned)((t + 255) / 256)), dim3(256), 0, st, k, k_nb[1], k_nb[2],
-                           k_nb[3], Nkv, nh, B, D, hdp, k16);
-    }
-    if (v16) {
-        const int64_t t = B * nh * Nkv * hdp;
-        hipLaunchKernelGGL(k_attn_prep16, dim3((unsigned)((t + 255) / 256)), dim3(256), 0, st, v, v_nb[1], v_nb[2],
-                           v_nb[3], Nkv, nh, B, D, hdp, v16);
-    }
-    if (!vt16) return hipGetLastError();
-    const int64_t total = B * nh * (ldv / 8) * (hdp / 8);
-    const bool vec = ((uintptr_t)v % 16 == 0) && v_nb[1] % 8 == 0 && v_nb[2] % 8 == 0 && v_nb[3] % 8 == 0;
+hipError_t launch_attn_prep16(const _Float16 *k, const int64_t k_nb[4], const _Float16 *v, const int64_t v_nb[4],
+                              int64_t N, int64_t nh, int64_t B, int D, int hdp, _Float16 *k16, _Float16 *v16,
+                              hipStream_t st) {
+    const PrepRows p{{k, v}, {}, {}, {}, {k16, v16}, {nullptr, nullptr}};
+    return attn_prep<_Float16>(p, k_nb, v_nb, N, nh, B, D, hdp, st);
+}
+
+template <typename T>
+hipError_t launch_vt(const T *v, const int64_t v_nb[4], int64_t Nkv, int64_t nh, int64_t B, _Float16 *vt, int64_t ldv,
+                     hipStream_t st) {
+    if (ldv % 16 != 0 || ldv < Nkv) return hipErrorInvalidValue;
+    constexpr int64_t E = 16 / (int64_t)sizeof(T);  // elements of a 16-byte load
+    const bool vec = (uintptr_t)v % 16 == 0 && v_nb[1] % E == 0 && v_nb[2] % E == 0 && v_nb[3] % E == 0;
+    const int64_t total = B * nh * (ldv / 8) * (256 / 8);
     const dim3 grid((unsigned)((total + 255) / 256));
-    if (vec)
-        hipLaunchKernelGGL(k_vt16<true>, grid, dim3(256), 0, st, v, v_nb[1], v_nb[2], v_nb[3], Nkv, nh, D, hdp, ldv,
-                           vt16, total);
-    else
-        hipLaunchKernelGGL(k_vt16<false>, grid, dim3(256), 0, st, v, v_nb[1], v_nb[2], v_nb[3], Nkv, nh, D, hdp, ldv,
-                           vt16, total);
+    if (vec) hipLaunchKernelGGL((k_vt<T, true>), grid, dim3(256), 0, st, v, v_nb[1], v_nb[2], v_nb[3], Nkv, nh, ldv, vt, total);
+    else hipLaunchKernelGGL((k_vt<T, false>), grid, dim3(256), 0, st, v, v_nb[1], v_nb[2], v_nb[3], Nkv, nh, ldv, vt, total);
     return hipGetLastError();
 }
+template hipError_t launch_vt<float>(const float *, const int64_t *, int64_t, int64_t, int64_t, _Float16 *, int64_t, hipStream_t);
+template hipError_t launch_vt<_Float16>(const _Float16 *, const int64_t *, int64_t, int64_t, int64_t, _Float16 *, int64_t,
+                                        hipStream_t);
 
 }  // namespace s3e
 

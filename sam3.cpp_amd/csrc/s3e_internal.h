@@ -228,15 +228,26 @@ __host__ __device__ inline int64_t vt_slot(int64_t q) {
 }
 __host__ __device__ inline int64_t vt_ld_for(int64_t nkv) { return (nkv + 15) / 16 * 16; }
 
+// A tile of 32 rows this far apart stays inside the 2^30 bytes one buffer
+// descriptor of the VN attention kernels spans.
+constexpr int64_t ATTN_MAX_ROW = 1 << 23;
+
 // Attention I/O.
 struct AttnArgs {
     const _Float16 *q = nullptr;   // [BH][Nq][hd]
     const _Float16 *k = nullptr;   // [BH][Nkv][hd]
     const _Float16 *vt = nullptr;  // [BH][hd][vt_ld_for(Nkv)], keys in vt_slot order
-    // V as ggml holds it, fp16 [BH][Nkv][hd] (hd 64 or 128, no lo planes):
-    // when set the kernel reads V where it lies (LDS transpose loads) and vt
-    // is not used
-    const _Float16 *v = nullptr;
+    // V as ggml holds it, rows of keys (VN kernels): when set the kernel reads
+    // V through LDS transpose loads (head dims 64 and 128), vt is not used, and
+    // Q, K and V go by element strides (row, head, batch): Q fp16, or f32 at
+    // q32 (q_vec: its rows allow 16-byte loads), K and V fp16 rows of kv_d
+    // channels (a multiple of 8; zeros from there to hd), 16-byte aligned,
+    // strides multiples of 8, rows at most ATTN_MAX_ROW apart.  Head dim 256
+    // takes Q and K so, and vt.  kv_d = 0: plain layouts and vt
+    const _Float16 *v = nullptr, *v_lo = nullptr;
+    const float *q32 = nullptr;
+    int64_t qs[3] = {0, 0, 0}, ks[3] = {0, 0, 0}, vs[3] = {0, 0, 0};
+    int q_vec = 0, kv_d = 0;
     // low halves (x = hi + lo) for split-precision attention, else null
     const _Float16 *q_lo = nullptr, *k_lo = nullptr, *vt_lo = nullptr;
     int Nq = 0, Nkv = 0, NH = 0, BH = 0;
@@ -324,19 +335,22 @@ hipError_t launch_rows_quant(AKind kind, const float *x, int64_t M, int64_t K, c
 hipError_t launch_layernorm(const float *x, int64_t M, int64_t E, float eps, const float *w,
                             const float *b, const Act &out, float *y_f32, hipStream_t st);
 hipError_t launch_attn(const AttnArgs &a, hipStream_t st);
-hipError_t launch_attn_prep(const float *q, const int64_t q_nb[4], const float *k,
-                            const int64_t k_nb[4], const float *v, const int64_t v_nb[4],
-                            int64_t Nq, int64_t Nkv, int64_t nh, int64_t B, int D, int hdp, _Float16 *q16,
-                            _Float16 *k16, _Float16 *vt16, _Float16 *q_lo, _Float16 *k_lo,
-                            _Float16 *vt_lo, int64_t ldv, hipStream_t st);
-// fp16 operands of s3e_flash_attn_ext_f16: Q, K and V (when q16 / k16 /
-// v16 are given) copied to [BH][N][hdp] with zeros for d ≥ D; when vt16 is
-// given V is transposed to Vᵀ [BH][hdp][ldv] in vt_slot order with zeros past
-// Nkv (every slot of every row is written).
-hipError_t launch_attn_prep16(const _Float16 *q, const int64_t q_nb[4], const _Float16 *k, const int64_t k_nb[4],
-                              const _Float16 *v, const int64_t v_nb[4], int64_t Nq, int64_t Nkv, int64_t nh,
-                              int64_t B, int D, int hdp, _Float16 *q16, _Float16 *k16, _Float16 *v16,
-                              _Float16 *vt16, int64_t ldv, hipStream_t st);
+// K and V of the flash_attn_ext entry points as the VN kernels read them: f32
+// or fp16 rows by element strides (nb[1] row, nb[2] head, nb[3] batch), head
+// dim D, to fp16 [BH][N][hdp] with zeros for d ≥ D; with lo planes (f32 only)
+// each value is the pair hi = fp16(v), lo = fp16(v − hi).  Either tensor may be
+// left out (null destination).
+hipError_t launch_attn_prep(const float *k, const int64_t k_nb[4], const float *v, const int64_t v_nb[4], int64_t N,
+                            int64_t nh, int64_t B, int D, int hdp, _Float16 *k16, _Float16 *v16, _Float16 *k_lo,
+                            _Float16 *v_lo, hipStream_t st);
+// V (f32 or fp16 rows by strides, head dim 256) to Vᵀ [BH][256][ldv] fp16 in
+// vt_slot order, zeros past Nkv (every slot of every row is written).
+template <typename T>
+hipError_t launch_vt(const T *v, const int64_t v_nb[4], int64_t Nkv, int64_t nh, int64_t B, _Float16 *vt, int64_t ldv,
+                     hipStream_t st);
+hipError_t launch_attn_prep16(const _Float16 *k, const int64_t k_nb[4], const _Float16 *v, const int64_t v_nb[4],
+                              int64_t N, int64_t nh, int64_t B, int D, int hdp, _Float16 *k16, _Float16 *v16,
+                              hipStream_t st);
 // Measurement kernels (k_probe.hip).  Stream: mode 0 read (sink: blocks·256
 // words), 1 copy, 2 write; bytes a multiple of 16.  MFMA: kind 0 i8
 // 32×32×32, 1 f16 32×32×16, 2 scaled fp6 32×32×64, 3 f16 32×32×8; iters

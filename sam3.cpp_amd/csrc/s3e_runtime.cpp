@@ -771,6 +771,52 @@ extern "C" int s3e_layer_norm(s3e_ctx *ctx, const float *x, int64_t rows, int64_
 } S3E_CATCH("s3e_layer_norm")
 
 // ---- ggml_flash_attn_ext --------------------------------------------------
+namespace {
+
+// Key ranges of one attention call: more than one when the query tiles alone
+// leave the chip idle, for about one round of work-groups (512: two or three
+// fit a CU; 256 at head dim 256, where one fits), each of at least four tiles.
+struct AttnSplit {
+    int64_t n = 1, po = 0, pml = 0;  // ranges; floats of the partial outputs and of their statistics
+    AttnSplit(int64_t BH, int64_t Nq, int64_t Nkv, int hdp) {
+        const int64_t qtiles = (Nq + 127) / 128, ktiles = (Nkv + 31) / 32, target = hdp == 256 ? 256 : 512;
+        if (qtiles * BH < target) {
+            const int64_t ns = std::min<int64_t>((target + qtiles * BH - 1) / (qtiles * BH), std::max<int64_t>(1, ktiles / 4));
+            const int64_t per = (ktiles + ns - 1) / ns;
+            n = (ktiles + per - 1) / per;
+        }
+        po = n * BH * Nq * hdp;
+        pml = n * BH * Nq * 2;
+    }
+    size_t bytes() const { return n > 1 ? (size_t)(po + pml) * 4 : 0; }
+    void set(AttnArgs &a, void *part) const {
+        a.nsplit = (int)n;
+        if (n > 1) {
+            a.part_o = (float *)part;
+            a.part_ml = a.part_o + po;
+        }
+    }
+};
+
+void set_strides(int64_t dst[3], const int64_t nb[4]) {
+    for (int i = 0; i < 3; i++) dst[i] = nb[i + 1];
+}
+
+void set_shape(AttnArgs &a, int64_t D, int hdp, int64_t Nq, int64_t Nkv, int64_t nh, int64_t BH, float scale, float *o) {
+    a.Nq = (int)Nq;
+    a.Nkv = (int)Nkv;
+    a.NH = (int)nh;
+    a.BH = (int)BH;
+    a.hd = hdp;
+    a.hd_out = D == hdp ? 0 : (int)D;
+    a.scale = scale;
+    a.out.kind = A_F32;
+    a.out.x = o;
+    a.out.ld = nh * D;
+}
+
+}  // namespace
+
 extern "C" int s3e_flash_attn_ext(s3e_ctx *ctx, const float *q, const int64_t q_nb[4], const float *k,
                                   const int64_t k_nb[4], const float *v, const int64_t v_nb[4], int64_t D,
                                   int64_t Nq, int64_t Nkv, int64_t nh, int64_t B, float scale, int prec,
@@ -794,56 +840,40 @@ extern "C" int s3e_flash_attn_ext(s3e_ctx *ctx, const float *q, const int64_t q_
     }
     if (B * nh > 65535 || Nq > (1 << 24) || Nkv > (1 << 24)) { set_error("s3e_flash_attn_ext: shape too large"); return S3E_ERR_INVALID; }
     HIP_TRY(hipSetDevice(ctx->device));
+    // K and V are converted to [BH][Nkv][hdp] fp16 rows (hi, and lo planes at
+    // S3E_PREC_F32); Q is read and converted by the attention kernel itself
+    const int np = (prec == S3E_PREC_F32) ? 2 : 1;
+    const int64_t BH = B * nh;
+    // (at head dim 256 V goes through the Vᵀ layout)
     const int64_t ldv = vt_ld_for(Nkv);
-    const int np = (prec == S3E_PREC_F32) ? 2 : 1;  // hi (+ lo) planes
-    const size_t qn = (size_t)(B * nh * Nq * hdp), kn = (size_t)(B * nh * Nkv * hdp), vn = (size_t)(B * nh * ldv * hdp);
-    // split the keys when the query tiles alone leave the chip idle (plain layouts only)
-    const int64_t BH = B * nh, qtiles = (Nq + 127) / 128, ktiles = (Nkv + 31) / 32;
-    int nsplit = 1;
-    // about one round of work-groups: 512 (two or three fit a CU), 256 at head dim 256 (one fits)
-    const int64_t target = hdp == 256 ? 256 : 512;
-    if (D == hdp && qtiles * BH < target) {
-        int64_t ns = std::min<int64_t>((target + qtiles * BH - 1) / (qtiles * BH), std::max<int64_t>(1, ktiles / 4));
-        const int64_t per = (ktiles + ns - 1) / ns;
-        nsplit = (int)((ktiles + per - 1) / per);
-    }
-    const size_t po = (size_t)nsplit * BH * Nq * hdp, pml = (size_t)nsplit * BH * Nq * 2;
-    // [Q][K][Vᵀ][partials]; every plane is a multiple of 128 bytes
+    const size_t kn = (size_t)(BH * Nkv * hdp), vn = hdp == 256 ? (size_t)(BH * hdp * ldv) : kn;
+    const AttnSplit sp(BH, Nq, Nkv, hdp);
+    // [K hi, lo][V hi, lo][partials]; every plane is a multiple of 128 bytes
     CallWs ws(ctx);
     void *base = nullptr;
-    hipError_t e = ws.get((qn + kn + vn) * 2 * np + (nsplit > 1 ? (po + pml) * 4 : 0), &base);
-    _Float16 *q16 = (_Float16 *)base, *k16 = q16 + qn * np, *vt16 = k16 + kn * np;
-    float *part = (float *)(vt16 + vn * np);
-    if (e == hipSuccess) e = hipMemsetAsync(vt16, 0, vn * 2 * np, ctx->stream);
+    hipError_t e = ws.get((kn + vn) * 2 * np + sp.bytes(), &base);
     AttnArgs a;
-    a.q = q16;
-    a.k = k16;
-    a.vt = vt16;
-    if (np == 2) {
-        a.q_lo = q16 + qn;
-        a.k_lo = k16 + kn;
-        a.vt_lo = vt16 + vn;
-    }
-    if (e == hipSuccess)
-        e = launch_attn_prep(q, q_nb, k, k_nb, v, v_nb, Nq, Nkv, nh, B, (int)D, hdp, q16, k16, vt16,
-                             (_Float16 *)a.q_lo, (_Float16 *)a.k_lo, (_Float16 *)a.vt_lo, ldv, ctx->stream);
     if (e == hipSuccess) {
-        a.Nq = (int)Nq;
-        a.Nkv = (int)Nkv;
-        a.NH = (int)nh;
-        a.BH = (int)BH;
-        a.hd = hdp;
-        a.hd_out = D == hdp ? 0 : (int)D;
-        a.scale = scale;
-        a.grid = 0;
-        a.nsplit = nsplit;
-        if (nsplit > 1) {
-            a.part_o = part;
-            a.part_ml = part + po;
-        }
-        a.out.kind = A_F32;
-        a.out.x = o;
-        a.out.ld = nh * D;
+        _Float16 *k16 = (_Float16 *)base, *v16 = k16 + kn * np;
+        _Float16 *k_lo = np == 2 ? k16 + kn : nullptr, *v_lo = np == 2 ? v16 + vn : nullptr;
+        a.q32 = q;
+        set_strides(a.qs, q_nb);
+        a.q_vec = (uintptr_t)q % 16 == 0 && q_nb[1] % 4 == 0 && q_nb[2] % 4 == 0 && q_nb[3] % 4 == 0;
+        a.k = k16;
+        (hdp == 256 ? a.vt : a.v) = v16;
+        a.k_lo = k_lo;
+        a.v_lo = v_lo;
+        a.kv_d = hdp;
+        a.ks[0] = a.vs[0] = hdp;
+        a.ks[1] = a.vs[1] = Nkv * hdp;
+        a.ks[2] = a.vs[2] = nh * Nkv * hdp;
+        e = launch_attn_prep(k, k_nb, v, v_nb, Nkv, nh, B, (int)D, hdp, k16, hdp == 256 ? nullptr : v16, k_lo, v_lo,
+                             ctx->stream);
+        if (e == hipSuccess && hdp == 256) e = launch_vt(v, v_nb, Nkv, nh, B, v16, ldv, ctx->stream);
+    }
+    if (e == hipSuccess) {
+        set_shape(a, D, hdp, Nq, Nkv, nh, BH, scale, o);
+        sp.set(a, (uint8_t *)base + (kn + vn) * 2 * np);
         e = launch_attn(a, ctx->stream);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -872,30 +902,22 @@ extern "C" int s3e_flash_attn_ext_f16(s3e_ctx *ctx, const uint16_t *q, const int
     }
     HIP_TRY(hipSetDevice(ctx->device));
     const int hdp = D <= 64 ? 64 : (D <= 128 ? 128 : 256);
-    const int64_t ldv = vt_ld_for(Nkv);
-    const int64_t BH = B * nh, qtiles = (Nq + 127) / 128, ktiles = (Nkv + 31) / 32;
-    // Q and K are read where they lie when they already are [B][nh][N][hdp]
-    auto plain = [&](const int64_t nb[4], int64_t N) {
-        return D == hdp && nb[1] == hdp && nb[2] == N * hdp && nb[3] == nh * N * hdp;
+    const int64_t BH = B * nh;
+    // K and V are read where they lie when whole 16-byte chunks can be moved
+    // (D and the strides multiples of 8, 16-byte aligned), else copied to
+    // [BH][Nkv][hdp]; Q is read by strides of any kind, and head dim 256 takes
+    // V through the Vᵀ layout
+    auto in_place = [&](const void *x, const int64_t nb[4]) {
+        return D % 8 == 0 && (uintptr_t)x % 16 == 0 && nb[1] % 8 == 0 && nb[2] % 8 == 0 && nb[3] % 8 == 0 &&
+               nb[1] <= ATTN_MAX_ROW;
     };
-    const bool q_in = plain(q_nb, Nq), k_in = plain(k_nb, Nkv);
-    // V: read where it lies as well (head dims up to 128), else copied to the
-    // plain layout; head dim 256 goes through the Vᵀ layout
-    const bool vnat = hdp <= 128, v_in = vnat && plain(v_nb, Nkv);
-    int nsplit = 1;
-    const int64_t target = hdp == 256 ? 256 : 512;
-    if (D == hdp && qtiles * BH < target) {
-        const int64_t ns = std::min<int64_t>((target + qtiles * BH - 1) / (qtiles * BH), std::max<int64_t>(1, ktiles / 4));
-        const int64_t per = (ktiles + ns - 1) / ns;
-        nsplit = (int)((ktiles + per - 1) / per);
-    }
-    // workspace: [V copy or Vᵀ][Q copy][K copy][partials], 256-byte aligned pieces
-    auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t vb = vnat ? (v_in ? 0 : al((size_t)(BH * Nkv * hdp) * 2)) : al((size_t)(BH * hdp * ldv) * 2), qb = q_in ? 0 : al((size_t)(BH * Nq * hdp) * 2),
-                 kb = k_in ? 0 : al((size_t)(BH * Nkv * hdp) * 2);
-    const size_t po = (size_t)nsplit * BH * Nq * hdp, pml = (size_t)nsplit * BH * Nq * 2;
-    const size_t pb = nsplit > 1 ? (po + pml) * 4 : 0;
-    const size_t need = vb + qb + kb + pb;
+    const bool k_in = in_place(k, k_nb), v_t = hdp == 256, v_in = !v_t && in_place(v, v_nb);
+    const int64_t ldv = vt_ld_for(Nkv);
+    const AttnSplit sp(BH, Nq, Nkv, hdp);
+    // workspace: [K copy][V copy or Vᵀ][partials]; a copy is a multiple of 128 bytes
+    const size_t kn = k_in ? 0 : (size_t)(BH * Nkv * hdp);
+    const size_t vn = v_in ? 0 : (size_t)(BH * hdp * (v_t ? ldv : Nkv));
+    const size_t need = (kn + vn) * 2 + sp.bytes();
     if (need > ctx->attn_ws_cap) {
         HIP_TRY(hipStreamSynchronize(ctx->stream));  // earlier calls may still read it
         if (ctx->attn_ws) (void)hipFree(ctx->attn_ws);
@@ -904,36 +926,30 @@ extern "C" int s3e_flash_attn_ext_f16(s3e_ctx *ctx, const uint16_t *q, const int
         HIP_TRY(hipMalloc(&ctx->attn_ws, need));
         ctx->attn_ws_cap = need;
     }
-    uint8_t *ws = (uint8_t *)ctx->attn_ws;
-    _Float16 *vt16 = vnat ? nullptr : (_Float16 *)ws;
-    _Float16 *v16 = (vnat && !v_in) ? (_Float16 *)ws : nullptr;
-    _Float16 *q16 = q_in ? nullptr : (_Float16 *)(ws + vb);
-    _Float16 *k16 = k_in ? nullptr : (_Float16 *)(ws + vb + qb);
+    _Float16 *k16 = (_Float16 *)ctx->attn_ws, *v16 = k16 + kn;
+    AttnArgs a;
+    a.q = (const _Float16 *)q;
+    set_strides(a.qs, q_nb);
+    a.q_vec = in_place(q, q_nb);
     hipError_t e = hipSuccess;
-    if (!q_in || !k_in || !v_in)
-        e = launch_attn_prep16((const _Float16 *)q, q_nb, (const _Float16 *)k, k_nb, (const _Float16 *)v, v_nb, Nq,
-                               Nkv, nh, B, (int)D, hdp, q16, k16, v16, vt16, ldv, ctx->stream);
+    const int64_t plain[4] = {1, hdp, Nkv * hdp, nh * Nkv * hdp};
+    a.kv_d = D % 8 == 0 ? (int)D : hdp;  // (no tensor is read in place unless D % 8 == 0)
+    const auto contiguous = [&](const int64_t nb[4], int64_t N) {
+        return nb[1] == hdp && nb[2] == N * hdp && nb[3] == nh * N * hdp;
+    };
+    if (v_t && a.q_vec && k_in && contiguous(q_nb, Nq) && contiguous(k_nb, Nkv)) a.kv_d = 0;
+    a.k = k_in ? (const _Float16 *)k : k16;
+    set_strides(a.ks, k_in ? k_nb : plain);
+    if (v_t) a.vt = v16;
+    else a.v = v_in ? (const _Float16 *)v : v16;
+    set_strides(a.vs, v_in ? v_nb : plain);
+    if (!k_in || (!v_in && !v_t))
+        e = launch_attn_prep16((const _Float16 *)k, k_nb, (const _Float16 *)v, v_nb, Nkv, nh, B, (int)D, hdp,
+                               k_in ? nullptr : k16, v_in || v_t ? nullptr : v16, ctx->stream);
+    if (e == hipSuccess && v_t) e = launch_vt((const _Float16 *)v, v_nb, Nkv, nh, B, v16, ldv, ctx->stream);
     if (e == hipSuccess) {
-        AttnArgs a;
-        a.q = q_in ? (const _Float16 *)q : q16;
-        a.k = k_in ? (const _Float16 *)k : k16;
-        if (vnat) a.v = v_in ? (const _Float16 *)v : v16;
-        else a.vt = vt16;
-        a.Nq = (int)Nq;
-        a.Nkv = (int)Nkv;
-        a.NH = (int)nh;
-        a.BH = (int)BH;
-        a.hd = hdp;
-        a.hd_out = D == hdp ? 0 : (int)D;
-        a.scale = scale;
-        a.nsplit = nsplit;
-        if (nsplit > 1) {
-            a.part_o = (float *)(ws + vb + qb + kb);
-            a.part_ml = a.part_o + po;
-        }
-        a.out.kind = A_F32;
-        a.out.x = o;
-        a.out.ld = nh * D;
+        set_shape(a, D, hdp, Nq, Nkv, nh, BH, scale, o);
+        sp.set(a, (uint8_t *)ctx->attn_ws + (kn + vn) * 2);
         e = launch_attn(a, ctx->stream);
     }
     if (e != hipSuccess) { set_error("s3e_flash_attn_ext_f16: %s", hipGetErrorString(e)); return S3E_ERR_HIP; }
@@ -2260,22 +2276,21 @@ extern "C" int s3e_vit_block_stage(s3e_state *st, int idx, int stage, const floa
             HIP_TRY(launch_vit_rope_split(in_device, b.freqs, st->stg, B, N, (int)NH, (int)HD, s));
             // the encoder's rule: split fp16 pairs unless the projection is F16
             const bool split = b.proj.kind != WK_F16;
-            _Float16 *q_lo = split ? st->q16 + st->T * E : nullptr;
-            _Float16 *k_lo = split ? st->k16 + st->T * E : nullptr;
-            _Float16 *vt_lo = split ? st->vt16 + st->vt_elems : nullptr;
-            HIP_TRY(hipMemsetAsync(st->vt16, 0, (size_t)(B * NH * HD * ldv) * 2, s));
-            if (split) HIP_TRY(hipMemsetAsync(vt_lo, 0, (size_t)(B * NH * HD * ldv) * 2, s));
+            AttnArgs a;
+            a.q32 = rq;
+            a.k = st->k16;
+            a.v = st->vt16;
+            a.k_lo = split ? st->k16 + st->T * E : nullptr;
+            a.v_lo = split ? st->vt16 + st->vt_elems : nullptr;
+            a.kv_d = (int)HD;
+            a.q_vec = 1;
             const int64_t qk_nb[4] = {1, HD, N * HD, NH * N * HD};
             const int64_t v_nb[4] = {1, 3 * E, HD, N * 3 * E};
-            HIP_TRY(launch_attn_prep(rq, qk_nb, rk, qk_nb, in_device + 2 * E, v_nb, N, N, NH, B, (int)HD, 64,
-                                     st->q16, st->k16, st->vt16, q_lo, k_lo, vt_lo, ldv, s));
-            AttnArgs a;
-            a.q = st->q16;
-            a.k = st->k16;
-            a.vt = st->vt16;
-            a.q_lo = q_lo;
-            a.k_lo = k_lo;
-            a.vt_lo = vt_lo;
+            set_strides(a.qs, qk_nb);
+            set_strides(a.ks, qk_nb);
+            set_strides(a.vs, qk_nb);
+            HIP_TRY(launch_attn_prep(rk, qk_nb, in_device + 2 * E, v_nb, N, NH, B, (int)HD, (int)HD, st->k16, st->vt16,
+                                     (_Float16 *)a.k_lo, (_Float16 *)a.v_lo, s));
             a.Nq = (int)N;
             a.Nkv = (int)N;
             a.NH = (int)NH;

@@ -1,0 +1,99 @@
+"""s3e_flash_attn_ext and s3e_flash_attn_ext_f16 read Q, K and V by strides:
+in place, or through copies where 16-byte chunks cannot be moved.  Both ways
+over orders, strides, alignments, head dims and ragged key counts, against
+softmax(Q·Kᵀ·scale)·V in 64 bits.
+
+Bounds: fp16 operands and probabilities leave 3e-4 to 5e-4 relative L2 (fp16's
+2^-11 per probability and operand, averaged), held to 2e-3; fp16 pairs 2^-22 per
+operand and fp32 sums, held to 2e-6.
+"""
+import numpy as np
+import pytest
+
+import s3e
+
+pytestmark = pytest.mark.gpu
+
+
+def _exact(q, k, v, scale):
+    s = np.einsum("bhid,bhjd->bhij", q, k) * scale
+    p = np.exp(s - s.max(-1, keepdims=True))
+    return np.einsum("bhij,bhjd->bihd", p / p.sum(-1, keepdims=True), v)
+
+
+def _place(x, layout, off):
+    """x [B][nh][N][D] in one flat array: the array, its first element and (row, head, batch) strides."""
+    B, nh, N, D = x.shape
+    rows = {"heads": x, "tokens": x.transpose(0, 2, 1, 3), "wide": x, "odd": x}[layout]
+    pad = {"wide": 8, "odd": 5}.get(layout, 0)
+    rows = np.concatenate([rows, np.full(rows.shape[:-1] + (pad,), np.nan, x.dtype)], -1)  # never read
+    flat = np.concatenate([np.full(off, np.nan, x.dtype), rows.ravel()])
+    w = D + pad
+    return flat, off, (w * nh, w, w * nh * N) if layout == "tokens" else (w, w * N, w * N * nh)
+
+
+def _run(ctx, q, k, v, prec, layouts, offs):
+    B, nh, Nq, D = q.shape
+    Nkv = k.shape[2]
+    half = prec == "f16"
+    views = []
+    for x, layout, off in zip((q, k, v), layouts, offs):
+        flat, first, st = _place(x.astype(np.float16 if half else np.float32), layout, off)
+        buf = ctx.to_device(flat)
+        views.append((buf, s3e.DeviceView(buf.ptr + first * flat.itemsize, flat.nbytes), (1,) + st))
+    O = ctx.buffer(B * Nq * nh * D * 4)
+    args = [a for _, view, st in views for a in (view, st)] + [D, Nq, Nkv, nh, B, D ** -0.5, O]
+    if half:
+        ctx.flash_attn_ext_f16(*args)
+    else:
+        ctx.flash_attn_ext(*args, prec=s3e.PREC_F32 if prec == "f32" else s3e.PREC_DEFAULT)
+    ctx.sync()
+    return O.download(np.float32, (B, Nq, nh, D))
+
+
+FORMS = [(("heads",) * 3, (0, 0, 0)), (("tokens",) * 3, (0, 0, 0)), (("heads", "heads", "tokens"), (8, 16, 8)),
+         (("wide", "heads", "wide"), (0, 0, 8)), (("heads", "odd", "heads"), (0, 0, 0)),
+         (("odd", "heads", "heads"), (3, 0, 1)), (("tokens", "odd", "odd"), (0, 1, 3))]
+SIZES = [(64, 2, 3, 40, 40), (64, 1, 2, 129, 1025), (32, 1, 1, 1, 1), (72, 2, 2, 16, 49), (96, 1, 3, 200, 196),
+         (36, 2, 2, 33, 31), (124, 1, 1, 5, 700), (128, 1, 2, 70, 64), (56, 40, 16, 13, 33)]
+
+
+@pytest.mark.parametrize("prec", ["f16", "default", "f32"])
+@pytest.mark.parametrize("D,B,nh,Nq,Nkv", SIZES + [(256, 1, 2, 33, 47), (256, 2, 1, 130, 300)])
+def test_layouts(ctx, prec, D, B, nh, Nq, Nkv):
+    if D == 256 and prec == "f32":
+        pytest.skip("head dim 256 runs on fp16 operands only")
+    rng = np.random.default_rng(D + Nq)
+    q, k, v = (rng.standard_normal((B, nh, n, D)) for n in (Nq, Nkv, Nkv))
+    if prec != "f32":
+        q, k, v = (x.astype(np.float16) for x in (q, k, v))
+    q, k, v = (x.astype(np.float32).astype(np.float64) for x in (q, k, v))
+    ref = _exact(q, k, v, D ** -0.5)
+    for layouts, offs in FORMS:
+        print(prec, D, layouts, offs, flush=True)
+        got = _run(ctx, q, k, v, prec, layouts, offs)
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert err <= (2e-6 if prec == "f32" else 2e-3), (layouts, offs, err)
+
+
+def test_padding_reads_nothing_of_the_next_head(ctx):
+    # heads of 72 channels side by side run padded to 128: head 1's NaN must stay out of head 0
+    rng = np.random.default_rng(1)
+    q, k, v = (rng.standard_normal((1, 2, n, 72)).astype(np.float16).astype(np.float64) for n in (20, 50, 50))
+    ref = _exact(q, k, v, 72 ** -0.5)
+    for x in (q, k, v):
+        x[:, 1] = np.nan
+    got = _run(ctx, q, k, v, "f16", ("tokens",) * 3, (0, 0, 0))[:, :, 0]
+    assert np.linalg.norm(got - ref[:, :, 0]) <= 2e-3 * np.linalg.norm(ref[:, :, 0])
+
+
+def test_repeated_rows_by_zero_stride(ctx):
+    # one K / V row stride of 0: every key is the same, so O is that row of V
+    rng = np.random.default_rng(2)
+    q, k, v = (rng.standard_normal((n, 64)).astype(np.float16) for n in (9, 1, 1))
+    O = ctx.buffer(9 * 64 * 4)
+    ctx.flash_attn_ext_f16(ctx.to_device(q), (1, 64, 0, 0), ctx.to_device(k), (1, 0, 0, 0), ctx.to_device(v),
+                           (1, 0, 0, 0), 64, 9, 100, 1, 1, 0.125, O)
+    ctx.sync()
+    got = O.download(np.float32, (9, 64))
+    assert np.linalg.norm(got - v.astype(np.float32)) <= 2e-3 * 3 * np.linalg.norm(v.astype(np.float32))
