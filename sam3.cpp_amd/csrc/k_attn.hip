@@ -80,8 +80,6 @@ struct AG {
     static constexpr int VPL = HD * KT * 2;    // bytes of one Vᵀ plane of a tile: HD rows × 32 keys
     static constexpr int KRUNS = KPL / 1024 / AW;  // 1 KB DMA runs per wave per K plane
     static constexpr int VRUNS = VPL / 1024 / AW;  // ... per Vᵀ plane
-    static constexpr int DS = HD / 16;         // K=16 steps of Sᵀ
-    static constexpr int DT = HD / 32;         // 32-row tiles of Oᵀ
 };
 
 __device__ __forceinline__ uint16_t f2h_bits(float v) { return half_bits(v); }
@@ -118,14 +116,48 @@ __device__ __forceinline__ int swzvn(int r) {
     }
 }
 
-typedef __fp16 v4fp16 __attribute__((__vector_size__(4 * sizeof(__fp16))));
-typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 
-// ds_read_b64_tr_b16: within each group of 16 lanes, lane i receives element
-// i % 4 of the 8 bytes addressed by lanes 4j + i / 4, j = 0..3
-__device__ __forceinline__ v4h lds_tr16(const uint8_t *p) {
-    const v4fp16 r = __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) v4fp16 *)(p));
-    return __builtin_bit_cast(v4h, r);
+// Eight ds_read_b64_tr_b16, with their wait: within each group of 16 lanes,
+// lane i receives element i % 4 of the 8 bytes addressed by lanes 4j + i / 4,
+// j = 0..3.  Operand r[k] is the pair of loads from a[2·(k / 2)] and
+// a[2·(k / 2) + 1] at byte offset (k % 2)·STEP (two address pairs), or from
+// a[0] and a[1] at (k % 2)·STEP + (k / 2)·PLANE (one pair, hi and lo planes).
+// In assembly, because the compiler does not tell the builtin's LDS reads from
+// the tile loads in flight to other LDS addresses and waits for all of them
+// first, once per tile (16 heads × 5184² fp16: 175 µs so, 171 µs without).
+template <int STEP, int PLANE>
+__device__ __forceinline__ void lds_tr16x8(const uint32_t (&a)[4], v8h (&r)[4]) {
+    v2u x[8];
+    if constexpr (PLANE == 0) {
+        __asm__ volatile("ds_read_b64_tr_b16 %0, %8\n\t"
+                         "ds_read_b64_tr_b16 %1, %9\n\t"
+                         "ds_read_b64_tr_b16 %2, %8 offset:%12\n\t"
+                         "ds_read_b64_tr_b16 %3, %9 offset:%12\n\t"
+                         "ds_read_b64_tr_b16 %4, %10\n\t"
+                         "ds_read_b64_tr_b16 %5, %11\n\t"
+                         "ds_read_b64_tr_b16 %6, %10 offset:%12\n\t"
+                         "ds_read_b64_tr_b16 %7, %11 offset:%12\n\t"
+                         "s_waitcnt lgkmcnt(0)"
+                         : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]),
+                           "=&v"(x[7])
+                         : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "n"(STEP));
+    } else {
+        __asm__ volatile("ds_read_b64_tr_b16 %0, %8\n\t"
+                         "ds_read_b64_tr_b16 %1, %9\n\t"
+                         "ds_read_b64_tr_b16 %2, %8 offset:%10\n\t"
+                         "ds_read_b64_tr_b16 %3, %9 offset:%10\n\t"
+                         "ds_read_b64_tr_b16 %4, %8 offset:%11\n\t"
+                         "ds_read_b64_tr_b16 %5, %9 offset:%11\n\t"
+                         "ds_read_b64_tr_b16 %6, %8 offset:%12\n\t"
+                         "ds_read_b64_tr_b16 %7, %9 offset:%12\n\t"
+                         "s_waitcnt lgkmcnt(0)"
+                         : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]),
+                           "=&v"(x[7])
+                         : "v"(a[0]), "v"(a[1]), "n"(STEP), "n"(PLANE), "n"(PLANE + STEP));
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) r[k] = __builtin_bit_cast(v8h, v4u{x[2 * k][0], x[2 * k][1], x[2 * k + 1][0], x[2 * k + 1][1]});
 }
 
 // p − h for the fp16 value h in the low or high half of h2, exact, in one
@@ -144,9 +176,19 @@ __device__ __forceinline__ float sub_hi_half(float p, uint32_t h2) {
 // CROP: the windowed, cropped output mapping and narrower real heads
 // (a.wo, a.hd_out; the Hiera layouts), kept out of the plain variants.
 // STR: Q and K (and V, VN) by strides.
-template <bool SPLIT, int HD, bool CROP, bool VN = false, bool STR = VN>
+// HR: channels that take part, the real head dim rounded up to whole MFMA
+// tiles (heads of 65 to 96 channels lie in rows of 128 and skip the last
+// quarter: its K chunks, Vᵀ rows, operand reads and MFMAs).
+template <bool SPLIT, int HD, bool CROP, bool VN = false, bool STR = VN, int HR = HD>
 __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_attn(AttnArgs a, int ldv) {
     using G = AG<HD>;
+    constexpr int DS = HR / 16, DT = HR / 32;  // K=16 steps of Sᵀ, 32-row tiles of Oᵀ
+    // The main loop takes two tiles per turn, so that scores and probabilities
+    // change places without copies: fp16 at head dim 64 (16 × 5184² 166 → 161
+    // µs) and head dim 256 (a memory-attention pass 1190 → 1160 µs).  Not the
+    // split kernels, which have no registers for it (the 32 ViT blocks 10.5 →
+    // 10.9 ms), nor the cropped ones, whose few tiles do not repay the code.
+    constexpr bool PAIRS = !SPLIT && ((HD == 64 && !CROP) || HD == 256);
     constexpr int NP = SPLIT ? 2 : 1;  // planes: hi (and lo)
     static_assert(VN ? STR && HD <= 128 : !STR || HD == 256, "natural V at head dim 64 or 128, by strides");
     constexpr int KPL = G::KPL, VPL = G::VPL;
@@ -161,13 +203,13 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
     const int qi = q0 + wave * 32 + lr;
     const bool qvalid = qi < a.Nq;
 
-    v8h qf[NP][G::DS];
+    v8h qf[NP][DS];
     if constexpr (STR) {
         const int64_t off = (int64_t)(bh / a.NH) * a.qs[2] + (int64_t)(bh % a.NH) * a.qs[1] +
                             (int64_t)(qvalid ? qi : 0) * a.qs[0];
         const int dr = a.hd_out > 0 ? a.hd_out : HD;
 #pragma unroll
-        for (int ds = 0; ds < G::DS; ds++) {
+        for (int ds = 0; ds < DS; ds++) {
             const int d0 = ds * 16 + lh * 8;
             if (a.q32) {
                 // (the head dim is a multiple of 4: four channels are all real or all padding)
@@ -209,7 +251,7 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         for (int pl = 0; pl < NP; pl++) {
             const _Float16 *qrow = (pl == 0 ? a.q : a.q_lo) + off;
 #pragma unroll
-            for (int ds = 0; ds < G::DS; ds++) {
+            for (int ds = 0; ds < DS; ds++) {
                 v8h z = {};
                 qf[pl][ds] = qvalid ? *(const v8h *)(qrow + ds * 16 + lh * 8) : z;
             }
@@ -217,15 +259,15 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
     }
     const float c = a.scale * 1.44269504088896340736f;
     float mrun = -INFINITY, lsum = 0.f;
-    v16f o[G::DT];
+    v16f o[DT];
 #pragma unroll
-    for (int dt = 0; dt < G::DT; dt++)
+    for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
 
     int64_t koff = (int64_t)bh * a.Nkv * HD, voff = (int64_t)bh * HD * ldv;
     // bytes from one K (V) row to the next, and of a row's real channels
-    int k_rb = G::ROWK, v_rb = G::ROWK, real = G::ROWK;
+    int k_rb = G::ROWK, v_rb = G::ROWK, real = 2 * HR;
     if constexpr (STR) {
         const int b = bh / a.NH, h = bh % a.NH;
         koff = b * a.ks[2] + h * a.ks[1];
@@ -260,7 +302,7 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
             __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)nrec, 0x00020000);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, LDS_PTR(ldsp), 16, lane_off, 0, 0, 0);
     };
-    // STR: chunks past a row's real channels load zeros (the launcher keeps
+    // chunks past a row's real channels load zeros (the launcher keeps
     // every tile's record count below this offset)
     constexpr int PAST = 1 << 30;
     int k_lane[G::KRUNS], v_lane[G::VRUNS];
@@ -270,7 +312,7 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         constexpr int CPR = G::ROWK / 16;        // chunks per row
         const int r = RPR * (wave * G::KRUNS + j) + lane / CPR;
         const int ch = ((lane % CPR) ^ swzk_hd<HD>(r)) << 4;
-        k_lane[j] = STR && ch >= real ? PAST : r * k_rb + ch;
+        k_lane[j] = (STR || HR < HD) && ch >= real ? PAST : r * k_rb + ch;
     }
     int vn_lane[G::KRUNS];  // VN: V tiles as K tiles, own swizzle
 #pragma unroll
@@ -326,7 +368,9 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         for (int pl = 0; pl < NP; pl++) {
             const _Float16 *base = (pl == 0 ? a.vt : a.vt_lo) + voff + (int64_t)tile * KT;
 #pragma unroll
-            for (int j = 0; j < G::VRUNS; j++) dma(base, nrec, L + pl * VPL + (wave * G::VRUNS + j) * 1024, off[j]);
+            for (int j = 0; j < G::VRUNS; j++)
+                if (HR == HD || 16 * (wave * G::VRUNS + j) < HR)
+                    dma(base, nrec, L + pl * VPL + (wave * G::VRUNS + j) * 1024, off[j]);
         }
     };
 
@@ -337,7 +381,7 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         const uint8_t *L = Kring + (tt & 1) * KBUF;
         v16f acc = {};
 #pragma unroll
-        for (int ds = 0; ds < G::DS; ds++) {
+        for (int ds = 0; ds < DS; ds++) {
             const int o_ = lr * G::ROWK + (((2 * ds + lh) ^ xk) << 4);
             const v8h kh = *(const v8h *)(L + o_);
             if constexpr (SPLIT) {
@@ -354,34 +398,46 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
     // 16·jj + 4·lh + j (+ 8 for the second load) at channels dt·32 + 16·gc +
     // 4q .. + 3, so each lane receives channel dt·32 + L % 32 of keys
     // 16·jj + 4·lh + 0..3 and + 8..11: the keys its K slots hold
+    // (the swizzle of a row does not depend on jj: the two K=16 steps are one
+    // address apart by 16 rows)
     const int tr_j = (lane & 15) >> 2, tr_q = lane & 3, tr_gc = (lane >> 4) & 1;
-    auto tr_off = [&](int dt, int jj, int half) {
-        const int row = 16 * jj + 8 * half + 4 * lh + tr_j;
+    const uint32_t vring = (uint32_t)(uintptr_t)LDS_PTR(Vring);
+    auto tr_at = [&](int tt, int dt, int half) {
+        const int row = 8 * half + 4 * lh + tr_j;
         const int chunk = 4 * dt + 2 * tr_gc + (tr_q >> 1);
-        return row * G::ROWK + ((chunk ^ swzvn<HD>(row)) << 4) + 8 * (tr_q & 1);
+        return vring + (uint32_t)((tt & 1) * VBUF + row * G::ROWK + ((chunk ^ swzvn<HD>(row)) << 4) + 8 * (tr_q & 1));
     };
     auto pv = [&](int tt, const v8h (&ph)[2], const v8h (&pl)[2]) {
         const uint8_t *L = Vring + (tt & 1) * VBUF;
-        if constexpr (VN) {
+        if constexpr (VN && SPLIT) {
 #pragma unroll
-            for (int dt = 0; dt < G::DT; dt++)
+            for (int dt = 0; dt < DT; dt++) {
+                v8h v[4];  // hi (jj = 0, 1), lo
+                lds_tr16x8<16 * G::ROWK, VPL>({tr_at(tt, dt, 0), tr_at(tt, dt, 1), 0u, 0u}, v);
 #pragma unroll
                 for (int jj = 0; jj < 2; jj++) {
-                    const int o0 = tr_off(dt, jj, 0), o1 = tr_off(dt, jj, 1);
-                    const v4h v0 = lds_tr16(L + o0), v1 = lds_tr16(L + o1);
-                    const v8h vh = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-                    if constexpr (SPLIT) {
-                        const v4h l0 = lds_tr16(L + VPL + o0), l1 = lds_tr16(L + VPL + o1);
-                        const v8h vl = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-                        o[dt] = mfma(vl, ph[jj], o[dt]);
-                        o[dt] = mfma(vh, pl[jj], o[dt]);
-                    }
-                    o[dt] = mfma(vh, ph[jj], o[dt]);
+                    o[dt] = mfma(v[2 + jj], ph[jj], o[dt]);
+                    o[dt] = mfma(v[jj], pl[jj], o[dt]);
+                    o[dt] = mfma(v[jj], ph[jj], o[dt]);
                 }
+            }
+            return;
+        } else if constexpr (VN) {
+#pragma unroll
+            for (int dt = 0; dt < DT; dt += 2) {
+                const int d1 = dt + 1 < DT ? dt + 1 : dt;  // an odd last tile is read twice
+                v8h v[4];
+                lds_tr16x8<16 * G::ROWK, 0>({tr_at(tt, dt, 0), tr_at(tt, dt, 1), tr_at(tt, d1, 0), tr_at(tt, d1, 1)}, v);
+#pragma unroll
+                for (int jj = 0; jj < 2; jj++) {
+                    o[dt] = mfma(v[jj], ph[jj], o[dt]);
+                    if (d1 != dt) o[d1] = mfma(v[2 + jj], ph[jj], o[d1]);
+                }
+            }
             return;
         }
 #pragma unroll
-        for (int dt = 0; dt < G::DT; dt++)
+        for (int dt = 0; dt < DT; dt++)
 #pragma unroll
             for (int jj = 0; jj < 2; jj++) {
                 const int o_ = (dt * 32 + lr) * 64 + (((2 * jj + lh) ^ xv) << 4);
@@ -435,35 +491,41 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         }
         return ps;
     };
-    // Issue is in order within a wave: the scheduling barriers interleave the
-    // MFMA stream (Sᵀ of the next tile, Oᵀ of the previous) with the softmax
-    // VALU of the current tile, which then runs in the MFMA shadow.
-    auto interleave = [&]() {
-#pragma unroll
-        for (int i = 0; i < 24; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // VALU
-        }
-    };
-
     // Software pipeline over tiles: iteration j forms Sᵀ(j+1) and Oᵀ += P(j−1)
     // on MFMA while the VALU turns Sᵀ(j) into P(j).  The K ring holds tiles
     // j+1 (read) and j+2 (in flight), the Vᵀ ring j−1 (read) and j (in
     // flight).  The running reference m is raised only when a tile's maximum
-    // exceeds it by more than 8 (p ≤ 2^8 meanwhile); then Oᵀ, which then
-    // holds P(j−1) terms under the old m, is rescaled after this iteration's
-    // MFMAs.  (Two alternating register sets instead of the copies at the end
-    // of an iteration need more VGPRs than 3 waves per SIMD allow; the
-    // occupancy is worth more.)
+    // exceeds it by more than 8 (p ≤ 2^8 meanwhile); Oᵀ, which then holds terms
+    // up to P(j−1) under the old m, is rescaled at the start of iteration j+1,
+    // so that the products, the softmax and all else of an iteration are one
+    // basic block: with the branch at its end the compiler moved the
+    // exponentials past it, behind the MFMAs (16 heads × 5184² fp16 171 → 166 µs).
     const bool wave_live = q0 + wave * 32 < a.Nq;  // waves past the queries only move tiles
-    v16f s_cur = {}, s_next = {};
-    v8h ph_prev[2], pl_prev[2], ph_cur[2], pl_cur[2];
-    auto iter = [&](int j, auto has_qk, auto has_sm, auto masked, auto has_pv) {
+    struct Probs { v8h h[2], l[2]; };
+    v16f s_a = {}, s_b = {};
+    Probs p_a, p_b;
+    bool raised = false;  // the last step's maxima moved the reference: rescale Oᵀ by o_alpha
+    float o_alpha = 1.f;
+    // scores of tile j in s_cur, of tile j + 1 to s_next; P(j − 1) in prev, P(j) to cur
+    auto iter = [&](int j, v16f &s_cur, v16f &s_next, Probs &prev, Probs &cur, auto has_qk, auto has_sm,
+                    auto masked, auto has_pv) {
         wait_and_barrier<0>();  // K(j+1), Vᵀ(j−1) landed; tiles of j−1 released
         if (j + 2 < ntiles) issue_k(j + 2);
         if (j < ntiles) issue_v(j);
         if (!wave_live) return;
+        if constexpr (decltype(has_pv)::value) {
+            if (__any(raised)) {
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++) {
+                    // (at head dim 256 Oᵀ lives in AGPRs: without this the
+                    // compiler copies all of it out before the branch, every tile)
+                    if constexpr (HD == 256) __asm__("" : "+a"(o[dt]));
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[dt][r] *= o_alpha;
+                    if constexpr (HD == 256) __asm__("" : "+a"(o[dt]));
+                }
+            }
+        }
         bool raise = false;
         float mnew = mrun, alpha = 1.f, ps = 0.f;
         if constexpr (decltype(has_sm)::value) {
@@ -474,23 +536,17 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
             alpha = __builtin_amdgcn_exp2f(mrun - mnew);
         }
         if constexpr (decltype(has_qk)::value) s_next = qk(j + 1);
-        if constexpr (decltype(has_pv)::value) pv(j - 1, ph_prev, pl_prev);
-        if constexpr (decltype(has_sm)::value) ps = softmax(s_cur, mnew, ph_cur, pl_cur);
-        interleave();
+        if constexpr (decltype(has_pv)::value) pv(j - 1, prev.h, prev.l);
+        if constexpr (decltype(has_sm)::value) ps = softmax(s_cur, mnew, cur.h, cur.l);
         if constexpr (decltype(has_sm)::value) {
             lsum = lsum * alpha + ps;
-            if (__any(raise)) {
-#pragma unroll
-                for (int dt = 0; dt < G::DT; dt++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
-            }
             mrun = mnew;
+            raised = raise;
+            o_alpha = alpha;
         }
-        if constexpr (decltype(has_qk)::value) s_cur = s_next;
-        if constexpr (decltype(has_sm)::value) {
-#pragma unroll
-            for (int jj = 0; jj < 2; jj++) { ph_prev[jj] = ph_cur[jj]; pl_prev[jj] = pl_cur[jj]; }
+        if constexpr (!PAIRS) {
+            if constexpr (decltype(has_qk)::value) s_cur = s_next;
+            if constexpr (decltype(has_sm)::value) prev = cur;
         }
     };
     using T_ = std::true_type;
@@ -500,19 +556,35 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
     issue_k(0);
     if (ntiles > 1) issue_k(1);
     wait_and_barrier<0>();
-    if (wave_live) s_cur = qk(0);
+    if (wave_live) s_a = qk(0);
     // j = 0 .. ntiles: Sᵀ(j+1) while j+1 < ntiles, P(j) while j < ntiles
-    // (masked on a partial last tile), Oᵀ += P(j−1) from j = 1
+    // (masked on a partial last tile), Oᵀ += P(j−1) from j = 1.  Before each
+    // step S(j) is in s_a and P(j − 1) in p_b
+    auto swap = [&] {
+        if constexpr (PAIRS) { s_a = s_b; p_b = p_a; }
+    };
     if (ntiles == 1) {
-        if (partial) iter(0, F_{}, T_{}, T_{}, F_{});
-        else iter(0, F_{}, T_{}, F_{}, F_{});
+        if (partial) iter(0, s_a, s_b, p_b, p_a, F_{}, T_{}, T_{}, F_{});
+        else iter(0, s_a, s_b, p_b, p_a, F_{}, T_{}, F_{}, F_{});
     } else {
-        iter(0, T_{}, T_{}, F_{}, F_{});
-        for (int j = 1; j + 1 < ntiles; j++) iter(j, T_{}, T_{}, F_{}, T_{});
-        if (partial) iter(ntiles - 1, F_{}, T_{}, T_{}, T_{});
-        else iter(ntiles - 1, F_{}, T_{}, F_{}, T_{});
+        iter(0, s_a, s_b, p_b, p_a, T_{}, T_{}, F_{}, F_{});
+        swap();
+        int j = 1;
+        if constexpr (PAIRS) {
+            for (; j + 2 < ntiles; j += 2) {
+                iter(j, s_a, s_b, p_b, p_a, T_{}, T_{}, F_{}, T_{});
+                iter(j + 1, s_b, s_a, p_a, p_b, T_{}, T_{}, F_{}, T_{});
+            }
+        }
+        for (; j + 1 < ntiles; j++) {
+            iter(j, s_a, s_b, p_b, p_a, T_{}, T_{}, F_{}, T_{});
+            swap();
+        }
+        if (partial) iter(ntiles - 1, s_a, s_b, p_b, p_a, F_{}, T_{}, T_{}, T_{});
+        else iter(ntiles - 1, s_a, s_b, p_b, p_a, F_{}, T_{}, F_{}, T_{});
     }
-    iter(ntiles, F_{}, F_{}, F_{}, T_{});
+    swap();
+    iter(ntiles, s_a, s_b, p_b, p_a, F_{}, F_{}, F_{}, T_{});
 
     lsum += __shfl_xor(lsum, 32, 64);
     if (a.nsplit > 1) {
@@ -521,7 +593,7 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         if (qvalid) {
             const int64_t prow = ((int64_t)blockIdx.z * a.BH + bh) * a.Nq + qi;
 #pragma unroll
-            for (int dt = 0; dt < G::DT; dt++)
+            for (int dt = 0; dt < DT; dt++)
 #pragma unroll
                 for (int g = 0; g < 4; g++)
                     *(float4 *)(a.part_o + prow * HD + dt * 32 + 8 * g + 4 * lh) =
@@ -532,7 +604,7 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
     }
     const float inv = (lsum == 0.f) ? 0.f : 1.0f / lsum;
 #pragma unroll
-    for (int dt = 0; dt < G::DT; dt++)
+    for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[dt][r] *= inv;
 
@@ -560,7 +632,7 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
     const int hdo = (CROP && a.hd_out > 0) ? a.hd_out : HD;  // real head dim: padded columns are not stored
     const int64_t colbase = (int64_t)h * hdo;
 #pragma unroll
-    for (int dt = 0; dt < G::DT; dt++) {
+    for (int dt = 0; dt < DT; dt++) {
         if (CROP && dt * 32 >= hdo) break;
         if (out.kind == A_F6) {
             // the same Q8_0 codes in the A_F6 layout: this lane holds block
@@ -743,6 +815,7 @@ hipError_t launch_attn(const AttnArgs &a, hipStream_t st) {
     if (a.out.kind == A_F16X2 && (!a.out.lo || a.out.ld % 4 != 0)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((a.Nq + QT - 1) / QT), (unsigned)a.BH, (unsigned)a.nsplit);
     const bool crop = a.wo > 0 || (a.hd_out > 0 && a.hd_out != hd);
+    const bool hd96 = hd == 128 && a.hd_out > 0 && a.hd_out <= 96;
     if (a.kv_d != 0) {
         // Q (fp16, or f32) and K by strides, and V where it is given by rows
         const bool split = a.k_lo != nullptr;
@@ -760,9 +833,11 @@ hipError_t launch_attn(const AttnArgs &a, hipStream_t st) {
         if (a.k_lo) {
             if (hd == 64 && !crop) hipLaunchKernelGGL((k_attn<true, 64, false, true>), grid, dim3(NTHR), 0, st, a, ldv);
             else if (hd == 64) hipLaunchKernelGGL((k_attn<true, 64, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
+            else if (hd96) hipLaunchKernelGGL((k_attn<true, 128, true, true, true, 96>), grid, dim3(NTHR), 0, st, a, ldv);
             else hipLaunchKernelGGL((k_attn<true, 128, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
         } else if (hd == 64 && !crop) hipLaunchKernelGGL((k_attn<false, 64, false, true>), grid, dim3(NTHR), 0, st, a, ldv);
         else if (hd == 64) hipLaunchKernelGGL((k_attn<false, 64, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
+        else if (hd96) hipLaunchKernelGGL((k_attn<false, 128, true, true, true, 96>), grid, dim3(NTHR), 0, st, a, ldv);
         else hipLaunchKernelGGL((k_attn<false, 128, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
     } else if (hd == 256) {
         // (the strided form costs the plain layouts 1.6 % of a memory-attention pass)
@@ -774,6 +849,9 @@ hipError_t launch_attn(const AttnArgs &a, hipStream_t st) {
     } else if (hd == 64) {
         if (a.q_lo) hipLaunchKernelGGL((k_attn<true, 64, true>), grid, dim3(NTHR), 0, st, a, ldv);
         else hipLaunchKernelGGL((k_attn<false, 64, true>), grid, dim3(NTHR), 0, st, a, ldv);
+    } else if (hd96) {
+        if (a.q_lo) hipLaunchKernelGGL((k_attn<true, 128, true, false, false, 96>), grid, dim3(NTHR), 0, st, a, ldv);
+        else hipLaunchKernelGGL((k_attn<false, 128, true, false, false, 96>), grid, dim3(NTHR), 0, st, a, ldv);
     } else {
         if (a.q_lo) hipLaunchKernelGGL((k_attn<true, 128, true>), grid, dim3(NTHR), 0, st, a, ldv);
         else hipLaunchKernelGGL((k_attn<false, 128, true>), grid, dim3(NTHR), 0, st, a, ldv);
