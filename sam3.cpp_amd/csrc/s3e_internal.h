@@ -467,6 +467,89 @@ __device__ __forceinline__ void f6_split(float v, float id, float &h, float &l) 
     l = __builtin_fmaf(-16.f, h, q);
 }
 
+// Write 4 consecutive values (columns col..col+3, col % 4 == 0) in the
+// activation format.  For the Q8 formats the 8 lanes 8k..8k+7 of the wave
+// must hold the 8 float4 of one 32-element block, in order.
+__device__ __forceinline__ void emit4(const float *v, const Act &o, int64_t row, int64_t col, int lane) {
+    if (o.kind == A_F32) {
+        *(float4 *)((float *)o.x + row * o.ld + col) = make_float4(v[0], v[1], v[2], v[3]);
+        return;
+    }
+    if (o.kind == A_F16 || o.kind == A_F16X2) {
+        _Float16 h[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) h[i] = to_half(v[i]);
+        auto pack = [](_Float16 a, _Float16 b) {
+            return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+        };
+        *(uint2 *)((_Float16 *)o.x + row * o.ld + col) = make_uint2(pack(h[0], h[1]), pack(h[2], h[3]));
+        if (o.kind == A_F16X2) {
+            // low half: fp16 of the exact fp32 difference
+            _Float16 l[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) l[i] = (_Float16)(v[i] - (float)h[i]);
+            *(uint2 *)((_Float16 *)o.lo + row * o.ld + col) = make_uint2(pack(l[0], l[1]), pack(l[2], l[3]));
+        }
+        return;
+    }
+    // Q8_0 / Q8_1 as ggml's x86 quantize_row_q8_0 / q8_1: d = amax/127,
+    // id = 127/amax, q = round-half-even(v·id), s = fp16(d·Σq).
+    float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 4, 64));
+    const float d = amax / 127.f;
+    const float id = (amax != 0.f) ? 127.f / amax : 0.f;
+    if (o.kind == A_F6) {
+        // the same codes, split q = 16·h + l; lane k of the block's 8 holds
+        // bits [24k, 24k + 24) of each part's 192-bit operand string, and
+        // lanes 0-5 of the 8 each assemble and store one 8-byte word
+        uint32_t ph = 0, pl = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int q = (int)__builtin_rintf(v[i] * id);
+            const int h = f6_hi(q);
+            ph |= f6_code(h) << (6 * i);
+            pl |= f6_code(q - 16 * h) << (6 * i);
+        }
+        const int g = lane & ~7, k = lane & 7;
+        uint32_t x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const uint32_t a = __shfl(ph, g + j, 64), b = __shfl(pl, g + j, 64);
+            x[j] = k < 3 ? a : b;
+        }
+        if (k < 6) {
+            const int t = k % 3;
+            uint64_t w;
+            if (t == 0) w = (uint64_t)x[0] | ((uint64_t)x[1] << 24) | ((uint64_t)(x[2] & 0xFFFFu) << 48);
+            else if (t == 1) w = (uint64_t)(x[2] >> 16) | ((uint64_t)x[3] << 8) | ((uint64_t)x[4] << 32) | ((uint64_t)(x[5] & 0xFFu) << 56);
+            else w = (uint64_t)(x[5] >> 8) | ((uint64_t)x[6] << 16) | ((uint64_t)x[7] << 40);
+            ((uint64_t *)o.x)[f6_act_word(o.ld / 128, row, col / QK, k / 3, t)] = w;
+        }
+        if (k == 0) o.d[scale_index(o.mp, row, col / QK)] = half_bits(d);
+        return;
+    }
+    int sum = 0;
+    uint32_t packed = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int q = (int)__builtin_rintf(v[i] * id);
+        sum += q;
+        packed |= ((uint32_t)(q & 0xff)) << (8 * i);
+    }
+    *(uint32_t *)((int8_t *)o.x + row * o.ld + col) = packed;
+    sum += __shfl_xor(sum, 1, 64);
+    sum += __shfl_xor(sum, 2, 64);
+    sum += __shfl_xor(sum, 4, 64);
+    if ((lane & 7) == 0) {
+        const int64_t blk = scale_index(o.mp, row, col / QK);
+        o.d[blk] = half_bits(d);
+        // s = fp16(fp32(d·Σq)): f2h_bits keeps the fp32 rounding of the product
+        if (o.kind == A_Q8_1) o.s[blk] = half_bits(d * (float)sum);
+    }
+}
+
 // 16 / 8 bytes loaded through a global-address-space pointer.  A pointer the
 // compiler cannot place (one read from memory rather than a kernel argument)
 // makes a flat load, which may address LDS, so behind LDS DMA the compiler

@@ -53,7 +53,7 @@ struct MemAttnModel {
 struct MemAttnState {
     int64_t capN = 0, capM = 0;
     int D = 0, MD = 0, FFN = 0;
-    float *x = nullptr, *att = nullptr, *kvp = nullptr, *part_o = nullptr, *part_ml = nullptr;
+    float *x = nullptr, *kvp = nullptr, *part_o = nullptr, *part_ml = nullptr;
     int64_t part_cap = 0;           // rows of part_ml (and of part_o at D floats each)
     int64_t part_o_floats = 0;      // part_o also serves the K-split residual GEMMs
     ActBuf an, ah, am1, am2;
@@ -63,10 +63,10 @@ struct MemAttnState {
         ah.release();
         am1.release();
         am2.release();
-        for (void *p : {(void *)x, (void *)att, (void *)kvp, (void *)part_o, (void *)part_ml, (void *)q16, (void *)k16,
+        for (void *p : {(void *)x, (void *)kvp, (void *)part_o, (void *)part_ml, (void *)q16, (void *)k16,
                         (void *)vt16})
             if (p) (void)hipFree(p);
-        x = att = kvp = part_o = part_ml = nullptr;
+        x = kvp = part_o = part_ml = nullptr;
         q16 = k16 = vt16 = nullptr;
         capN = capM = part_cap = part_o_floats = 0;
     }
@@ -211,7 +211,6 @@ hipError_t grow(const MemAttnModel *m, MemAttnState *s, int64_t N, int64_t M, hi
     s->FFN = m->FFN;
     const int64_t D = m->D, MD = m->MD, NK = std::max(cN, cM);
     hipError_t e = hipMalloc(&s->x, (size_t)(cN * D * 4));
-    if (e == hipSuccess) e = hipMalloc(&s->att, (size_t)(cN * D * 4));
     if (e == hipSuccess) e = hipMalloc(&s->kvp, (size_t)(cM * MD * 4));
     if (e == hipSuccess) e = s->an.alloc(cN, D, st);
     if (e == hipSuccess) e = s->ah.alloc(cN, m->FFN, st);
@@ -297,7 +296,7 @@ int memattn_run(const MemAttnModel *m, MemAttnState **sp, const float *curr, con
         a.ld = ld;
         return a;
     };
-    auto attend = [&](int64_t Nkv, int ns) {
+    auto attend = [&](int64_t Nkv, int ns, const Act &out) {
         AttnArgs aa;
         aa.q = s->q16;
         aa.k = s->k16;
@@ -311,7 +310,7 @@ int memattn_run(const MemAttnModel *m, MemAttnState **sp, const float *curr, con
         aa.nsplit = ns;
         aa.part_o = s->part_o;
         aa.part_ml = s->part_ml;
-        aa.out = f32_act(s->att, D);
+        aa.out = out;
         return launch_attn(aa, st);
     };
     auto qkv_args = [&](const float *bias, int64_t rows, int sel0, const float *freqs, int64_t rope_rows) {
@@ -340,9 +339,8 @@ int memattn_run(const MemAttnModel *m, MemAttnState **sp, const float *curr, con
         const Act aq = s->an.as(act_kind_for(ly.sa_qkv.kind), D);
         MA_TRY(launch_layernorm(s->x, N, D, 1e-5f, ly.n1w, ly.n1b, aq, nullptr, st));
         MA_TRY(launch_gemm(ly.sa_qkv, aq, N, EPI_QKV, qkv_args(ly.sa_qkv_b, N, 0, rope_q, 0), st));
-        MA_TRY(attend(N, nsS));
         const Act ao = s->an.as(act_kind_for(ly.sa_out.kind), D);
-        MA_TRY(launch_rows_quant(ao.kind, s->att, N, D, ao, st));
+        MA_TRY(attend(N, nsS, ao));
         EpiArgs er;
         er.bias = ly.sa_out_b;
         er.y = s->x;
@@ -358,9 +356,8 @@ int memattn_run(const MemAttnModel *m, MemAttnState **sp, const float *curr, con
                            qkv_args(ly.ca_k_b, M, 1, Msp > 0 ? rope_k : nullptr, Msp), st));
         MA_TRY(launch_gemm(ly.ca_v, s->am2.as(act_kind_for(ly.ca_v.kind), MD), M, EPI_QKV,
                            qkv_args(ly.ca_v_b, M, 2, nullptr, 0), st));
-        MA_TRY(attend(M, nsC));
         const Act ao2 = s->an.as(act_kind_for(ly.ca_out.kind), D);
-        MA_TRY(launch_rows_quant(ao2.kind, s->att, N, D, ao2, st));
+        MA_TRY(attend(M, nsC, ao2));
         er.bias = ly.ca_out_b;
         MA_TRY(launch_gemm(ly.ca_out, ao2, N, EPI_RESID, er, st));
         // FFN with ReLU
