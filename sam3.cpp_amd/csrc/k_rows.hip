@@ -24,29 +24,38 @@ __device__ __forceinline__ double swz16_d(double v) {  // lane ^ 16 within each 
     return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
 }
 
-// Sum over the wave's 64 lanes, in every lane: DPP within rows of 16 (quad
-// xor 1, quad xor 2, half-row mirror, row mirror), a swizzle across the rows
-// of each half, a permute across the halves.  Only the last two wait on LDS.
+// Sum over each group of LPR lanes (16 or the whole wave), in every lane of
+// it: DPP within rows of 16 (quad xor 1, quad xor 2, half-row mirror, row
+// mirror), a swizzle across the rows of each half, a permute across the
+// halves.  Only the last two wait on LDS.
+template <int LPR = 64>
 __device__ __forceinline__ double wave_sum_d(double v) {
     v += dpp_d<0xB1>(v);   // quad_perm [1,0,3,2]
     v += dpp_d<0x4E>(v);   // quad_perm [2,3,0,1]
     v += dpp_d<0x141>(v);  // row_half_mirror
     v += dpp_d<0x140>(v);  // row_mirror
-    v += swz16_d(v);
-    v += __shfl_xor(v, 32, 64);
+    if constexpr (LPR == 64) {
+        v += swz16_d(v);
+        v += __shfl_xor(v, 32, 64);
+    }
     return v;
 }
 
-// One wave per row; lane L holds float4 number L + 64·it of the row
-// (it < NIT = ceil(E / 256)), so every load and store of the wave is one
-// contiguous run.
-template <int NIT>
+// LPR lanes per row (64, or 16 with four rows per wave); lane L of them holds
+// float4 number L + LPR·it of the row (it < NIT = ceil(E / (4·LPR))), so every
+// load and store is made of contiguous runs.  Rows of up to 128 values take 16
+// lanes: a whole wave leaves most lanes idle on them (24 of 64 work at 96
+// values), and the kernel is bound by the double-precision reduction's VALU
+// work, which four rows of a wave then share (65536 rows of 96: 21.3 → 10.6
+// µs).  Wider rows have enough lanes at work (4096 rows of 256: 4.8 µs on whole
+// waves, 5.5 on 16 lanes, whose loads are fewer and longer chains).
+template <int NIT, int LPR>
 __global__ __launch_bounds__(256) void k_layernorm(const float *__restrict__ x, int64_t M, int64_t E,
                                                    float eps, const float *__restrict__ w,
                                                    const float *__restrict__ b, Act o,
                                                    float *__restrict__ y32) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & (LPR - 1);
+    const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
     if (row >= M) return;
     const int nf4 = (int)(E / 4);
     const float4 *xr = (const float4 *)(x + row * E);
@@ -57,7 +66,7 @@ __global__ __launch_bounds__(256) void k_layernorm(const float *__restrict__ x, 
     // matches the CPU path bit for bit.
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
-        const int f = lane + 64 * it;
+        const int f = lane + LPR * it;
         const float4 q = (f < nf4) ? xr[f] : make_float4(0.f, 0.f, 0.f, 0.f);
         v[it][0] = q.x; v[it][1] = q.y; v[it][2] = q.z; v[it][3] = q.w;
     }
@@ -66,12 +75,12 @@ __global__ __launch_bounds__(256) void k_layernorm(const float *__restrict__ x, 
     for (int it = 0; it < NIT; it++)
 #pragma unroll
         for (int j = 0; j < 4; j++) s += (double)v[it][j];
-    s = wave_sum_d(s);
+    s = wave_sum_d<LPR>(s);
     const float mean = (float)(s / (double)E);
     double s2 = 0.0;
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
-        const bool ok = lane + 64 * it < nf4;
+        const bool ok = lane + LPR * it < nf4;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const float c = __fsub_rn(v[it][j], mean);
@@ -79,13 +88,13 @@ __global__ __launch_bounds__(256) void k_layernorm(const float *__restrict__ x, 
             if (ok) s2 += (double)__fmul_rn(c, c);
         }
     }
-    s2 = wave_sum_d(s2);
+    s2 = wave_sum_d<LPR>(s2);
     const float var = (float)(s2 / (double)E);
     const float scale = 1.0f / sqrtf(var + eps);
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
-        const int f = lane + 64 * it;
-        if (64 * it >= nf4) break;  // whole wave past the row (nf4 is a multiple of 8)
+        const int f = lane + LPR * it;
+        if (LPR * it >= nf4) break;  // every lane past the row (nf4 is a multiple of 8)
         if (f < nf4) {
             const float4 wf = w ? ((const float4 *)w)[f] : make_float4(1.f, 1.f, 1.f, 1.f);
             const float4 bf = b ? ((const float4 *)b)[f] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -101,7 +110,7 @@ __global__ __launch_bounds__(256) void k_layernorm(const float *__restrict__ x, 
         // the 8 lanes of a Q8 block are all inside or all past the row
         if (f < nf4) {
             if (y32) *(float4 *)(y32 + row * E + 4 * f) = make_float4(v[it][0], v[it][1], v[it][2], v[it][3]);
-            else emit4(v[it], o, row, 4 * (int64_t)f, lane);
+            else emit4(v[it], o, row, 4 * (int64_t)f, (int)(threadIdx.x & 63));
         }
     }
 }
@@ -489,7 +498,6 @@ hipError_t launch_layernorm(const float *x, int64_t M, int64_t E, float eps, con
     const bool q8 = !y_f32 && (out.kind == A_Q8_0 || out.kind == A_Q8_1);
     const bool f6 = !y_f32 && out.kind == A_F6;
     if (E % 4 != 0 || E > 4096 || (q8 && E % 32 != 0) || (f6 && (E % 128 != 0 || out.ld != E))) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((M + 3) / 4));
     if (f6 && E <= 1024 && (w != nullptr) == (b != nullptr)) {
         // rows of up to 1024 (the ViT's); the ViT's norms carry both gamma and
         // beta (sam3_layer_norm, sam3.cpp:1037-1046)
@@ -499,11 +507,17 @@ hipError_t launch_layernorm(const float *x, int64_t M, int64_t E, float eps, con
         else hipLaunchKernelGGL((k_layernorm_f6<1, false, W>), gf, dim3(64 * W), 0, st, x, M, E, eps, w, b, out);
         return hipGetLastError();
     }
-    if (E <= 256) hipLaunchKernelGGL(k_layernorm<1>, grid, dim3(256), 0, st, x, M, E, eps, w, b, out, y_f32);
-    else if (E <= 512) hipLaunchKernelGGL(k_layernorm<2>, grid, dim3(256), 0, st, x, M, E, eps, w, b, out, y_f32);
-    else if (E <= 1024) hipLaunchKernelGGL(k_layernorm<4>, grid, dim3(256), 0, st, x, M, E, eps, w, b, out, y_f32);
-    else if (E <= 2048) hipLaunchKernelGGL(k_layernorm<8>, grid, dim3(256), 0, st, x, M, E, eps, w, b, out, y_f32);
-    else hipLaunchKernelGGL(k_layernorm<16>, grid, dim3(256), 0, st, x, M, E, eps, w, b, out, y_f32);
+    auto run = [&](auto kernel, int rows_per_wg) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((M + rows_per_wg - 1) / rows_per_wg)), dim3(256), 0, st, x, M, E, eps,
+                           w, b, out, y_f32);
+    };
+    if (E <= 64) run(k_layernorm<1, 16>, 16);
+    else if (E <= 128) run(k_layernorm<2, 16>, 16);
+    else if (E <= 256) run(k_layernorm<1, 64>, 4);
+    else if (E <= 512) run(k_layernorm<2, 64>, 4);
+    else if (E <= 1024) run(k_layernorm<4, 64>, 4);
+    else if (E <= 2048) run(k_layernorm<8, 64>, 4);
+    else run(k_layernorm<16, 64>, 4);
     return hipGetLastError();
 }
 
