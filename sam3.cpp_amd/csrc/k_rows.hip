@@ -125,7 +125,9 @@ __global__ __launch_bounds__(256) void k_layernorm(const float *__restrict__ x, 
 // the work-group then writes every (block, part, word) run of its 16 rows
 // (128 contiguous bytes in A_F6) and every stage's 16 rows of block scales
 // as whole lines.  The same statistics and per-element operations as
-// k_layernorm, so the same codes.
+// k_layernorm, so the same codes.  NORM = false converts the rows as they are:
+// work-groups of 16 rows × 1024 columns (blockIdx.y), whole lines out instead
+// of scattered 8-byte words and 16 shuffles per float4 (5184 × 1024: 13.4 → 9.2 µs).
 constexpr int LNF6_ROWS = 16;
 // waves per work-group, LNF6_ROWS / LNF6_WAVES rows each: one row per wave
 // (no chain of dependent row loads; 5184 rows: 11.42 → 11.33 ms per ViT frame
@@ -133,7 +135,7 @@ constexpr int LNF6_ROWS = 16;
 constexpr int LNF6_WAVES = 16;
 constexpr int LNF6_BSTRIDE = 98;  // 8-byte LDS words per block: 6 runs of 16 rows, padded (bank spread, 16 B aligned)
 
-template <int NIT, bool WB, int LNW>
+template <int NIT, bool WB, int LNW, bool NORM = true>
 __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restrict__ x, int64_t M, int64_t E,
                                                       float eps, const float *__restrict__ w,
                                                       const float *__restrict__ b, Act o) {
@@ -142,7 +144,9 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
     // gamma and beta, read once per work-group (every wave's row uses all of them)
     __shared__ __attribute__((aligned(16))) float swb[WB ? 2 * 1024 * NIT : 4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nseg = (int)(E / 16), nblk = (int)(E / 32);
+    // this work-group's columns c0 .. c0 + 16·nseg
+    const int c0 = NORM ? 0 : (int)blockIdx.y * 1024;
+    const int nseg = NORM ? (int)(E / 16) : min((int)E - c0, 1024) / 16, nblk = nseg / 2;
     const int64_t r0 = (int64_t)blockIdx.x * LNF6_ROWS;
     uint32_t *stg32 = (uint32_t *)stg;
     // pairwise sums in double (exact enough that the order never shows in
@@ -157,7 +161,7 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
     };
     float nx[NIT][16];
     auto load_row = [&](int64_t r) {
-        const float4 *xr = (const float4 *)(x + r * E);
+        const float4 *xr = (const float4 *)(x + r * E + c0);
 #pragma unroll
         for (int it = 0; it < NIT; it++) {
             const int seg = lane + 64 * it;
@@ -192,26 +196,29 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
 #pragma unroll
             for (int j = 0; j < 16; j++) v[it][j] = nx[it][j];
         if (k + 1 < RPW && row + 1 < M) load_row(row + 1);
-        double s = 0.0;
+        float scale = 1.f;
+        if constexpr (NORM) {
+            double s = 0.0;
 #pragma unroll
-        for (int it = 0; it < NIT; it++) s += dsum16(v[it]);
-        s = wave_sum_d(s);
-        const float mean = (float)(s / (double)E);
-        double s2 = 0.0;
+            for (int it = 0; it < NIT; it++) s += dsum16(v[it]);
+            s = wave_sum_d(s);
+            const float mean = (float)(s / (double)E);
+            double s2 = 0.0;
 #pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            float sq[16];
+            for (int it = 0; it < NIT; it++) {
+                float sq[16];
 #pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const float c = __fsub_rn(v[it][j], mean);
-                v[it][j] = c;
-                sq[j] = __fmul_rn(c, c);
+                for (int j = 0; j < 16; j++) {
+                    const float c = __fsub_rn(v[it][j], mean);
+                    v[it][j] = c;
+                    sq[j] = __fmul_rn(c, c);
+                }
+                if (lane + 64 * it < nseg) s2 += dsum16(sq);
             }
-            if (lane + 64 * it < nseg) s2 += dsum16(sq);
+            s2 = wave_sum_d(s2);
+            const float var = (float)(s2 / (double)E);
+            scale = 1.0f / sqrtf(var + eps);
         }
-        s2 = wave_sum_d(s2);
-        const float var = (float)(s2 / (double)E);
-        const float scale = 1.0f / sqrtf(var + eps);
 #pragma unroll
         for (int it = 0; it < NIT; it++) {
             const int seg = lane + 64 * it;
@@ -230,7 +237,8 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
                 }
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    float t = __fmul_rn(v[it][4 * j4 + j], scale);
+                    float t = v[it][4 * j4 + j];
+                    if constexpr (NORM) t = __fmul_rn(t, scale);
                     if constexpr (WB) t = __fadd_rn(__fmul_rn(t, wv[j]), bv[j]);
                     v[it][4 * j4 + j] = t;
                     amax = fmaxf(amax, fabsf(t));
@@ -246,8 +254,8 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 float a, c, e, g;
-                f6_split(v[it][2 * i], id, a, c);
-                f6_split(v[it][2 * i + 1], id, e, g);
+                f6_split<!NORM>(v[it][2 * i], id, a, c);
+                f6_split<!NORM>(v[it][2 * i + 1], id, e, g);
                 ev[i] = a;
                 od[i] = e;
                 ev[8 + i] = c;
@@ -284,13 +292,13 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
         const int blk = run / 6, pt = run % 6;
         if (r0 + 2 * q >= M) continue;
         const uint4 val = *(const uint4 *)(stg + blk * LNF6_BSTRIDE + pt * 16 + 2 * q);
-        *(uint4 *)((uint64_t *)o.x + f6_act_word(nst, r0, blk, pt / 3, pt % 3) + 2 * q) = val;
+        *(uint4 *)((uint64_t *)o.x + f6_act_word(nst, r0, c0 / 32 + blk, pt / 3, pt % 3) + 2 * q) = val;
     }
     // block scales: per stage, 16 rows × 4 fp16 = 128 contiguous bytes
     for (int pc = threadIdx.x; pc < (nblk / 4) * 8; pc += 64 * LNW) {
         const int sg = pc >> 3, q = pc & 7;
         if (r0 + 2 * q >= M) continue;
-        *(uint4 *)(o.d + scale_index(o.mp, r0 + 2 * q, 4 * sg)) = *(const uint4 *)&stgd[sg][2 * q][0];
+        *(uint4 *)(o.d + scale_index(o.mp, r0 + 2 * q, c0 / 32 + 4 * sg)) = *(const uint4 *)&stgd[sg][2 * q][0];
     }
 }
 
@@ -529,6 +537,12 @@ hipError_t launch_rows_quant(AKind kind, const float *x, int64_t M, int64_t K, c
     if ((q8 && K % 32 != 0) || K % 4 != 0 || (out.kind == A_F6 && (K % 128 != 0 || out.ld != K)))
         return hipErrorInvalidValue;
     if (M <= 0) return hipSuccess;  // no rows: a launch would have an empty grid
+    if (out.kind == A_F6) {
+        const dim3 gf((unsigned)((M + LNF6_ROWS - 1) / LNF6_ROWS), (unsigned)((K + 1023) / 1024));
+        hipLaunchKernelGGL((k_layernorm_f6<1, false, LNF6_WAVES, false>), gf, dim3(64 * LNF6_WAVES), 0, st, x, M, K, 0.f,
+                           (const float *)nullptr, (const float *)nullptr, out);
+        return hipGetLastError();
+    }
     const int64_t nf4 = (K + 127) / 128 * 32;  // float4 up to the 128-element group
     const dim3 grid((unsigned)((nf4 + 63) / 64), (unsigned)((M + 3) / 4));
     hipLaunchKernelGGL(k_rows_quant, grid, dim3(256), 0, st, x, M, K, out);
