@@ -4,13 +4,19 @@
 // (v − 0.5)/0.5) or sam2_preprocess_image (sam3.cpp:3518-3544, ImageNet mean
 // and std).
 //
-// One thread per output pixel computes its three channels.  The resize runs
-// in double precision with the reference's operation order (half-pixel
-// centres clamped at 0, edge replication on the high side, weights
+// The resize runs in double precision with the reference's operation order
+// (half-pixel centres clamped at 0, edge replication on the high side, weights
 // (1 − w, w), round half up by truncating v + 0.5), so the resized bytes are
 // the reference's bit for bit: every step is a correctly rounded IEEE
 // operation on both sides and no contraction happens (-ffp-contract=off).
-// The normalisation is two correctly rounded f32 operations, as on the host.
+// The normalisation is two correctly rounded f32 operations, as on the host;
+// it depends on the byte and the channel alone, so a work-group makes the 768
+// results once and looks them up.
+//
+// A thread computes PX neighbouring pixels of a row.  What bounds the kernel is
+// instructions, not its 18 MB (1920×1080 → 1008²): the scale quotients come
+// from the host, and the six bytes that a pixel needs of a source row are two
+// 4-byte loads instead of six of one byte.  8.0 → 6.8 µs a call.
 #include "s3e_internal.h"
 
 namespace s3e {
@@ -20,44 +26,90 @@ struct PrepImg {
     const uint8_t *hwc;
     float *chw;
     int w, h, S, norm;
+    double sx, sy;  // source pixels per output pixel
 };
 
+constexpr int PX = 2;  // pixels per thread
+
+// the two neighbouring pixels at b of a row (6 bytes), packed: channels of
+// the first in bytes 0-2 of .x, of the second in bytes 1-3 of .y
+__device__ __forceinline__ uint2 pixel_pair(const uint8_t *row, int b) {
+    uint2 v;
+    __builtin_memcpy(&v.x, row + 3 * b, 4);
+    __builtin_memcpy(&v.y, row + 3 * b + 2, 4);
+    return v;
+}
+
 __global__ __launch_bounds__(256) void k_preprocess(PrepImg p) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t plane = (int64_t)p.S * p.S;
-    if (i >= plane) return;
-    const int y = (int)(i / p.S), x = (int)(i - (int64_t)y * p.S);
-    float v[3];
-    if (p.w == p.S && p.h == p.S) {
-        const uint8_t *q = p.hwc + i * 3;
+    __shared__ float lut[3][256];
+    {
+        const float mean[3] = {0.485f, 0.456f, 0.406f}, stdv[3] = {0.229f, 0.224f, 0.225f};
+        const float u = (float)threadIdx.x / 255.0f;
 #pragma unroll
-        for (int c = 0; c < 3; c++) v[c] = (float)q[c];
-    } else {
-        const double sx = (double)p.w / p.S, sy = (double)p.h / p.S;
-        double fy = (y + 0.5) * sy - 0.5;
-        if (fy < 0.0) fy = 0.0;
-        const int y0 = (int)fy, y1 = (y0 < p.h - 1) ? y0 + 1 : y0;
-        const double wy = fy - y0, wy0 = 1.0 - wy;
-        double fx = (x + 0.5) * sx - 0.5;
+        for (int c = 0; c < 3; c++) lut[c][threadIdx.x] = p.norm == 1 ? (u - mean[c]) / stdv[c] : (u - 0.5f) / 0.5f;
+    }
+    __syncthreads();
+    const int per_row = (p.S + PX - 1) / PX;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)per_row * p.S) return;
+    const int y = (int)(i / per_row), xs = (int)(i - (int64_t)y * per_row) * PX;
+    const bool same = p.w == p.S && p.h == p.S;
+    double fy = (y + 0.5) * p.sy - 0.5;
+    if (fy < 0.0) fy = 0.0;
+    const int y0 = (int)fy, y1 = (y0 < p.h - 1) ? y0 + 1 : y0;
+    const double wy = fy - y0, wy0 = 1.0 - wy;
+    const uint8_t *r0 = p.hwc + (int64_t)y0 * p.w * 3, *r1 = p.hwc + (int64_t)y1 * p.w * 3;
+    int iv[PX][3];
+#pragma unroll
+    for (int j = 0; j < PX; j++) {
+        const int x = min(xs + j, p.S - 1);
+        if (same) {
+            const uint8_t *q = p.hwc + ((int64_t)y * p.S + x) * 3;
+#pragma unroll
+            for (int c = 0; c < 3; c++) iv[j][c] = q[c];
+            continue;
+        }
+        double fx = (x + 0.5) * p.sx - 0.5;
         if (fx < 0.0) fx = 0.0;
-        const int x0 = (int)fx, x1 = (x0 < p.w - 1) ? x0 + 1 : x0;
+        const int x0 = (int)fx;
         const double wx = fx - x0, wx0 = 1.0 - wx;
-        const uint8_t *r0 = p.hwc + (int64_t)y0 * p.w * 3, *r1 = p.hwc + (int64_t)y1 * p.w * 3;
+        // pixels x0 and x0 + 1, the last one twice at the right edge
+        const bool edge = x0 >= p.w - 1;
+        const int b = edge ? p.w - 2 : x0;
+        uint2 t, u;
+        if (p.w > 1) {
+            t = pixel_pair(r0, b);
+            u = pixel_pair(r1, b);
+        } else {
+            t.x = r0[0] | (uint32_t)r0[1] << 8 | (uint32_t)r0[2] << 16;
+            u.x = r1[0] | (uint32_t)r1[1] << 8 | (uint32_t)r1[2] << 16;
+            t.y = t.x << 8;
+            u.y = u.x << 8;
+        }
+        if (edge) {
+            t.x = t.y >> 8;
+            u.x = u.y >> 8;
+        }
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const double p00 = r0[x0 * 3 + c], p01 = r0[x1 * 3 + c];
-            const double p10 = r1[x0 * 3 + c], p11 = r1[x1 * 3 + c];
+            const double p00 = (t.x >> (8 * c)) & 0xffu, p01 = (t.y >> (8 * c + 8)) & 0xffu;
+            const double p10 = (u.x >> (8 * c)) & 0xffu, p11 = (u.y >> (8 * c + 8)) & 0xffu;
             const double vv = wy0 * (wx0 * p00 + wx * p01) + wy * (wx0 * p10 + wx * p11);
-            int iv = (int)(vv + 0.5);
-            iv = iv < 0 ? 0 : (iv > 255 ? 255 : iv);
-            v[c] = (float)iv;
+            const int v = (int)(vv + 0.5);
+            iv[j][c] = v < 0 ? 0 : (v > 255 ? 255 : v);
         }
     }
-    const float mean[3] = {0.485f, 0.456f, 0.406f}, stdv[3] = {0.229f, 0.224f, 0.225f};
+    const int64_t plane = (int64_t)p.S * p.S, o = (int64_t)y * p.S + xs;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        const float u = v[c] / 255.0f;
-        p.chw[c * plane + i] = p.norm == 1 ? (u - mean[c]) / stdv[c] : (u - 0.5f) / 0.5f;
+        float *dst = p.chw + c * plane + o;
+        if (PX == 2 && p.S % 2 == 0 && (uintptr_t)p.chw % 8 == 0) {
+            *(float2 *)dst = make_float2(lut[c][iv[0][c]], lut[c][iv[PX - 1][c]]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < PX; j++)
+                if (xs + j < p.S) dst[j] = lut[c][iv[j][c]];
+        }
     }
 }
 
@@ -67,8 +119,8 @@ hipError_t launch_preprocess(const uint8_t *hwc, int w, int h, int S, int norm, 
     if (!hwc || !chw || w <= 0 || h <= 0 || S <= 0 || (norm != 0 && norm != 1)) return hipErrorInvalidValue;
     // byte offsets of the source stay within int for the per-row index math
     if ((int64_t)w * 3 > INT32_MAX / 2) return hipErrorInvalidValue;
-    const PrepImg p{hwc, chw, w, h, S, norm};
-    const int64_t n = (int64_t)S * S;
+    const PrepImg p{hwc, chw, w, h, S, norm, (double)w / S, (double)h / S};
+    const int64_t n = (int64_t)S * ((S + PX - 1) / PX);
     hipLaunchKernelGGL(k_preprocess, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
     return hipGetLastError();
 }
