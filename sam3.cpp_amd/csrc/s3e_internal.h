@@ -442,6 +442,24 @@ __device__ __forceinline__ float gelu_erf(float x) {
     return 0.5f * x * w;
 }
 
+// ggml_gelu of the fp16 value xh, as ggml's fp16 table holds it, without
+// looking it up where the result is certain: y = xh / (1 + e^(−2u)), u =
+// √(2/π)·xh·(1 + 0.044715·xh²), is 0.5·xh·(1 + tanh u) up to the rounding
+// errors of both: at most 1.1e-7·|x| for the table's fp32 evaluation (the
+// rounding of 1 + tanh u and of tanh) and 5e-7·|y| for this one.  Where fp16
+// rounds both ends of that interval alike, `certain` is set and the result is
+// the table's entry bit for bit; else the caller looks it up (0.3 % of
+// standard normal values, most below −2.5).
+__device__ __forceinline__ uint16_t gelu_tanh_half(_Float16 xh, bool &certain) {
+    const float x = (float)xh;
+    const float a = x * __builtin_fmaf(x * x, -0.10294324f, -2.30220819f);  // −2u·log2(e)
+    const float y = x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(a));
+    const float eps = __builtin_fmaf(fabsf(y), 6e-7f, fabsf(x) * 1.3e-7f);
+    const uint16_t lo = __builtin_bit_cast(uint16_t, (_Float16)(y - eps)), hi = __builtin_bit_cast(uint16_t, (_Float16)(y + eps));
+    certain = lo == hi;
+    return lo;
+}
+
 // ---- fp6 (E3M2) operand strings on the device ----
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x6 __attribute__((ext_vector_type(6)));
