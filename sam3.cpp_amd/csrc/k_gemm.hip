@@ -261,9 +261,11 @@ __device__ __forceinline__ void activate(const EpiArgs &e, const float *bias, fl
 }
 
 // Epilogue from the fp32 tile Ct [BM][CLD] in LDS (scaled, complete), run by
-// the NT_ threads of the work-group.
+// the NT_ threads of the work-group.  tab: EPI_TAB<EPI, BM> bytes of LDS.
+template <int EPI, int BM>
+constexpr int EPI_TAB = EPI == EPI_HQKV ? 4 * (2 * BM + BN) : 0;
 template <int EPI, int BM, int NT_, bool TABLE = true>
-__device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, int m0, int n0, int t) {
+__device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, int *tab, int m0, int n0, int t) {
     const EpiArgs &e = p.e;
     if constexpr (EPI == EPI_QKV) {
         const int sel = n0 / e.E + e.sel0;  // 0 = Q, 1 = K, 2 = V (a tile never straddles)
@@ -373,8 +375,31 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
         const int C = e.E, HD = e.HD, HDp = e.hdp, W = e.grid;
         const int wh = e.window > 0 ? e.window : e.grid_h, ww = e.window > 0 ? e.window : W;
         const int nwx = (W + ww - 1) / ww, Nkv = wh * ww;
+        // Where a row and a column go, worked out once per tile: (window,
+        // position in it) of the BM tokens and (Q / K / V / none, head,
+        // channel) of the BN columns.  Done per stored piece, the divisions
+        // were most of the kernel: 65536 × 576 × 96 fp16 63 µs, now 55.
+        int2 *const tok = (int2 *)tab;
+        int *const colw = tab + 2 * BM;
+        for (int i = t; i < BM + BN; i += NT_) {
+            if (i < BM) {
+                const int gm = m0 + i;
+                int2 v = make_int2(-1, 0);
+                if (gm < p.M) {
+                    const int py = gm / W, px = gm - py * W, wy = py / wh, wx = px / ww;
+                    v = make_int2(wy * nwx + wx, (py - wy * wh) * ww + px - wx * ww);
+                }
+                tok[i] = v;
+            } else {
+                const int gn = n0 + i - BM;
+                const int sel = gn < C ? 0 : gn < 2 * C ? 1 : gn < 3 * C ? 2 : 3;
+                const int r2 = gn - sel * C, h = r2 / HD;
+                colw[i - BM] = sel == 3 ? 3 << 28 : sel << 28 | h << 12 | (r2 - h * HD);
+            }
+        }
+        __syncthreads();
         // Q, K: a unit is one token and 8 columns (one 16-byte store per plane)
-        for (int u = t; u < BM * (BN / 8); u += NT_) {
+        for (int u = t; u < BM * (BN / 8) && n0 < 2 * C; u += NT_) {
             const int row = u / (BN / 8), cc = u % (BN / 8);
             const int gm = m0 + row, gn0 = n0 + cc * 8;
             if (gm >= p.M || gn0 >= 2 * C) continue;
@@ -388,17 +413,14 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
                 v[4] = x1.x + b1.x; v[5] = x1.y + b1.y; v[6] = x1.z + b1.z; v[7] = x1.w + b1.w;
             }
             const int sel = gn0 >= C;
-            const int r2 = gn0 - sel * C;
             if (sel == 0 && e.qpool) {  // Q rows for the pooling pass
-                float4 *dst = (float4 *)(e.y + (int64_t)gm * e.ldy + r2);
+                float4 *dst = (float4 *)(e.y + (int64_t)gm * e.ldy + gn0);
                 dst[0] = make_float4(v[0], v[1], v[2], v[3]);
                 dst[1] = make_float4(v[4], v[5], v[6], v[7]);
                 continue;
             }
-            const int h = r2 / HD, d0 = r2 % HD;
-            const int py = gm / W, px = gm % W;
-            const int b = (py / wh) * nwx + px / ww;
-            const int pp = (py % wh) * ww + px % ww;
+            const int2 tk = tok[row];
+            const int cw = colw[cc * 8], h = cw >> 12 & 0xffff, d0 = cw & 0xfff, b = tk.x, pp = tk.y;
             const int64_t o = ((int64_t)(b * e.NH + h) * Nkv + pp) * HDp + d0;
             _Float16 *hi = sel == 0 ? e.q : e.k;
             _Float16 *lo = sel == 0 ? e.q_lo : e.k_lo;
@@ -423,37 +445,29 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
         // store instruction covers runs of consecutive key slots; a pair that
         // stays inside one window row at an even position fills two adjacent
         // slots (vt_slot keeps aligned pairs together) with one 4-byte store
-        for (int u = t; u < (BM / 2) * BN; u += NT_) {
+        for (int u = t; u < (BM / 2) * BN && n0 + BN > 2 * C; u += NT_) {
             const int rp = u % (BM / 2), col = u / (BM / 2);
             const int gm = m0 + 2 * rp, gn = n0 + col;
             if (gm >= p.M || gn < 2 * C || gn >= 3 * C) continue;
             const float bv = e.bias[gn];
             const float v0 = Ct[(2 * rp) * CLD + col] + bv, v1 = Ct[(2 * rp + 1) * CLD + col] + bv;
-            const int r2 = gn - 2 * C;
-            const int h = r2 / HD, d = r2 % HD;
-            const int py = gm / W, px = gm % W;
-            const int b = (py / wh) * nwx + px / ww;
-            const int pp = (py % wh) * ww + px % ww;
-            const int64_t base = ((int64_t)(b * e.NH + h) * HDp + d) * e.vt_ld;
+            const int cw = colw[col], h = cw >> 12 & 0xffff, d = cw & 0xfff;
+            const int2 t0 = tok[2 * rp], t1 = tok[2 * rp + 1];
+            const int64_t ch = (int64_t)h * HDp + d, base = ((int64_t)t0.x * e.NH * HDp + ch) * e.vt_ld;
             const _Float16 h0 = to_half(v0), h1 = to_half(v1);
             const _Float16 l0 = (_Float16)(v0 - (float)h0), l1 = (_Float16)(v1 - (float)h1);
-            const bool pair = gm + 1 < p.M && px + 1 < W && (px % ww) + 1 < ww && (pp & 1) == 0;
-            if (pair) {
-                const int64_t o = base + vt_slot(pp);
+            const int64_t o = base + vt_slot(t0.y);
+            if (t1.x == t0.x && t1.y == t0.y + 1 && (t0.y & 1) == 0) {
                 *(uint32_t *)(e.vt + o) =
                     (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
                 if (e.vt_lo)
                     *(uint32_t *)(e.vt_lo + o) =
                         (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
             } else {
-                const int64_t o = base + vt_slot(pp);
                 e.vt[o] = h0;
                 if (e.vt_lo) e.vt_lo[o] = l0;
-                if (gm + 1 < p.M) {
-                    const int pyb = (gm + 1) / W, pxb = (gm + 1) % W;
-                    const int bb = (pyb / wh) * nwx + pxb / ww;
-                    const int ppb = (pyb % wh) * ww + pxb % ww;
-                    const int64_t ob = ((int64_t)(bb * e.NH + h) * HDp + d) * e.vt_ld + vt_slot(ppb);
+                if (t1.x >= 0) {
+                    const int64_t ob = ((int64_t)t1.x * e.NH * HDp + ch) * e.vt_ld + vt_slot(t1.y);
                     e.vt[ob] = h1;
                     if (e.vt_lo) e.vt_lo[ob] = l1;
                 }
@@ -659,7 +673,8 @@ template <int WK, int EPI, int BM, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 3 : 256 / BM) void k_gemm(GemmParams p) {
     using C = Cfg<WK, BM, WAVES>;
     constexpr int MT = C::MT, NT = C::NT, NBUF = C::NBUF;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS + EPI_TAB<EPI, BM>];
+    int *const tab = (int *)(lds + C::LDS);
 
     // ---- tile of this work-group (and its K range when split) ----
     const int per = gridDim.x >> 3;
@@ -1025,11 +1040,11 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 3 : 256 / BM) void k_gemm(
             q.e.y = p.part + (int64_t)kpart * p.M * p.N;
             q.e.ldy = p.N;
             q.e.bias = nullptr;
-            epilogue<EPI_F32, BM, C::NTH>(q, Ct, m0, n0, t);
+            epilogue<EPI_F32, BM, C::NTH>(q, Ct, nullptr, m0, n0, t);
             return;
         }
     }
-    epilogue<EPI, BM, C::NTH>(p, Ct, m0, n0, t);
+    epilogue<EPI, BM, C::NTH>(p, Ct, tab, m0, n0, t);
 }
 
 // ---- Q4_0 weights × A_F6 activations --------------------------------------
@@ -1216,11 +1231,11 @@ __global__ __launch_bounds__(256, 3) void k_gemm_f6(GemmParams p) {
             q.e.y = p.part + (int64_t)kpart * p.M * p.N;
             q.e.ldy = p.N;
             q.e.bias = nullptr;
-            epilogue<EPI_F32, BM, NTH>(q, Ct, m0, n0, t);
+            epilogue<EPI_F32, BM, NTH>(q, Ct, nullptr, m0, n0, t);
             return;
         }
     }
-    epilogue<EPI, BM, NTH, false>(p, Ct, m0, n0, t);  // (no table: its registers would spill here)
+    epilogue<EPI, BM, NTH, false>(p, Ct, nullptr, m0, n0, t);  // (no table: its registers would spill here)
 }
 
 // y = Σ_k part[k] (+ bias) for EPI_F32, y += Σ_k part[k] (+ bias) for
