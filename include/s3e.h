@@ -109,7 +109,10 @@ int s3e_weight_info(const s3e_weight *w, int64_t out[4]);
  * The converted X lives in a workspace that the context keeps and shares
  * with s3e_flash_attn_ext, as large as the largest call so far (freed with the
  * context); a call that needs more than 1 GiB allocates for itself.  Calls
- * that convert wait for their result before they return. */
+ * that convert wait for their result before they return.  Products with few
+ * output tiles add up K in ranges whose partial sums take 25 MB of the context
+ * (made once; not while its stream is being captured: a captured s3e_mul_mat_q
+ * sums K in one range, equal up to fp32 summation order). */
 int s3e_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const float *X, int64_t M,
                 const float *bias, float *Y);
 

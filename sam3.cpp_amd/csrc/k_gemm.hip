@@ -66,7 +66,7 @@ constexpr int CLD = BN + 4;   // fp32 C-tile row stride
 // 3-deep ring, 4 waves per SIMD at BM = 64 (two work-groups per CU).
 // WAVES = 4: waves 2 × 2, each BM/2 × 64 (two MFMA column tiles share one A
 // fragment and one scale operand), 2-deep ring, three work-groups per CU.
-template <int WK, int BM_, int WAVES_>
+template <int WK, int BM_, int WAVES_, int NBUF_ = 0>
 struct Cfg {
     static constexpr int BM = BM_;
     static constexpr int WAVES = WAVES_;
@@ -80,7 +80,7 @@ struct Cfg {
     static constexpr int WM = 2, WN = WAVES / 2;
     static constexpr int MT = BM / (32 * WM);            // 32-row MFMA tiles per wave
     static constexpr int NT = BN / (32 * WN);            // 32-column MFMA tiles per wave
-    static constexpr int NBUF = WAVES == 4 ? 2 : 3;      // LDS ring depth
+    static constexpr int NBUF = NBUF_ > 0 ? NBUF_ : (WAVES == 4 ? 2 : 3);  // LDS ring depth
     static constexpr int OFF_A = 0;
     static constexpr int OFF_B = BM * ROWB;
     static constexpr int OFF_ALO = BM * 64, OFF_BLO = OFF_B + BN * 64;  // split: lo planes
@@ -669,9 +669,28 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
     }
 }
 
-template <int WK, int EPI, int BM, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 3 : 256 / BM) void k_gemm(GemmParams p) {
-    using C = Cfg<WK, BM, WAVES>;
+// Wait until at most `ahead` (≤ MAXA) later stages of LOADS loads each are in
+// flight, then for the other waves.
+template <int LOADS, int MAXA>
+__device__ __forceinline__ void wait_stages(int ahead) {
+    if constexpr (MAXA > 0) {
+        if (ahead >= MAXA) {
+            wait_and_barrier<LOADS * MAXA>();
+            return;
+        }
+        wait_stages<LOADS, MAXA - 1>(ahead);
+    } else {
+        wait_and_barrier<0>();
+    }
+}
+
+// RING: LDS ring depth (0: by work-group size).  DEEP_RING stages fill a CU's
+// LDS: one work-group per CU with five stages of loads in flight, for grids
+// that leave no second work-group to a CU anyway.
+constexpr int DEEP_RING = 6;
+template <int WK, int EPI, int BM, int WAVES, int RING = 0>
+__global__ __launch_bounds__(64 * WAVES, RING ? 1 : (WAVES == 4 ? 3 : 256 / BM)) void k_gemm(GemmParams p) {
+    using C = Cfg<WK, BM, WAVES, RING>;
     constexpr int MT = C::MT, NT = C::NT, NBUF = C::NBUF;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS + EPI_TAB<EPI, BM>];
     int *const tab = (int *)(lds + C::LDS);
@@ -998,14 +1017,16 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 3 : 256 / BM) void k_gemm(
     // stage s is consumed ----
     const int kper = (p.nstages + p.ksplit - 1) / p.ksplit;
     const int s0 = kpart * kper, s1 = min(p.nstages, s0 + kper);
-    if constexpr (NBUF == 3) {
-        issue(s0, 0);
-        if (s0 + 1 < s1) issue(s0 + 1, 1);
+    if constexpr (NBUF >= 3) {
+#pragma unroll
+        for (int i = 0; i < NBUF - 1; i++)
+            if (s0 + i < s1) issue(s0 + i, i);
+        int buf = 0;
         for (int s = s0; s < s1; s++) {
-            if (s + 1 < s1) wait_and_barrier<C::NLOAD>();
-            else wait_and_barrier<0>();
-            if (s + 2 < s1) issue(s + 2, (s + 2 - s0) % NBUF);
-            compute((s - s0) % NBUF);
+            wait_stages<C::NLOAD, NBUF - 2>(s1 - 1 - s);  // stage s landed; every wave is done with stage s−1
+            if (s + NBUF - 1 < s1) issue(s + NBUF - 1, buf == 0 ? NBUF - 1 : buf - 1);
+            compute(buf);
+            buf = buf + 1 == NBUF ? 0 : buf + 1;
         }
     } else {
         issue(s0, 0);
@@ -1272,10 +1293,10 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(const float *__restrict__ p
     *o = v;
 }
 
-template <int WK, int EPI, int BM, int WAVES>
+template <int WK, int EPI, int BM, int WAVES, int RING = 0>
 hipError_t launch_one(const GemmParams &p, hipStream_t st) {
     const int grid = ((p.ntiles * p.ksplit + 7) / 8) * 8;
-    hipLaunchKernelGGL((k_gemm<WK, EPI, BM, WAVES>), dim3(grid), dim3(64 * WAVES), 0, st, p);
+    hipLaunchKernelGGL((k_gemm<WK, EPI, BM, WAVES, RING>), dim3(grid), dim3(64 * WAVES), 0, st, p);
     return hipGetLastError();
 }
 
@@ -1303,13 +1324,14 @@ hipError_t dispatch_epi(Epi epi, const GemmParams &p, hipStream_t st) {
 // ViT frame (518 per band) and on short K (Hiera's first stages) the 64-row
 // tiles' three work-groups per CU measured as fast or faster.
 constexpr int64_t F16_WIDE_MIN_TILES = 1200;
+constexpr int64_t F16_WIDE_LONE_TILES = 480;
 constexpr int64_t F16_WIDE_MIN_K = 512;
 
 template <int WK>
 hipError_t dispatch_waves(Epi epi, GemmParams &p, hipStream_t st) {
     if constexpr (WK == WK_F16) {
         const int64_t t128 = (int64_t)(p.M + 127) / 128 * p.tiles_n;
-        if (p.ksplit == 1 && t128 >= F16_WIDE_MIN_TILES && p.a_kbytes >= 2 * F16_WIDE_MIN_K &&
+        if (p.ksplit == 1 && t128 >= (p.e.lone ? F16_WIDE_LONE_TILES : F16_WIDE_MIN_TILES) && p.a_kbytes >= 2 * F16_WIDE_MIN_K &&
             (epi == EPI_F32 || epi == EPI_GELU || epi == EPI_QKV || epi == EPI_HQKV || epi == EPI_DECONV)) {
             p.tiles_m = (p.M + 127) / 128;
             p.ntiles = p.tiles_m * p.tiles_n;
@@ -1325,6 +1347,13 @@ hipError_t dispatch_waves(Epi epi, GemmParams &p, hipStream_t st) {
     constexpr int BM = 64;
     p.tiles_m = (p.M + BM - 1) / BM;
     p.ntiles = p.tiles_m * p.tiles_n;
+    // fp16 products that give each CU at most one work-group
+    if constexpr (WK == WK_F16 || WK == WK_F16X3) {
+        if (p.e.lone && p.ntiles * p.ksplit <= 256) {
+            if (epi == EPI_F32) return launch_one<WK, EPI_F32, BM, 4, DEEP_RING>(p, st);
+            if (epi == EPI_RESID) return launch_one<WK, EPI_RESID, BM, 4, DEEP_RING>(p, st);
+        }
+    }
     // 4-wave work-groups (three per CU, 4-12% faster on the SAM 3 shapes)
     // except for Q4_1, whose extra minimum term needs more registers than
     // three work-groups per CU leave
@@ -1333,15 +1362,34 @@ hipError_t dispatch_waves(Epi epi, GemmParams &p, hipStream_t st) {
 }
 
 // K ranges for a product that leaves CUs idle: fewer 64 × 128 tiles than CUs
-// and at least 8 stages of K; about 512 work-groups, each range at least four
-// stages.
+// and at least 8 stages of K, each range at least four stages.  At most about
+// 512 work-groups, as quantized and fp32 products overlap their matrix and
+// vector instructions across the waves of a SIMD; one per CU for fp16 (the deep
+// ring) and Q4_1 (whose ring leaves room for no second).  Of those the count
+// that saves most: a stage less takes 0.95 µs off a quantized product, 0.45 off
+// an fp16 and 1.4 off an fp32 one at these grids, while the ranges cost a
+// launch (2 µs) and 64 KB of partial sums written and read per tile and range.
+// Measured on one range and split (µs a call): 65 × 1024 × 4736 Q8_0 56 → 28
+// (16 tiles), 1601 × 1024 × 4736 62 → 55 (208); with 8 stages 65 × 1024 × 1024
+// 27 → 25 (16 tiles) but 1300 × 1024 × 1024 29 → 34 (168), which stays whole.
 int splitk_of(const Weight &w, int64_t M) {
     const int esize = (w.kind == WK_F16) ? 2 : (w.kind == WK_F32 ? 4 : 1);
     const int64_t ns = w.kind == WK_F16X3 ? w.Kp / 32 : w.Kp * esize / 128, tiles = (M + 63) / 64 * (w.Np / BN);
     if (tiles >= 256 || ns < 8 || w.N % 4 != 0) return 1;
-    int64_t ks = std::min<int64_t>((512 + tiles - 1) / tiles, ns / 4);
-    const int64_t per = (ns + ks - 1) / ks;
-    return (int)((ns + per - 1) / per);
+    const bool fp16 = w.kind == WK_F16 || w.kind == WK_F16X3;
+    const int64_t most = std::min<int64_t>(fp16 || w.kind == WK_Q4_1 ? 256 / tiles : (512 + tiles - 1) / tiles, ns / 4);
+    const double stage_us = fp16 ? 0.45 : (w.kind == WK_F32 ? 1.4 : 0.95);
+    int64_t best = 1;
+    double gain = 0.5;
+    for (int64_t k = 2; k <= most; k++) {
+        const int64_t per = (ns + k - 1) / k, ks = (ns + per - 1) / per;
+        const double g = stage_us * (double)(ns - per) - 2.0 - 0.0164 * (double)(ks * tiles);
+        if (g > gain) {
+            gain = g;
+            best = ks;
+        }
+    }
+    return (int)best;
 }
 
 }  // namespace

@@ -608,6 +608,7 @@ hipError_t hiera_block(const HieraModel *m, HieraState *s, int bi, const float *
         ed.bias = b.dp_b;
         ed.y = b.qs ? s->dp : y;
         ed.ldy = C;
+        ed.lone = true;
         if ((e = launch_gemm(b.dp, a_in, T, EPI_F32, ed, st)) != hipSuccess) return e;
         if (b.qs && (e = launch_pool_act(s->dp, H, W, C, 2, f32_act(y, C), st)) != hipSuccess) return e;
     } else if (b.qs) {
@@ -688,6 +689,7 @@ hipError_t hiera_block(const HieraModel *m, HieraState *s, int bi, const float *
     ep.bias = b.proj_b;
     ep.y = y;
     ep.ldy = C;
+    ep.lone = true;
     ep.ws = s->gws;
     ep.ws_cap = s->gws_cap;
     if ((e = launch_gemm(b.proj, a_proj, Tt, EPI_RESID, ep, st)) != hipSuccess) return e;
@@ -703,6 +705,7 @@ hipError_t hiera_block(const HieraModel *m, HieraState *s, int bi, const float *
     e2.bias = b.fc2_b;
     e2.y = y;
     e2.ldy = C;
+    e2.lone = true;
     e2.ws = s->gws;
     e2.ws_cap = s->gws_cap;
     return launch_gemm(b.fc2, e1.out, Tt, EPI_RESID, e2, st);

@@ -169,6 +169,9 @@ struct EpiArgs {
     const float *bias = nullptr;
     float *y = nullptr;          // EPI_F32 / EPI_RESID / EPI_POS
     int64_t ldy = 0;
+    // the product runs alone on the device: with few tiles it may fill the CUs'
+    // LDS (EPI_F32 / EPI_RESID, fp16 weights)
+    bool lone = false;
     // EPI_F32 / EPI_RESID: workspace for a split over K (gemm_splitk_floats
     // floats); null: never split
     float *ws = nullptr;

@@ -345,6 +345,7 @@ int memattn_run(const MemAttnModel *m, MemAttnState **sp, const float *curr, con
         er.bias = ly.sa_out_b;
         er.y = s->x;
         er.ldy = D;
+        er.lone = true;
         er.ws = s->part_o;
         er.ws_cap = s->part_o_floats;
         MA_TRY(launch_gemm(ly.sa_out, ao, N, EPI_RESID, er, st));

@@ -77,9 +77,20 @@ extern "C" int s3e_mul_mat_noalloc(s3e_ctx *ctx, const s3e_weight *w, const floa
     a.kind = ak;
     a.ld = W.K;
     a.mp = round_up(M, ROW_PAD);
+    ea.lone = true;
+    // a product split over K leaves its partial sums in the scratch array
+    // too, behind the converted rows, where there is room for them
+    const int64_t parts = gemm_splitk_floats(W, M);
+    auto split_at = [&](int64_t used) {
+        if (parts > 0 && used + parts * 4 <= (int64_t)S3E_NOALLOC_SCRATCH_BYTES) {
+            ea.ws = (float *)((uint8_t *)ctx->scratch + used);
+            ea.ws_cap = parts;
+        }
+    };
     hipError_t e = hipSetDevice(ctx->device);
     if (ak == A_F32) {  // f32 weights take the rows as they are
         a.x = (void *)X;
+        split_at(0);
         if (e == hipSuccess) e = launch_gemm(W, a, M, EPI_F32, ea, ctx->stream);
     } else {
         // [values M × K][d: (Kp/128) groups × mp rows × 4 fp16][s: same, Q8_1]
@@ -94,6 +105,7 @@ extern "C" int s3e_mul_mat_noalloc(s3e_ctx *ctx, const s3e_weight *w, const floa
         }
         uint8_t *base = (uint8_t *)ctx->scratch;
         a.x = base;
+        split_at(need);
         if (q8) {
             a.d = (uint16_t *)(base + vbytes);
             if (ak == A_Q8_1) a.s = (uint16_t *)(base + vbytes + pbytes);

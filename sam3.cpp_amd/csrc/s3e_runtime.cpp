@@ -474,18 +474,16 @@ int sm_kgroups(const Weight &W) {
     return std::max(1, std::min({SM_WG_GOAL / cgs, nst / (SM_KS * SM_MIN_STAGES), SM_KG_MAX}));
 }
 
-// Grow the context's split workspace to hold `parts` partial sums.
-hipError_t sk_workspace(s3e_ctx *ctx, int64_t parts) {
-    if (parts <= ctx->sk_part_cap) return hipSuccess;
-    hipError_t e = hipStreamSynchronize(ctx->stream);  // earlier launches may still read it
-    if (e != hipSuccess) return e;
-    if (ctx->sk_part) (void)hipFree(ctx->sk_part);
-    ctx->sk_part = nullptr;
-    ctx->sk_part_cap = 0;
-    e = hipMalloc(&ctx->sk_part, (size_t)parts * sizeof(float));
-    if (e != hipSuccess) return e;
-    ctx->sk_part_cap = parts;
-    return hipSuccess;
+// The context's split workspace, made once at its largest (a split product has
+// fewer than 768 tile × range pairs, a small-M one a tenth of that) and never
+// moved: captured small-M products hold its address.
+constexpr int64_t SK_PARTS = 768LL * 64 * GEMM_BN;
+hipError_t sk_workspace(s3e_ctx *ctx) {
+    if (ctx->sk_part) return hipSuccess;
+    const hipError_t e = hipMalloc(&ctx->sk_part, (size_t)SK_PARTS * sizeof(float));
+    if (e != hipSuccess) ctx->sk_part = nullptr;
+    else ctx->sk_part_cap = SK_PARTS;
+    return e;
 }
 
 }  // namespace
@@ -518,10 +516,30 @@ hipError_t s3e::CallWs::get(size_t bytes, void **out) {
 
 namespace {
 
+// A product on the tiled kernels.  Where few tiles leave CUs idle, K goes in
+// ranges whose partial sums lie in the context's workspace (1601 × 1024 × 4736
+// Q8_0, 208 tiles: 45.6 µs on one range, 34.4 + 5.1 on three).  While the
+// stream is being captured the product runs unsplit: a graph may be replayed
+// on another stream, beside calls that use the workspace.
+hipError_t run_tiles(s3e_ctx *ctx, const Weight &W, const Act &a, int64_t M, EpiArgs ea) {
+    ea.lone = true;
+    if (gemm_splitk_floats(W, M) > 0) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        hipError_t e = hipStreamIsCapturing(ctx->stream, &cap);
+        if (e != hipSuccess) return e;
+        if (cap == hipStreamCaptureStatusNone) {
+            if ((e = sk_workspace(ctx)) != hipSuccess) return e;
+            ea.ws = ctx->sk_part;
+            ea.ws_cap = ctx->sk_part_cap;
+        }
+    }
+    return launch_gemm(W, a, M, EPI_F32, ea, ctx->stream);
+}
+
 hipError_t run_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const Act &a, int64_t M, const EpiArgs &ea) {
     const Weight &W = w->w;
     hipStream_t st = ctx->stream;
-    if (!sm_eligible(W, M)) return launch_gemm(W, a, M, EPI_F32, ea, st);
+    if (!sm_eligible(W, M)) return run_tiles(ctx, W, a, M, ea);
     const uint8_t *wsm = nullptr;
     hipError_t e = sm_weights(w, st, &wsm);
     if (e != hipSuccess) return e;
@@ -549,7 +567,7 @@ hipError_t sm_prepare(s3e_ctx *ctx, const s3e_weight *w) {
     hipError_t e = sm_weights(w, ctx->stream, &wsm);
     if (e != hipSuccess) return e;
     const int kg = sm_kgroups(W);
-    return kg > 1 ? sk_workspace(ctx, (int64_t)kg * 64 * W.N) : hipSuccess;
+    return kg > 1 ? sk_workspace(ctx) : hipSuccess;
 }
 
 }  // namespace
@@ -606,12 +624,13 @@ extern "C" int s3e_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const float *X, in
     ea.bias = bias;
     ea.y = Y;
     ea.ldy = W.N;
+    CallWs ws(ctx);
     if (ak == A_F32) {
         Act a;
         a.kind = A_F32;
         a.x = (void *)X;
         a.ld = W.K;
-        HIP_TRY(launch_gemm(W, a, M, EPI_F32, ea, ctx->stream));
+        HIP_TRY(run_tiles(ctx, W, a, M, ea));
         return S3E_OK;
     }
     // [values of X in the product's format][d][s (Q8_1)].  Rows past M of the
@@ -624,7 +643,6 @@ extern "C" int s3e_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const float *X, in
     const bool f16 = a.kind == A_F16;
     const size_t vb = (size_t)(a.mp * W.K) * (f16 ? 4 : 3) / 2;  // fp6 pairs take 1.5 bytes, Q8 codes 1
     const size_t sb = f16 ? 0 : (size_t)(a.mp * (round_up(W.K, 128) / QK)) * 2;
-    CallWs ws(ctx);
     void *base = nullptr;
     hipError_t e = ws.get(vb + 2 * sb, &base);
     if (e == hipSuccess) {
@@ -660,7 +678,8 @@ extern "C" int s3e_mul_mat_q_f6(s3e_ctx *ctx, const s3e_weight *w, const void *x
     ea.bias = bias;
     ea.y = Y;
     ea.ldy = W.N;
-    HIP_TRY(launch_gemm(W, a, M, EPI_F32, ea, ctx->stream));
+    std::lock_guard<std::mutex> lock(ctx->call_mu);  // the split workspace: one product's launches at a time
+    HIP_TRY(run_tiles(ctx, W, a, M, ea));
     return S3E_OK;
 } S3E_CATCH("s3e_mul_mat_q_f6")
 
@@ -685,6 +704,7 @@ extern "C" int s3e_mul_mat_q(s3e_ctx *ctx, const s3e_weight *w, const void *xq, 
     ea.bias = bias;
     ea.y = Y;
     ea.ldy = W.N;
+    std::lock_guard<std::mutex> lock(ctx->call_mu);  // the split workspace: one product's launches at a time
     HIP_TRY(run_mul_mat(ctx, w, a, M, ea));
     return S3E_OK;
 } S3E_CATCH("s3e_mul_mat_q")

@@ -1,0 +1,59 @@
+"""s3e_mul_mat's ways through the device by row count and shape.
+
+Products of at most 64 rows convert X inside the kernel: bit for bit the
+product of rows converted beforehand.  Above, few tiles split K into ranges,
+and fp16 products then stage up to six stages at once: against the product in
+64 bits, where sums of K fp32 products in any order stay within 1e-6 relative
+L2 (2^-24 per sum, averaged over K ≤ 4736).
+"""
+import numpy as np
+import pytest
+
+import oracle_lib as orc
+import s3e
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [orc.Q4_0, orc.Q4_1, orc.Q8_0, orc.F16]
+VDT = {orc.Q4_0: s3e.TYPE_Q8_0, orc.Q8_0: s3e.TYPE_Q8_0, orc.Q4_1: s3e.TYPE_Q8_1, orc.F16: s3e.TYPE_F16}
+
+
+def _inputs(ctx, t, M, N, K, seed):
+    rng = np.random.default_rng(seed)
+    W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    X[:, : 32] *= 0 if M % 2 else 1  # a block of zeros: scale 0
+    bias = rng.standard_normal(N).astype(np.float32)
+    wb = orc.to_weight_bytes(t, W)
+    return wb, X, bias, ctx.weight(t, K, N, wb)
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("M,N,K", [(1, 33, 32), (7, 1024, 1024), (32, 96, 160), (33, 130, 4736), (64, 4736, 1024)])
+def test_rows_converted_in_the_product(ctx, t, M, N, K):
+    _, X, bias, w = _inputs(ctx, t, M, N, K, M + N)
+    Xd, Bd, Y0, Y = ctx.to_device(X), ctx.to_device(bias), ctx.buffer(M * N * 4), ctx.buffer(M * N * 4)
+    planes = (K + 127) // 128 * 4 * ((M + 127) // 128 * 128) * 2
+    q, d, s = ctx.buffer(M * K * 2), ctx.buffer(planes), ctx.buffer(planes)
+    print(t, M, N, K, flush=True)
+    ctx.quantize_rows(VDT[t], Xd, M, K, q, d, s)
+    ctx.mul_mat_q(w, q, d, s, M, Y0, Bd)
+    ctx.mul_mat(w, Xd, M, Y, Bd)
+    ctx.sync()
+    assert np.array_equal(Y.download(np.float32, (M, N)), Y0.download(np.float32, (M, N)))
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("M,N,K", [(65, 128, 512), (65, 96, 1024), (129, 1024, 4736), (1601, 1024, 4736),
+                                   (200, 130, 2080), (2048, 1024, 448), (1984, 1024, 64), (2049, 1024, 1056)])
+def test_split_products(ctx, t, M, N, K):
+    wb, X, bias, w = _inputs(ctx, t, M, N, K, M + K)
+    Y = ctx.buffer(M * N * 4)
+    print(t, M, N, K, flush=True)
+    ctx.mul_mat(w, ctx.to_device(X), M, Y, ctx.to_device(bias))
+    ctx.sync()
+    pick = np.unique(np.r_[0:3, M // 2 : M // 2 + 3, M - 3 : M])  # rows are independent: the oracle takes a few
+    ref = orc.mul_mat(t, wb, N, K, X[pick]).astype(np.float64) + bias
+    got = Y.download(np.float32, (M, N))
+    assert np.isfinite(got).all()
+    assert orc.rel_l2(got[pick], ref) <= 1e-6
