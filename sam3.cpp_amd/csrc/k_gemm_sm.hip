@@ -53,16 +53,32 @@ struct SmCfg {
     static constexpr int WL = WK == WK_F16 ? 8 : 4;                  // 16-byte weight loads per stage per lane
 };
 
-// Operands of one stage (4 blocks) for MT row tiles.
-template <int WK, int MT>
+// Operands of one stage (4 blocks) for MT row tiles; with XF the rows as f32.
+template <int WK, int MT, bool XF>
 struct SmStage {
     uint4 w[SmCfg<WK>::WL];
     uint2 wd, wm;
-    uint4 a[MT][SmCfg<WK>::WL];
+    uint4 a[XF ? 1 : MT][SmCfg<WK>::WL];
     uint2 ad[MT], as[MT];
+    float4 x[XF ? MT : 1][16];
 };
 
-template <int WK, int MT, int KS>
+// The larger of v over the two lanes (l, l ^ 32) that share a row.
+__device__ __forceinline__ float half_max(float v) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto sw = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return fmaxf(__builtin_bit_cast(float, (uint32_t)sw[0]), __builtin_bit_cast(float, (uint32_t)sw[1]));
+}
+__device__ __forceinline__ int half_sum(int v) {
+    const auto sw = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+    return (int)sw[0] + (int)sw[1];
+}
+
+// XF: X comes as f32 rows and every wave converts the K range it multiplies,
+// in registers, to the bit as the separate conversion pass does.  The strips
+// repeat the conversion (a third of a stage's work), but one launch and the
+// round trip through memory go: 7 × 1024 × 1024 Q4_0 21.7 → 19.2 µs a call.
+template <int WK, int MT, int KS, bool XF = false>
 __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
     using C = SmCfg<WK>;
     constexpr int SPW = SM_WAVES / KS;  // strips per work-group
@@ -88,7 +104,8 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
 #pragma unroll
     for (int i = 0; i < MT; i++) rows[i] = min(r0 + 32 * i + lr, M - 1);
 
-    auto load = [&](int s, SmStage<WK, MT> &f) {
+    using Stage = SmStage<WK, MT, XF>;
+    auto load = [&](int s, Stage &f) {
         const int b0 = 4 * s;
 #pragma unroll
         for (int j = 0; j < C::WL; j++) {
@@ -101,6 +118,21 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
         if constexpr (C::quant) {
             f.wd = *(const uint2 *)(G.wd + ((int64_t)s * G.np + n) * 4);
             if constexpr (C::q41) f.wm = *(const uint2 *)(G.wm + ((int64_t)s * G.np + n) * 4);
+        }
+        if constexpr (XF) {
+            // lane half lh holds 16 elements of each of the 4 blocks (quantized:
+            // 16·lh ..; F16: the 8-element slabs 16·(j & 1) + 8·lh); blocks past
+            // K re-read the row's end, against zero weights
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                const float *xr = p.x32 + (int64_t)rows[i] * G.ldx;
+#pragma unroll
+                for (int j = 0; j < 16; j++) {
+                    const int k = (b0 + j / 4) * 32 + (C::quant ? lh * 16 + 4 * (j & 3) : 16 * ((j >> 1) & 1) + 8 * lh + 4 * (j & 1));
+                    f.x[i][j] = *(const float4 *)(xr + min(k, G.K - 4));
+                }
+            }
+            return;
         }
 #pragma unroll
         for (int i = 0; i < MT; i++) {
@@ -130,7 +162,57 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[i][r] = 0.f;
 
-    auto compute = [&](const SmStage<WK, MT> &f) {
+    // the stage's rows in the product's format (ggml's from_float): the codes'
+    // operands, block scales and (Q4_1) sums
+    auto convert = [&](const Stage &f, uint4 (&fa)[MT][C::WL], uint2 (&fd)[MT], uint2 (&fs)[MT]) {
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            if constexpr (!XF) {
+#pragma unroll
+                for (int j = 0; j < C::WL; j++) fa[i][j] = f.a[i][j];
+                fd[i] = f.ad[i];
+                fs[i] = f.as[i];
+            } else if constexpr (C::quant) {
+                uint32_t dw[2] = {0u, 0u}, sw[2] = {0u, 0u};
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float *v = (const float *)&f.x[i][4 * j];
+                    float amax = 0.f;
+#pragma unroll
+                    for (int k = 0; k < 16; k++) amax = fmaxf(amax, fabsf(v[k]));
+                    amax = half_max(amax);
+                    const float d = amax / 127.f;
+                    const float id = (amax != 0.f) ? 127.f / amax : 0.f;
+                    uint32_t w[4] = {0u, 0u, 0u, 0u};
+                    int sum = 0;
+#pragma unroll
+                    for (int k = 0; k < 16; k++) {
+                        const int q = (int)__builtin_rintf(v[k] * id);
+                        sum += q;
+                        w[k / 4] |= ((uint32_t)(q & 0xff)) << (8 * (k & 3));
+                    }
+                    fa[i][j] = make_uint4(w[0], w[1], w[2], w[3]);
+                    dw[j >> 1] |= (uint32_t)half_bits(d) << (16 * (j & 1));
+                    if constexpr (C::q41) sw[j >> 1] |= (uint32_t)half_bits(d * (float)half_sum(sum)) << (16 * (j & 1));
+                }
+                fd[i] = make_uint2(dw[0], dw[1]);
+                fs[i] = make_uint2(sw[0], sw[1]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float *v = (const float *)&f.x[i][2 * j];
+                    uint32_t w[4];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) w[k] = (uint32_t)half_bits(v[2 * k]) | ((uint32_t)half_bits(v[2 * k + 1]) << 16);
+                    fa[i][j] = make_uint4(w[0], w[1], w[2], w[3]);
+                }
+            }
+        }
+    };
+    auto compute = [&](const Stage &f) {
+        uint4 fa[MT][C::WL];
+        uint2 fd[MT], fs[MT];
+        convert(f, fa, fd, fs);
         if constexpr (C::quant) {
             const v16i zi = {};
             const v16f zf = {};
@@ -154,9 +236,9 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
                 const v4u hb = {hw, 0u, 0u, 0u};
 #pragma unroll
                 for (int i = 0; i < MT; i++) {
-                    const v4i a = __builtin_bit_cast(v4i, f.a[i][j]);
+                    const v4i a = __builtin_bit_cast(v4i, fa[i][j]);
                     v16i S = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, zi, 0, 0, 0);
-                    const uint32_t adw[2] = {f.ad[i].x, f.ad[i].y};
+                    const uint32_t adw[2] = {fd[i].x, fd[i].y};
                     const uint32_t ha_ = (adw[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
                     const v4u ha = {ha_, 0u, 0u, 0u};
                     const v16f Cs = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, ha),
@@ -169,7 +251,7 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
                 const v4u hb = {f.wm.x, f.wm.y, 0u, 0u};
 #pragma unroll
                 for (int i = 0; i < MT; i++) {
-                    const v4u ha = {f.as[i].x, f.as[i].y, 0u, 0u};
+                    const v4u ha = {fs[i].x, fs[i].y, 0u, 0u};
                     acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, ha),
                                                                     __builtin_bit_cast(v8h, hb), acc[i], 0, 0, 0);
                 }
@@ -180,7 +262,7 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
                 const v8h b = __builtin_bit_cast(v8h, f.w[j]);
 #pragma unroll
                 for (int i = 0; i < MT; i++)
-                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, f.a[i][j]), b, acc[i], 0,
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, fa[i][j]), b, acc[i], 0,
                                                                     0, 0);
             }
         }
@@ -188,7 +270,7 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
 
     // stage s + 1 is in flight while stage s is consumed
     if (s0 < s1) {
-        SmStage<WK, MT> cur, nxt;
+        Stage cur, nxt;
         load(s0, cur);
         for (int s = s0; s < s1; s++) {
             const bool more = s + 1 < s1;
@@ -597,11 +679,13 @@ hipError_t launch_gemm_sm(WKind kind, const SmArgs &a, int wgs, int ks, hipStrea
     if (a.kg < 1 || a.kg > SM_KG_MAX || (a.kg > 1 && (a.many || !a.part || wgs % a.kg != 0)))
         return hipErrorInvalidValue;
     if (a.rt != 1 && (a.rt != 2 || a.M <= 32 || a.many || wgs % (2 * a.kg) != 0)) return hipErrorInvalidValue;
+    if (a.x32 && (a.many || (a.M > 32 && a.rt != 2) || a.one.K % 32 != 0 || a.one.ldx < a.one.K)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)wgs), block(64 * SM_WAVES);
     const bool two = a.M > 32 && a.rt == 1;
 #define S3E_SM(WK)                                                                                       \
     do {                                                                                                 \
-        if (two) hipLaunchKernelGGL((k_gemm_sm<WK, 2, 4>), grid, block, 0, st, a);                       \
+        if (a.x32) hipLaunchKernelGGL((k_gemm_sm<WK, 1, 4, true>), grid, block, 0, st, a);               \
+        else if (two) hipLaunchKernelGGL((k_gemm_sm<WK, 2, 4>), grid, block, 0, st, a);                  \
         else hipLaunchKernelGGL((k_gemm_sm<WK, 1, 4>), grid, block, 0, st, a);                           \
     } while (0)
     switch (kind) {

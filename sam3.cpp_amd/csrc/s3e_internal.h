@@ -304,6 +304,9 @@ struct SmArgs {
     float *part = nullptr;
     // k_gemm_sm with M > 32: 2 gives each 32-row tile work-groups of its own
     int rt = 1;
+    // k_gemm_sm, one product: X as f32 rows of one.ldx, converted in the kernel
+    // (one.x, xd and xs are then unused)
+    const float *x32 = nullptr;
 };
 
 // ---- kernel launchers (k_*.hip) ----

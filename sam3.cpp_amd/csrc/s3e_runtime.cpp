@@ -516,6 +516,16 @@ hipError_t s3e::CallWs::get(size_t bytes, void **out) {
 
 namespace {
 
+// Whether a small-M product converts its rows inside the kernel.  Every
+// 32-column strip repeats the conversion of its K range, so few rows (little to
+// load and convert) or a small weight (few strips, short ranges) favour it: at
+// Q4_0, µs a call in two passes and in one, 7 × 1024 × 1024 21.2 → 19.3, 7 × 4736
+// × 1024 20.1 → 19.2, 64 × 1024 × 1024 21.7 → 20.5, but 64 × 4736 × 1024 22.5 →
+// 26.0 and 64 × 1024 × 4736 24.4 → 26.7.  fp16 rows cost less to convert.
+bool sm_converts(const Weight &W, int64_t M) {
+    return sm_eligible(W, M) && (M <= (W.kind == WK_F16 ? 32 : 16) || W.N * W.K <= (int64_t)1 << 21);
+}
+
 // A product on the tiled kernels.  Where few tiles leave CUs idle, K goes in
 // ranges whose partial sums lie in the context's workspace (1601 × 1024 × 4736
 // Q8_0, 208 tiles: 45.6 µs on one range, 34.4 + 5.1 on three).  While the
@@ -536,7 +546,9 @@ hipError_t run_tiles(s3e_ctx *ctx, const Weight &W, const Act &a, int64_t M, Epi
     return launch_gemm(W, a, M, EPI_F32, ea, ctx->stream);
 }
 
-hipError_t run_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const Act &a, int64_t M, const EpiArgs &ea) {
+// x32: the rows of a product of at most 64 rows in f32 (a.x is then unused)
+hipError_t run_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const Act &a, int64_t M, const EpiArgs &ea,
+                       const float *x32 = nullptr) {
     const Weight &W = w->w;
     hipStream_t st = ctx->stream;
     if (!sm_eligible(W, M)) return run_tiles(ctx, W, a, M, ea);
@@ -546,6 +558,7 @@ hipError_t run_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const Act &a, int64_t 
     SmArgs sa;
     sa.one = sm_desc(W, wsm, a, ea.bias, ea.y, 0);
     sa.M = (int)M;
+    sa.x32 = x32;
     const int cgs = sm_wgs(W.N, SM_KS);
     sa.kg = sm_kgroups(W);
     sa.rt = (SM_ROW_TILES && M > 32) ? 2 : 1;
@@ -633,25 +646,30 @@ extern "C" int s3e_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const float *X, in
         HIP_TRY(run_tiles(ctx, W, a, M, ea));
         return S3E_OK;
     }
-    // [values of X in the product's format][d][s (Q8_1)].  Rows past M of the
-    // values and scale planes are never written: they only reach output rows
-    // past M, which no kernel stores.
+    hipError_t e;
     Act a;
-    a.kind = sm_eligible(W, M) ? ak : act_kind_gemm(W);
     a.ld = W.K;
-    a.mp = round_up(M, ROW_PAD);
-    const bool f16 = a.kind == A_F16;
-    const size_t vb = (size_t)(a.mp * W.K) * (f16 ? 4 : 3) / 2;  // fp6 pairs take 1.5 bytes, Q8 codes 1
-    const size_t sb = f16 ? 0 : (size_t)(a.mp * (round_up(W.K, 128) / QK)) * 2;
-    void *base = nullptr;
-    hipError_t e = ws.get(vb + 2 * sb, &base);
-    if (e == hipSuccess) {
-        a.x = base;
-        a.d = (uint16_t *)((uint8_t *)base + vb);
-        a.s = (uint16_t *)((uint8_t *)base + vb + sb);
-        e = launch_rows_quant(a.kind, X, M, W.K, a, ctx->stream);
+    if (sm_converts(W, M)) {
+        e = run_mul_mat(ctx, w, a, M, ea, X);
+    } else {
+        // [values of X in the product's format][d][s (Q8_1)].  Rows past M of
+        // the values and scale planes are never written: they only reach
+        // output rows past M, which no kernel stores.
+        a.kind = sm_eligible(W, M) ? ak : act_kind_gemm(W);
+        a.mp = round_up(M, ROW_PAD);
+        const bool f16 = a.kind == A_F16;
+        const size_t vb = (size_t)(a.mp * W.K) * (f16 ? 4 : 3) / 2;  // fp6 pairs take 1.5 bytes, Q8 codes 1
+        const size_t sb = f16 ? 0 : (size_t)(a.mp * (round_up(W.K, 128) / QK)) * 2;
+        void *base = nullptr;
+        e = ws.get(vb + 2 * sb, &base);
+        if (e == hipSuccess) {
+            a.x = base;
+            a.d = (uint16_t *)((uint8_t *)base + vb);
+            a.s = (uint16_t *)((uint8_t *)base + vb + sb);
+            e = launch_rows_quant(a.kind, X, M, W.K, a, ctx->stream);
+        }
+        if (e == hipSuccess) e = run_mul_mat(ctx, w, a, M, ea);
     }
-    if (e == hipSuccess) e = run_mul_mat(ctx, w, a, M, ea);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) { set_error("s3e_mul_mat: %s", hipGetErrorString(e)); return S3E_ERR_HIP; }
     return S3E_OK;
