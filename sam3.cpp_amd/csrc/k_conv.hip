@@ -304,11 +304,7 @@ hipError_t dispatch(Epi epi, bool conv3, ConvParams &p, hipStream_t st) {
             if (p.M > 128 * 512) return launch_one<SPLIT, 1, EPI_F32, 256>(p, st);
         return launch_one<SPLIT, 1, EPI_F32>(p, st);
     }
-    switch (epi) {
-        case EPI_F32: return launch_one<SPLIT, 0, EPI_F32>(p, st);
-        case EPI_ACT: return launch_one<SPLIT, 0, EPI_ACT>(p, st);
-        default: return hipErrorInvalidValue;
-    }
+    return epi == EPI_ACT ? launch_one<SPLIT, 0, EPI_ACT>(p, st) : hipErrorInvalidValue;
 }
 
 }  // namespace

@@ -8,43 +8,65 @@
 namespace s3e {
 namespace {
 
-// im2col of the patch embedding (Conv2d 3→E, k×k, stride, pad): CHW f32
-// [3][S][S] → rows [OH·OW][ldk] in F32 or F16 (ggml's im2col in the kernel
-// type), K ordered [c][ky][kx] as the kernel rows are; taps outside the image
-// and columns K..ldk are zero.
-__global__ void k_im2col_conv(const float *__restrict__ chw, int S, int k, int stride, int pad, int OW, int64_t T,
-                              int64_t ldk, int kind, void *out, _Float16 *lo) {
-    // 32-bit index arithmetic (the launcher keeps T·ldk below 2^31)
-    const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (uint32_t)(T * ldk)) return;
-    const uint32_t t = idx / (uint32_t)ldk;
-    const int kk = (int)(idx - t * (uint32_t)ldk);
-    float val = 0.f;
-    if (kk < 3 * k * k) {
-        const int c = kk / (k * k), r = kk % (k * k), ky = r / k, kx = r % k;
-        const int oy = (int)(t / (uint32_t)OW), ox = (int)(t - (uint32_t)oy * OW);
-        const int iy = oy * stride + ky - pad, ix = ox * stride + kx - pad;
-        if (iy >= 0 && iy < S && ix >= 0 && ix < S) val = chw[(int64_t)c * S * S + (int64_t)iy * S + ix];
-    }
-    if (kind == A_F16 || kind == A_F16X2) {
-        const _Float16 h = to_half(val);
-        ((_Float16 *)out)[idx] = h;
-        if (kind == A_F16X2) lo[idx] = (_Float16)(val - (float)h);  // fp16 of the exact difference
-    } else {
-        ((float *)out)[idx] = val;
+// 8 values as fp16 (h) and as the fp16 of what that rounding left (l), packed
+__device__ __forceinline__ void split8(const float (&v)[8], uint32_t (&h)[4], uint32_t (&l)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const _Float16 a = to_half(v[2 * j]), b = to_half(v[2 * j + 1]);
+        h[j] = (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+        const _Float16 c = (_Float16)(v[2 * j] - (float)a), d = (_Float16)(v[2 * j + 1] - (float)b);
+        l[j] = (uint32_t)__builtin_bit_cast(uint16_t, c) | ((uint32_t)__builtin_bit_cast(uint16_t, d) << 16);
     }
 }
 
-// Attention operands of one Hiera block from the QKV GEMM output (f32
-// [H·W][3C], bias already added).  Windows of wh × ww tokens, row-major over
-// nwx per row, cover the zero-padded grid; a padded position takes the QKV
-// bias, as ggml_pad's zero rows do after the projection.  Q is max-pooled
-// 2×2 inside each window under Q stride (sam2_maxpool_2d on the window's
-// grid).  Heads are zero-padded from HD to HDp channels.  Q, K: [b·NH + h]
-// [pos][HDp]; Vᵀ: [b·NH + h][HDp][ldv] with keys in vt_slot order and zeros
-// for keys Nkv .. ldv − 1.  With lo planes the values are split hi + lo.
+// im2col of the patch embedding (Conv2d 3→E, k×k, stride, pad): CHW f32
+// [3][S][S] → rows [OH·OW][ldk] in F32 or F16 (ggml's im2col in the kernel
+// type), K ordered [c][ky][kx] as the kernel rows are; taps outside the image
+// and columns K..ldk are zero.  A thread makes 8 columns of one row (one
+// 16-byte store per fp16 plane) and steps c, ky, kx from the first, so the
+// divisions are paid once per 8 values; lanes run along the row.  1024² fp16: 36.6 → 18.5 µs.
+__global__ __launch_bounds__(256) void k_im2col_conv(const float *__restrict__ chw, int S, int k, int stride, int pad,
+                                                     int OW, uint32_t n8, uint32_t ld8, int kind, void *out,
+                                                     _Float16 *lo) {
+    // 32-bit index arithmetic (the launcher keeps T·ldk below 2^31)
+    const uint32_t idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= n8) return;
+    const uint32_t t = idx / ld8;
+    const int k0 = (int)(idx - t * ld8) * 8;
+    const int oy = (int)(t / (uint32_t)OW), ox = (int)(t - (uint32_t)oy * OW);
+    const int y0 = oy * stride - pad, x0 = ox * stride - pad;
+    int c = k0 / (k * k), r = k0 - c * k * k, ky = r / k, kx = r - ky * k;
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int iy = y0 + ky, ix = x0 + kx;
+        v[j] = c < 3 && iy >= 0 && iy < S && ix >= 0 && ix < S ? chw[((int64_t)c * S + iy) * S + ix] : 0.f;
+        if (++kx == k) {
+            kx = 0;
+            if (++ky == k) { ky = 0; c++; }
+        }
+    }
+    if (kind == A_F16 || kind == A_F16X2) {
+        uint32_t h[4], l[4];
+        split8(v, h, l);
+        ((uint4 *)out)[idx] = make_uint4(h[0], h[1], h[2], h[3]);
+        if (kind == A_F16X2) ((uint4 *)lo)[idx] = make_uint4(l[0], l[1], l[2], l[3]);
+    } else {
+        ((float4 *)out)[2 * (int64_t)idx] = make_float4(v[0], v[1], v[2], v[3]);
+        ((float4 *)out)[2 * (int64_t)idx + 1] = make_float4(v[4], v[5], v[6], v[7]);
+    }
+}
+
+// Attention operands of one Hiera block that the QKV GEMM does not write.
+// Windows of wh × ww tokens, row-major over nwx per row, cover the
+// zero-padded grid; a padded position takes the QKV bias, as ggml_pad's zero
+// rows do after the projection.  Q is max-pooled 2×2 inside each window under
+// Q stride (sam2_maxpool_2d on the window's grid).  Heads are zero-padded from
+// HD to HDp channels.  Q, K: [b·NH + h][pos][HDp]; Vᵀ: [b·NH + h][HDp][ldv]
+// with keys in vt_slot order and zeros for keys Nkv .. ldv − 1.  With lo
+// planes the values are split hi + lo.
 struct Prep {
-    const float *qkv, *bias;
+    const float *qkv, *bias;  // Q rows (f32, bias added); the QKV bias
     int64_t ld;  // row stride of qkv in floats
     int H, W, C, NH, HD, HDp;
     int wh, ww, nwx, qs;
@@ -52,46 +74,39 @@ struct Prep {
     _Float16 *q, *k, *vt, *q_lo, *k_lo, *vt_lo;
 };
 
-__device__ __forceinline__ float qkv_at(const Prep &p, int b, int py, int px, int col) {
-    const int wy = b / p.nwx, wx = b % p.nwx;
-    const int y = wy * p.wh + py, x = wx * p.ww + px;
-    if (y < p.H && x < p.W) return p.qkv[((int64_t)y * p.W + x) * p.ld + col];
-    return p.bias[col];
-}
-
-__device__ __forceinline__ void put(_Float16 *hi, _Float16 *lo, int64_t i, float v) {
-    const _Float16 h = to_half(v);
-    hi[i] = h;
-    if (lo) lo[i] = (_Float16)(v - (float)h);
-}
-
-// mode 0: Q (one thread per (b, h, query, d)); 1: K; 2: Vᵀ (keys up to ldv)
-__global__ void k_hiera_prep(Prep p, int mode, int64_t total) {
+// Max-pooled Q of a Q-stride block from its f32 Q rows: one thread per (b, h,
+// query, 8 channels), so the index arithmetic and the window lookup are paid
+// once per 8 values and rows go by 16 and 32 bytes (HD % 8 = 0).  256² tokens of
+// 192 in 8 × 8 windows: 22.6 µs a value per thread, 11 so.
+__global__ __launch_bounds__(256) void k_hiera_qpool(Prep p, uint32_t n8) {
     // 32-bit index arithmetic (the launcher keeps totals below 2^31)
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint32_t)total) return;
-    const uint32_t r = i / (uint32_t)p.HDp;
-    const int d = (int)(i - r * (uint32_t)p.HDp);
-    const uint32_t npos = mode == 0 ? p.Nq : (mode == 1 ? p.Nkv : p.ldv);
-    const uint32_t bh32 = r / npos;
-    const int pos = (int)(r - bh32 * npos);
-    const int64_t bh = bh32;
-    const int b = (int)(bh32 / (uint32_t)p.NH), h = (int)(bh32 - (uint32_t)b * p.NH);
-    float v = 0.f;
-    if (d < p.HD && pos < (mode == 0 ? p.Nq : p.Nkv)) {
-        const int col = (p.ld == 3LL * p.C ? mode * p.C : 0) + h * p.HD + d;
-        if (mode == 0 && p.qs) {
-            const int qw = p.ww / 2;
-            const int qy = pos / qw, qx = pos % qw;
-            v = fmaxf(fmaxf(qkv_at(p, b, 2 * qy, 2 * qx, col), qkv_at(p, b, 2 * qy, 2 * qx + 1, col)),
-                      fmaxf(qkv_at(p, b, 2 * qy + 1, 2 * qx, col), qkv_at(p, b, 2 * qy + 1, 2 * qx + 1, col)));
-        } else {
-            v = qkv_at(p, b, pos / p.ww, pos % p.ww, col);
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const uint32_t nch = (uint32_t)p.HDp / 8;
+    const uint32_t r = i / nch;
+    const int d0 = (int)(i - r * nch) * 8;
+    const uint32_t bh = r / (uint32_t)p.Nq;
+    const int pos = (int)(r - bh * p.Nq);
+    const int b = (int)(bh / (uint32_t)p.NH), h = (int)(bh - (uint32_t)b * p.NH);
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (d0 < p.HD) {
+        const int col = h * p.HD + d0, qw = p.ww / 2;
+        const int wy = b / p.nwx, wx = b - wy * p.nwx, qy = pos / qw, qx = pos - qy * qw;
+        const int y = wy * p.wh + 2 * qy, x = wx * p.ww + 2 * qx;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int yy = y + (k >> 1), xx = x + (k & 1);
+            const float *src = yy < p.H && xx < p.W ? p.qkv + ((int64_t)yy * p.W + xx) * p.ld + col : p.bias + col;
+            const float4 a = *(const float4 *)src, c = *(const float4 *)(src + 4);
+            const float u[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = k == 0 ? u[j] : fmaxf(v[j], u[j]);
         }
     }
-    if (mode == 0) put(p.q, p.q_lo, (bh * p.Nq + pos) * p.HDp + d, v);
-    else if (mode == 1) put(p.k, p.k_lo, (bh * p.Nkv + pos) * p.HDp + d, v);
-    else put(p.vt, p.vt_lo, (bh * p.HDp + d) * p.ldv + vt_slot(pos), v);
+    uint32_t hw[4], lw[4];
+    split8(v, hw, lw);
+    ((uint4 *)p.q)[i] = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+    if (p.q_lo) ((uint4 *)p.q_lo)[i] = make_uint4(lw[0], lw[1], lw[2], lw[3]);
 }
 
 // Window positions outside the grid (ggml pads the normed input with zeros, so
@@ -124,12 +139,36 @@ __global__ void k_hiera_pad(Prep p, int with_q, uint32_t n_pad, uint32_t n_tail)
         const int64_t bh = (int64_t)b * p.NH + h;
         const int64_t vrow = bh * p.HDp;
         const int64_t slot = vt_slot(pos);
-        for (int d = d0; d < d0 + 8; d++) {
-            const bool real = d < p.HD;
-            const float bk = real ? p.bias[p.C + h * p.HD + d] : 0.f;
-            put(p.k, p.k_lo, (bh * p.Nkv + pos) * p.HDp + d, bk);
-            if (real) put(p.vt, p.vt_lo, (vrow + d) * p.ldv + slot, p.bias[2 * p.C + h * p.HD + d]);
-            if (with_q) put(p.q, p.q_lo, (bh * p.Nkv + pos) * p.HDp + d, real ? p.bias[h * p.HD + d] : 0.f);
+        // (HD is a multiple of 8: the 8 channels are all real or all padding)
+        const bool real = d0 < p.HD;
+        const int col = h * p.HD + d0;
+        uint32_t hw[4], lw[4];
+        auto bias8 = [&](int sel) {
+            float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (real) {
+                const float4 a = *(const float4 *)(p.bias + sel * p.C + col), c = *(const float4 *)(p.bias + sel * p.C + col + 4);
+                v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+                v[4] = c.x; v[5] = c.y; v[6] = c.z; v[7] = c.w;
+            }
+            split8(v, hw, lw);
+        };
+        const int64_t o = (bh * p.Nkv + pos) * p.HDp + d0;
+        bias8(1);
+        *(uint4 *)(p.k + o) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+        if (p.k_lo) *(uint4 *)(p.k_lo + o) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+        if (with_q) {
+            bias8(0);
+            *(uint4 *)(p.q + o) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+            if (p.q_lo) *(uint4 *)(p.q_lo + o) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+        }
+        if (real) {
+            bias8(2);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int64_t ov = (vrow + d0 + j) * p.ldv + slot;
+                p.vt[ov] = __builtin_bit_cast(_Float16, (uint16_t)(hw[j / 2] >> (16 * (j & 1))));
+                if (p.vt_lo) p.vt_lo[ov] = __builtin_bit_cast(_Float16, (uint16_t)(lw[j / 2] >> (16 * (j & 1))));
+            }
         }
         return;
     }
@@ -172,9 +211,10 @@ hipError_t launch_im2col_conv(const float *chw, int S, int k, int stride, int pa
     if ((kind != A_F16 && kind != A_F32 && kind != A_F16X2) || (kind == A_F16X2 && !lo) || ldk < 3LL * k * k)
         return hipErrorInvalidValue;
     const int64_t T = (int64_t)O * O, total = T * ldk;
-    if (total >= INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_im2col_conv, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, chw, S, k, stride,
-                       pad, O, T, ldk, (int)kind, out, (_Float16 *)lo);
+    if (total >= INT32_MAX || ldk % 8 != 0 || (uintptr_t)out % 16 != 0 || (uintptr_t)lo % 16 != 0) return hipErrorInvalidValue;
+    const uint32_t n8 = (uint32_t)(total / 8);
+    hipLaunchKernelGGL(k_im2col_conv, dim3((n8 + 255) / 256), dim3(256), 0, st, chw, S, k, stride, pad, O, n8,
+                       (uint32_t)(ldk / 8), (int)kind, out, (_Float16 *)lo);
     return hipGetLastError();
 }
 
@@ -184,7 +224,7 @@ Prep make_prep(const HieraPrepArgs &a) {
     Prep p;
     p.qkv = a.qkv;
     p.bias = a.bias;
-    p.ld = a.qkv_ld > 0 ? a.qkv_ld : 3LL * a.C;
+    p.ld = a.qkv_ld;
     p.H = a.H; p.W = a.W; p.C = a.C; p.NH = a.NH; p.HD = a.HD; p.HDp = a.HDp;
     p.qs = a.q_stride;
     if (a.window > 0) {
@@ -206,25 +246,21 @@ Prep make_prep(const HieraPrepArgs &a) {
 
 }  // namespace
 
-// With qkv_ld = C (Q rows only), the Q pass alone; with the full QKV rows,
-// all three operands.
-hipError_t launch_hiera_prep(const HieraPrepArgs &a, hipStream_t st) {
+hipError_t launch_hiera_qpool(const HieraPrepArgs &a, hipStream_t st) {
     const Prep p = make_prep(a);
-    if (p.HD > p.HDp || p.HDp % 8 != 0 || (p.ld != 3LL * p.C && p.ld != p.C)) return hipErrorInvalidValue;
-    const int64_t bh = (int64_t)p.NW * p.NH;
-    const int64_t tq = bh * p.Nq * p.HDp, tk = bh * p.Nkv * p.HDp, tv = bh * p.ldv * p.HDp;
-    if (tv >= INT32_MAX || tk >= INT32_MAX || tq >= INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_hiera_prep, dim3((unsigned)((tq + 255) / 256)), dim3(256), 0, st, p, 0, tq);
-    if (p.ld == 3LL * p.C) {
-        hipLaunchKernelGGL(k_hiera_prep, dim3((unsigned)((tk + 255) / 256)), dim3(256), 0, st, p, 1, tk);
-        hipLaunchKernelGGL(k_hiera_prep, dim3((unsigned)((tv + 255) / 256)), dim3(256), 0, st, p, 2, tv);
-    }
+    if (!a.q_stride || p.HD <= 0 || p.HD > p.HDp || p.HD % 8 != 0 || p.HDp % 8 != 0 || p.ld < p.C || p.ld % 4 != 0 ||
+        p.C % 8 != 0 || p.wh % 2 != 0 || p.ww % 2 != 0 || !p.q || !p.qkv || !p.bias)
+        return hipErrorInvalidValue;
+    const int64_t n8 = (int64_t)p.NW * p.NH * p.Nq * (p.HDp / 8);
+    if (n8 >= INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_hiera_qpool, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, st, p, (uint32_t)n8);
     return hipGetLastError();
 }
 
 hipError_t launch_hiera_pad(const HieraPrepArgs &a, hipStream_t st) {
     const Prep p = make_prep(a);
-    if (p.HD > p.HDp || !p.k || !p.vt || !p.bias || (!a.q_stride && !p.q)) return hipErrorInvalidValue;
+    if (p.HD > p.HDp || p.HD % 8 != 0 || p.HDp % 8 != 0 || !p.k || !p.vt || !p.bias || (!a.q_stride && !p.q))
+        return hipErrorInvalidValue;
     const int64_t Wp = (int64_t)p.nwx * p.ww, Hp = (int64_t)(p.NW / p.nwx) * p.wh;
     if (Wp < p.W || Hp < p.H || (int64_t)(p.NW / p.nwx) * p.nwx != p.NW || p.ldv < p.Nkv) return hipErrorInvalidValue;
     const int64_t n_pad = (Hp * Wp - (int64_t)p.H * p.W) * p.NH * (p.HDp / 8);

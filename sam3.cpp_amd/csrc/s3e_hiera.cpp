@@ -16,7 +16,7 @@
 //   QKV GEMM (+ bias) whose epilogue writes Q, K, Vᵀ in window order as
 //             fp16 (hi, lo) planes, heads zero-padded to 64/128; a small
 //             pass fills window padding with the bias; under Q stride Q goes
-//             out as f32 rows and k_hiera_prep max-pools it inside windows
+//             out as f32 rows and k_hiera_qpool max-pools it inside windows
 //   attention (k_attn, head dim 64 or 128) → proj input, written at the
 //             un-partitioned, cropped token rows
 //   proj GEMM + bias + residual; LayerNorm; fc1 + bias + ggml_gelu (fp16
@@ -539,6 +539,8 @@ int hiera_state_create(const HieraModel *m, int img, hipStream_t st, HieraState 
             W = Wt;
         }
     }
+    for (int i = 0; i < 4; i++)
+        gws_cap = std::max(gws_cap, gemm_splitk_floats(m->fpn[3 - i], (int64_t)s->side[i] * s->side[i]));
     if (e == hipSuccess) e = s->a1.alloc(T0, emax, st);
     if (e == hipSuccess) e = s->a2.alloc(T0, 4 * emax, st);
     for (int i = 0; i < 4 && e == hipSuccess; i++)
@@ -647,7 +649,7 @@ hipError_t hiera_block(const HieraModel *m, HieraState *s, int bi, const float *
     eq.ldy = C;
     if ((e = launch_gemm(b.qkv, a_in, T, EPI_HQKV, eq, st)) != hipSuccess) return e;
     if ((e = launch_hiera_pad(pa, st)) != hipSuccess) return e;
-    if (b.qs && (e = launch_hiera_prep(pa, st)) != hipSuccess) return e;
+    if (b.qs && (e = launch_hiera_qpool(pa, st)) != hipSuccess) return e;
     // 4. attention → the proj input at the un-partitioned, cropped token rows
     const int nwx = b.ws > 0 ? (W + b.ws - 1) / b.ws : 1, nwy = b.ws > 0 ? (H + b.ws - 1) / b.ws : 1;
     AttnArgs aa;
@@ -746,7 +748,10 @@ hipError_t hiera_encode(const HieraModel *m, HieraState *s, const float *chw, hi
         el.bias = m->fpn_b[3 - i];
         el.y = s->lat[i];
         el.ldy = m->D;
-        if ((e = launch_conv(w, in, (int64_t)sd * sd, EPI_F32, el, nullptr, st)) != hipSuccess) return e;
+        el.lone = true;
+        el.ws = s->gws;
+        el.ws_cap = s->gws_cap;
+        if ((e = launch_gemm(w, in, (int64_t)sd * sd, EPI_F32, el, st)) != hipSuccess) return e;
     }
     int prev = -1;
     for (int i = 3; i >= 0; i--) {

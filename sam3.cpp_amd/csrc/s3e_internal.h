@@ -329,8 +329,8 @@ hipError_t launch_gemm_sm(WKind kind, const SmArgs &a, int wgs, int ks, hipStrea
 // LDS; wgs = total of sm_wgs(N, 1).
 hipError_t launch_gemm_smb(WKind kind, const SmArgs &a, int wgs, hipStream_t st);
 // Neck GEMMs (k_conv.hip; WK_F16 or WK_F16X3 weights with N padded to
-// CONV_BN): EPI_ACT / EPI_F32 on plain rows, or EPI_F32 as a 3×3 implicit
-// GEMM when g is given.
+// CONV_BN): EPI_ACT on plain rows, or EPI_F32 as a 3×3 implicit GEMM when g is
+// given.
 hipError_t launch_conv(const Weight &w, const Act &a, int64_t M, Epi epi, const EpiArgs &ea,
                        const ConvGeom *g, hipStream_t st);
 // NHWC f32 [h][w][c] → act (A_F16 or A_F16X2) of the same pixels (pool = 1)
@@ -393,20 +393,19 @@ hipError_t launch_add_pos(const float *x, const float *pos, float *y, int G, int
 // Patch-embedding im2col: CHW f32 [3][S][S], k×k / stride / pad → rows of ldk.
 hipError_t launch_im2col_conv(const float *chw, int S, int k, int stride, int pad, int64_t ldk, AKind kind,
                               void *out, hipStream_t st, void *lo = nullptr);
-// Attention operands of a Hiera block from its QKV GEMM output (window
-// partition with bias-valued padding, Q max-pool, head split, zero-padded
-// head dim, fp16 hi/lo).
+// The attention operands of a Hiera block that its QKV GEMM does not write.
 struct HieraPrepArgs {
-    const float *qkv = nullptr;   // [H·W][3C] f32, bias added
+    const float *qkv = nullptr;   // Q rows [H·W][qkv_ld] f32, bias added (Q stride)
     const float *bias = nullptr;  // [3C]: the value of padded window positions
     int H = 0, W = 0, C = 0, NH = 0, HD = 0, HDp = 0;
     int window = 0;               // 0: one window of the whole grid (global attention)
     int q_stride = 0;
-    int qkv_ld = 0;               // row stride of qkv in floats (0: 3C); Q columns start at 0
+    int qkv_ld = 0;               // row stride of qkv in floats
     _Float16 *q = nullptr, *k = nullptr, *vt = nullptr;
     _Float16 *q_lo = nullptr, *k_lo = nullptr, *vt_lo = nullptr;
 };
-hipError_t launch_hiera_prep(const HieraPrepArgs &a, hipStream_t st);
+// Q under Q stride, max-pooled 2×2 inside each window
+hipError_t launch_hiera_qpool(const HieraPrepArgs &a, hipStream_t st);
 // The attention operands that the EPI_HQKV epilogue does not write: window
 // positions outside the grid (the QKV bias; zeros past HD), Q only without Q
 // stride, and the Vᵀ key slots from the window size up to vt_ld (zeros).
