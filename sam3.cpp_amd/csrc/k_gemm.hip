@@ -263,7 +263,7 @@ __device__ __forceinline__ void activate(const EpiArgs &e, const float *bias, fl
 // Epilogue from the fp32 tile Ct [BM][CLD] in LDS (scaled, complete), run by
 // the NT_ threads of the work-group.  tab: EPI_TAB<EPI, BM> bytes of LDS.
 template <int EPI, int BM>
-constexpr int EPI_TAB = EPI == EPI_HQKV ? 4 * (2 * BM + BN) : 0;
+constexpr int EPI_TAB = EPI == EPI_HQKV || EPI == EPI_QKV ? 4 * (2 * BM + 2 * BN) : 0;
 template <int EPI, int BM, int NT_, bool TABLE = true>
 __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, int *tab, int m0, int n0, int t) {
     const EpiArgs &e = p.e;
@@ -271,6 +271,24 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
         const int sel = n0 / e.E + e.sel0;  // 0 = Q, 1 = K, 2 = V (a tile never straddles)
         const int Nw = e.window * e.window;
         const int nwx = e.grid / e.window;
+        // (window, position) of the tile's tokens and (head, channel) of its
+        // columns, worked out once per tile as for EPI_HQKV below (5184 × 3072 ×
+        // 1024 Q4_0 in the encoder, with the loads before the stores, 59.5 →
+        // 58.2 µs)
+        int2 *const tok = (int2 *)tab;
+        int *const colw = tab + 2 * BM;
+        float *const colb = (float *)(colw + BN);  // the bias (see EPI_RESID on loads behind stores)
+        for (int i = t; i < BM + BN; i += NT_) {
+            if (i < BM) {
+                const int gm = m0 + i, py = gm / e.grid, px = gm - py * e.grid, wy = py / e.window, wx = px / e.window;
+                tok[i] = make_int2(wy * nwx + wx, (py - wy * e.window) * e.window + px - wx * e.window);
+            } else {
+                const int r2 = n0 + i - BM - (sel - e.sel0) * e.E, h = r2 / e.HD;
+                colw[i - BM] = h << 12 | (r2 - h * e.HD);
+                colb[i - BM] = e.bias[n0 + i - BM];
+            }
+        }
+        __syncthreads();
         if (sel == 2) {
             // Vᵀ [b][h][d][slot]: a unit is one column d and 8 consecutive
             // tokens.  Window and image-row boundaries fall on multiples of 8
@@ -281,13 +299,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
                 const int col = u / (BM / 8), r0 = (u % (BM / 8)) * 8;
                 const int gm = m0 + r0;
                 if (gm >= p.M) continue;
-                const int gn = n0 + col;
-                const float bv = e.bias[gn];
-                const int r2 = gn - (2 - e.sel0) * e.E;
-                const int h = r2 / e.HD, d = r2 % e.HD;
-                const int py = gm / e.grid, px = gm % e.grid;
-                const int b = (py / e.window) * nwx + px / e.window;
-                const int pp = (py % e.window) * e.window + px % e.window;
+                const float bv = colb[col];
+                const int h = colw[col] >> 12, d = colw[col] & 0xfff, b = tok[r0].x, pp = tok[r0].y;
                 uint32_t w[4], wl[4];
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
@@ -308,8 +321,24 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
                 }
             }
         } else {
-            // Q, K [b][h][p][d] with RoPE: a unit is one token and 16 columns
-            for (int u = t; u < BM * (BN / 16); u += NT_) {
+            // Q, K [b][h][p][d] with RoPE: a unit is one token and 16 columns;
+            // the angles of all of a thread's units are loaded before the
+            // first store
+            constexpr int UP = BM * (BN / 16) / NT_;
+            float4 cs4[UP][4];
+            if (e.freqs) {
+#pragma unroll
+                for (int k = 0; k < UP; k++) {
+                    const int u = t + k * NT_, row = min(u / (BN / 16), p.M - 1 - m0), cc = u % (BN / 16);
+                    const float4 *f4 = (const float4 *)(e.freqs + ((int64_t)tok[row].y * (e.HD / 2) + (colw[cc * 16] & 0xfff) / 2) * 2);
+                    const bool on = e.rope_rows <= 0 || m0 + row < e.rope_rows;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) cs4[k][j] = on ? f4[j] : make_float4(1.f, 0.f, 1.f, 0.f);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < UP; k++) {
+                const int u = t + k * NT_;
                 const int row = u / (BN / 16), cc = u % (BN / 16);
                 const int gm = m0 + row;
                 if (gm >= p.M) continue;
@@ -318,24 +347,19 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
 #pragma unroll
                 for (int j = 0; j < 16; j += 4) {
                     const float4 x = *(const float4 *)(Ct + row * CLD + cc * 16 + j);
-                    const float4 bb = *(const float4 *)(e.bias + gn0 + j);
+                    const float4 bb = *(const float4 *)(colb + cc * 16 + j);
                     v[j] = x.x + bb.x;
                     v[j + 1] = x.y + bb.y;
                     v[j + 2] = x.z + bb.z;
                     v[j + 3] = x.w + bb.w;
                 }
-                const int py = gm / e.grid, px = gm % e.grid;
-                const int b = (py / e.window) * nwx + px / e.window;
-                const int pp = (py % e.window) * e.window + px % e.window;
-                const int r2 = gn0 - (sel - e.sel0) * e.E;
-                const int h = r2 / e.HD, d0 = r2 % e.HD;
+                const int h = colw[cc * 16] >> 12, d0 = colw[cc * 16] & 0xfff, b = tok[row].x, pp = tok[row].y;
                 if (e.freqs && (e.rope_rows <= 0 || gm < e.rope_rows)) {
                     // sam3_apply_rope: out_re = re·cos − im·sin, out_im = re·sin + im·cos,
                     // each product rounded on its own (separate ggml ops).
-                    const float4 *f4 = (const float4 *)(e.freqs + ((int64_t)pp * (e.HD / 2) + d0 / 2) * 2);
 #pragma unroll
                     for (int j = 0; j < 16; j += 4) {
-                        const float4 cs = f4[j / 4];  // cos, sin of pairs j/2 and j/2 + 1
+                        const float4 cs = cs4[k][j / 4];  // cos, sin of pairs j/2 and j/2 + 1
                         const float c0 = cs.x, s0 = cs.y, c1 = cs.z, s1 = cs.w;
                         const float re0 = v[j], im0 = v[j + 1], re1 = v[j + 2], im1 = v[j + 3];
                         v[j] = __fsub_rn(__fmul_rn(re0, c0), __fmul_rn(im0, s0));
@@ -378,9 +402,11 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
         // Where a row and a column go, worked out once per tile: (window,
         // position in it) of the BM tokens and (Q / K / V / none, head,
         // channel) of the BN columns.  Done per stored piece, the divisions
-        // were most of the kernel: 65536 × 576 × 96 fp16 63 µs, now 55.
+        // were most of the kernel: 65536 × 576 × 96 fp16 63 µs, now 49 (the last 6
+        // by the bias in LDS: no load waits behind a store).
         int2 *const tok = (int2 *)tab;
         int *const colw = tab + 2 * BM;
+        float *const colb = (float *)(colw + BN);  // the bias (see EPI_RESID on loads behind stores)
         for (int i = t; i < BM + BN; i += NT_) {
             if (i < BM) {
                 const int gm = m0 + i;
@@ -395,6 +421,7 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
                 const int sel = gn < C ? 0 : gn < 2 * C ? 1 : gn < 3 * C ? 2 : 3;
                 const int r2 = gn - sel * C, h = r2 / HD;
                 colw[i - BM] = sel == 3 ? 3 << 28 : sel << 28 | h << 12 | (r2 - h * HD);
+                colb[i - BM] = sel == 3 ? 0.f : e.bias[gn];
             }
         }
         __syncthreads();
@@ -407,8 +434,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
             {
                 const float4 x0 = *(const float4 *)(Ct + row * CLD + cc * 8);
                 const float4 x1 = *(const float4 *)(Ct + row * CLD + cc * 8 + 4);
-                const float4 b0 = *(const float4 *)(e.bias + gn0);
-                const float4 b1 = *(const float4 *)(e.bias + gn0 + 4);
+                const float4 b0 = *(const float4 *)(colb + cc * 8);
+                const float4 b1 = *(const float4 *)(colb + cc * 8 + 4);
                 v[0] = x0.x + b0.x; v[1] = x0.y + b0.y; v[2] = x0.z + b0.z; v[3] = x0.w + b0.w;
                 v[4] = x1.x + b1.x; v[5] = x1.y + b1.y; v[6] = x1.z + b1.z; v[7] = x1.w + b1.w;
             }
@@ -449,7 +476,7 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
             const int rp = u % (BM / 2), col = u / (BM / 2);
             const int gm = m0 + 2 * rp, gn = n0 + col;
             if (gm >= p.M || gn < 2 * C || gn >= 3 * C) continue;
-            const float bv = e.bias[gn];
+            const float bv = colb[col];
             const float v0 = Ct[(2 * rp) * CLD + col] + bv, v1 = Ct[(2 * rp + 1) * CLD + col] + bv;
             const int cw = colw[col], h = cw >> 12 & 0xffff, d = cw & 0xfff;
             const int2 t0 = tok[2 * rp], t1 = tok[2 * rp + 1];
@@ -480,23 +507,37 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
             // 8 columns (one 16-byte store) per thread, 16 neighbouring threads
             // a row: whole lines, where 32 columns a thread stores every
             // line in pieces (4096 × 1536 × 384: 19.0 → 17.7 µs)
-            for (int u = t; u < BM * (BN / 8); u += NT_) {
-                const int row = u / (BN / 8), cc = u % (BN / 8) * 8;
-                const int gm = m0 + row, gn0 = n0 + cc;
-                if (gm >= p.M || gn0 >= p.N) continue;
-                float v[8], bias[8];
+            // The bias is the same for all of a thread's units, and every value
+            // is made before the first store (see EPI_RESID).
+            constexpr int UP = BM * (BN / 8) / NT_;
+            const int cc = t % (BN / 8) * 8, gn0 = n0 + cc;
+            if (gn0 >= p.N) return;
+            float bias[8];
+#pragma unroll
+            for (int j = 0; j < 8; j += 4) {
+                const float4 bb = *(const float4 *)(e.bias + gn0 + j);
+                bias[j] = bb.x; bias[j + 1] = bb.y; bias[j + 2] = bb.z; bias[j + 3] = bb.w;
+            }
+            uint4 w[UP];
+#pragma unroll
+            for (int k = 0; k < UP; k++) {
+                const int row = (t + k * NT_) / (BN / 8);
+                float v[8];
 #pragma unroll
                 for (int j = 0; j < 8; j += 4) {
-                    const float4 bb = *(const float4 *)(e.bias + gn0 + j);
-                    bias[j] = bb.x; bias[j + 1] = bb.y; bias[j + 2] = bb.z; bias[j + 3] = bb.w;
                     const float4 x = *(const float4 *)(Ct + row * CLD + cc + j);
                     v[j] = x.x; v[j + 1] = x.y; v[j + 2] = x.z; v[j + 3] = x.w;
                 }
                 activate<TABLE>(e, bias, v);
-                uint32_t w[4];
+                uint32_t h[4];
 #pragma unroll
-                for (int j = 0; j < 4; j++) w[j] = (uint32_t)f2h_bits(v[2 * j]) | ((uint32_t)f2h_bits(v[2 * j + 1]) << 16);
-                *(uint4 *)((_Float16 *)o.x + (int64_t)gm * o.ld + gn0) = make_uint4(w[0], w[1], w[2], w[3]);
+                for (int j = 0; j < 4; j++) h[j] = (uint32_t)f2h_bits(v[2 * j]) | ((uint32_t)f2h_bits(v[2 * j + 1]) << 16);
+                w[k] = make_uint4(h[0], h[1], h[2], h[3]);
+            }
+#pragma unroll
+            for (int k = 0; k < UP; k++) {
+                const int gm = m0 + (t + k * NT_) / (BN / 8);
+                if (gm < p.M) *(uint4 *)((_Float16 *)o.x + (int64_t)gm * o.ld + gn0) = w[k];
             }
             return;
         }
@@ -625,6 +666,44 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
                     *(float4 *)(e.y + (int64_t)gm * e.ldy + gn) =
                         make_float4(__fadd_rn(res[k].x, v[0]), __fadd_rn(res[k].y, v[1]),
                                     __fadd_rn(res[k].z, v[2]), __fadd_rn(res[k].w, v[3]));
+                }
+                return;
+            }
+        }
+        if constexpr (EPI == EPI_F32 || EPI == EPI_POS) {
+            if (vec) {
+                // likewise: loads behind stores made each row wait for the
+                // row before it to reach memory (65536 × 96 × 160 with
+                // positions 32.0 → 21.2 µs, 5184 × 3072 × 1024 fp16 69.5 → 67.8
+                // a call)
+                const float4 bb = e.bias ? *(const float4 *)(e.bias + gn) : make_float4(0.f, 0.f, 0.f, 0.f);
+                const float bj[4] = {bb.x, bb.y, bb.z, bb.w};
+                float4 pos[EPI == EPI_POS ? RPT : 1];
+                if constexpr (EPI == EPI_POS) {
+#pragma unroll
+                    for (int k = 0; k < RPT; k++) {
+                        const int gm = min(m0 + (t >> 5) + k * (NT_ / 32), p.M - 1);
+                        const int py = gm / e.grid, px = gm - py * e.grid;
+                        pos[k] = *(const float4 *)(e.pos + ((int64_t)(py % e.pos_grid) * e.pos_grid + px % e.pos_grid) * p.N + gn);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < RPT; k++) {
+                    const int row = (t >> 5) + k * (NT_ / 32), gm = m0 + row;
+                    if (gm >= p.M) continue;
+                    const float4 x = *(const float4 *)(Ct + row * CLD + 4 * f);
+                    float v[4] = {x.x, x.y, x.z, x.w};
+                    if (e.bias) {
+#pragma unroll
+                        for (int j = 0; j < 4; j++) v[j] = __fadd_rn(v[j], bj[j]);
+                    }
+                    if constexpr (EPI == EPI_POS) {
+                        v[0] = __fadd_rn(v[0], pos[k].x);
+                        v[1] = __fadd_rn(v[1], pos[k].y);
+                        v[2] = __fadd_rn(v[2], pos[k].z);
+                        v[3] = __fadd_rn(v[3], pos[k].w);
+                    }
+                    *(float4 *)(e.y + (int64_t)gm * e.ldy + gn) = make_float4(v[0], v[1], v[2], v[3]);
                 }
                 return;
             }
@@ -1090,7 +1169,7 @@ __global__ __launch_bounds__(256, 3) void k_gemm_f6(GemmParams p) {
     constexpr int OFF_A = 0, OFF_B = 12288, OFF_AD = 24576, OFF_BD = OFF_AD + BM * 8;
     constexpr int STAGE = OFF_BD + BN * 8;  // 26112
     constexpr int LDSZ = 2 * STAGE > BM * CLD * 4 ? 2 * STAGE : BM * CLD * 4;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[LDSZ];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[LDSZ + EPI_TAB<EPI, BM>];
 
     const int per = gridDim.x >> 3;
     const int logical0 = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -1256,7 +1335,7 @@ __global__ __launch_bounds__(256, 3) void k_gemm_f6(GemmParams p) {
             return;
         }
     }
-    epilogue<EPI, BM, NTH, false>(p, Ct, nullptr, m0, n0, t);  // (no table: its registers would spill here)
+    epilogue<EPI, BM, NTH, false>(p, Ct, (int *)(lds + LDSZ), m0, n0, t);  // (no table: its registers would spill here)
 }
 
 // y = Σ_k part[k] (+ bias) for EPI_F32, y += Σ_k part[k] (+ bias) for
@@ -1324,6 +1403,8 @@ hipError_t dispatch_epi(Epi epi, const GemmParams &p, hipStream_t st) {
 // ViT frame (518 per band) and on short K (Hiera's first stages) the 64-row
 // tiles' three work-groups per CU measured as fast or faster.
 constexpr int64_t F16_WIDE_MIN_TILES = 1200;
+// A lone product overlaps nothing else: 5184 × 3072 × 1024 (984 such tiles) 67.8
+// → 63.4 µs a call.  From 480 tiles on every CU has nearly two work-groups.
 constexpr int64_t F16_WIDE_LONE_TILES = 480;
 constexpr int64_t F16_WIDE_MIN_K = 512;
 
