@@ -538,6 +538,18 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         if constexpr (decltype(has_qk)::value) s_next = qk(j + 1);
         if constexpr (decltype(has_pv)::value) pv(j - 1, prev.h, prev.l);
         if constexpr (decltype(has_sm)::value) ps = softmax(s_cur, mnew, cur.h, cur.l);
+        if constexpr (SPLIT && !VN) {
+            // operand reads and softmax VALU spread between the 24 MFMAs: the
+            // ViT's windowed blocks 49.5 → 48.8 µs, the global ones 352 → 347.
+            // The other kernels measured equal or slower with such an order
+            // (head dim 256 by 13 %).
+#pragma unroll
+            for (int i = 0; i < 24; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // VALU
+            }
+        }
         if constexpr (decltype(has_sm)::value) {
             lsum = lsum * alpha + ps;
             mrun = mnew;
