@@ -11,6 +11,7 @@ import pytest
 
 import oracle_lib as orc
 import s3e
+from test_zz_no_alloc import _Graphs
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +58,34 @@ def test_split_products(ctx, t, M, N, K):
     got = Y.download(np.float32, (M, N))
     assert np.isfinite(got).all()
     assert orc.rel_l2(got[pick], ref) <= 1e-6
+
+
+@pytest.mark.parametrize("t", [orc.Q8_0, orc.F16])
+def test_captured_product_sums_in_one_range(ctx, t):
+    # a graph must not hold the context's workspace: its replays may run beside other calls
+    M, N, K = 300, 512, 1024
+    _, X, bias, w = _inputs(ctx, t, M, N, K, 5)
+    Xd, Bd = ctx.to_device(X), ctx.to_device(bias)
+    planes = (K + 127) // 128 * 4 * ((M + 127) // 128 * 128) * 2
+    q, d, s = ctx.buffer(M * K * 2), ctx.buffer(planes), ctx.buffer(planes)
+    ctx.quantize_rows(VDT[t], Xd, M, K, q, d, s)
+    ref, got = ctx.buffer(M * N * 4), ctx.buffer(M * N * 4)
+    ctx.mul_mat_q(w, q, d, s, M, ref, Bd)
+    ctx.sync()
+    want = ref.download(np.float32, (M, N))
+    gr = _Graphs()
+    g, ex = gr.capture(ctx.stream, lambda: ctx.mul_mat_q(w, q, d, s, M, got, Bd))
+    try:
+        first = None
+        for rep in range(3):
+            got.upload(np.full((M, N), np.nan, np.float32))
+            assert gr.h.hipGraphLaunch(ex, ctx.stream) == 0
+            ctx.sync()
+            out = got.download(np.float32, (M, N))
+            first = out if first is None else first
+            assert np.array_equal(out, first) and orc.rel_l2(out, want) <= 1e-6, rep
+            ctx.mul_mat_q(w, q, d, s, M, ref, Bd)  # eager work on the workspace between replays
+            ctx.sync()
+    finally:
+        gr.h.hipGraphExecDestroy(ex)
+        gr.h.hipGraphDestroy(g)
