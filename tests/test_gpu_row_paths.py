@@ -1,7 +1,7 @@
 """s3e_mul_mat's ways through the device by row count and shape.
 
-Products of at most 64 rows convert X inside the kernel: bit for bit the
-product of rows converted beforehand.  Above, few tiles split K into ranges,
+Products of few rows convert X inside the kernel where that is cheaper: bit
+for bit the product of rows converted beforehand, on either side of the rule.  Above, few tiles split K into ranges,
 and fp16 products then stage up to six stages at once: against the product in
 64 bits, where sums of K fp32 products in any order stay within 1e-6 relative
 L2 (2^-24 per sum, averaged over K ≤ 4736).
