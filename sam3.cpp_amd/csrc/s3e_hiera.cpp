@@ -522,8 +522,8 @@ int hiera_state_create(const HieraModel *m, int img, hipStream_t st, HieraState 
             if (b.qs) qkv_cap = std::max(qkv_cap, T * b.dout);  // Q rows before pooling
             dp_cap = std::max(dp_cap, T * b.dout);
             attn_cap = std::max(attn_cap, (int64_t)Ht * Wt * b.dout);
-            gws_cap = std::max({gws_cap, gemm_splitk_floats(b.proj, (int64_t)Ht * Wt),
-                                gemm_splitk_floats(b.fc2, (int64_t)Ht * Wt)});
+            gws_cap = std::max({gws_cap, gemm_splitk_floats(b.proj, (int64_t)Ht * Wt, true),
+                                gemm_splitk_floats(b.fc2, (int64_t)Ht * Wt, true)});
             int wh = b.ws > 0 ? b.ws : H, ww = b.ws > 0 ? b.ws : W;
             const int64_t NW = b.ws > 0 ? (int64_t)((H + b.ws - 1) / b.ws) * ((W + b.ws - 1) / b.ws) : 1;
             const int64_t nkv = (int64_t)wh * ww, nq = b.qs ? (int64_t)(wh / 2) * (ww / 2) : nkv;
@@ -539,8 +539,6 @@ int hiera_state_create(const HieraModel *m, int img, hipStream_t st, HieraState 
             W = Wt;
         }
     }
-    for (int i = 0; i < 4; i++)
-        gws_cap = std::max(gws_cap, gemm_splitk_floats(m->fpn[3 - i], (int64_t)s->side[i] * s->side[i]));
     if (e == hipSuccess) e = s->a1.alloc(T0, emax, st);
     if (e == hipSuccess) e = s->a2.alloc(T0, 4 * emax, st);
     for (int i = 0; i < 4 && e == hipSuccess; i++)
@@ -692,6 +690,7 @@ hipError_t hiera_block(const HieraModel *m, HieraState *s, int bi, const float *
     ep.y = y;
     ep.ldy = C;
     ep.lone = true;
+    ep.frame = true;
     ep.ws = s->gws;
     ep.ws_cap = s->gws_cap;
     if ((e = launch_gemm(b.proj, a_proj, Tt, EPI_RESID, ep, st)) != hipSuccess) return e;
@@ -708,6 +707,7 @@ hipError_t hiera_block(const HieraModel *m, HieraState *s, int bi, const float *
     e2.y = y;
     e2.ldy = C;
     e2.lone = true;
+    e2.frame = true;
     e2.ws = s->gws;
     e2.ws_cap = s->gws_cap;
     return launch_gemm(b.fc2, e1.out, Tt, EPI_RESID, e2, st);
@@ -749,8 +749,6 @@ hipError_t hiera_encode(const HieraModel *m, HieraState *s, const float *chw, hi
         el.y = s->lat[i];
         el.ldy = m->D;
         el.lone = true;
-        el.ws = s->gws;
-        el.ws_cap = s->gws_cap;
         if ((e = launch_gemm(w, in, (int64_t)sd * sd, EPI_F32, el, st)) != hipSuccess) return e;
     }
     int prev = -1;

@@ -172,6 +172,9 @@ struct EpiArgs {
     // the product runs alone on the device: with few tiles it may fill the CUs'
     // LDS (EPI_F32 / EPI_RESID, fp16 weights)
     bool lone = false;
+    // a product of an encode or a memory-attention pass: the K ranges of those
+    // (splitk_of)
+    bool frame = false;
     // EPI_F32 / EPI_RESID: workspace for a split over K (gemm_splitk_floats
     // floats); null: never split
     float *ws = nullptr;
@@ -312,7 +315,8 @@ struct SmArgs {
 // ---- kernel launchers (k_*.hip) ----
 // Floats of workspace a product of M rows against w would use when split over
 // K (0: it runs unsplit): products with fewer tiles than CUs and a long K.
-int64_t gemm_splitk_floats(const Weight &w, int64_t M);
+// frame: as EpiArgs.
+int64_t gemm_splitk_floats(const Weight &w, int64_t M, bool frame);
 // Products against uploaded weights (k_gemm.hip): every epilogue but EPI_ACT;
 // EPI_DECONV takes WK_F16 weights and A_F16 rows.
 hipError_t launch_gemm(const Weight &w, const Act &a, int64_t M, Epi epi, const EpiArgs &ea,

@@ -261,8 +261,8 @@ int memattn_run(const MemAttnModel *m, MemAttnState **sp, const float *curr, con
     // attention partials are merged before each of them on the same stream
     int64_t gws = 0;
     for (const MemAttnLayer &ly : m->layers)
-        gws = std::max({gws, gemm_splitk_floats(ly.sa_out, N), gemm_splitk_floats(ly.ca_out, N),
-                        gemm_splitk_floats(ly.fc2, N)});
+        gws = std::max({gws, gemm_splitk_floats(ly.sa_out, N, true), gemm_splitk_floats(ly.ca_out, N, true),
+                        gemm_splitk_floats(ly.fc2, N, true)});
     const int64_t need_o = std::max(part * D, gws);
     if (e == hipSuccess && (part > s->part_cap || need_o > s->part_o_floats)) {
         if (s->part_o) (void)hipFree(s->part_o);
@@ -346,6 +346,7 @@ int memattn_run(const MemAttnModel *m, MemAttnState **sp, const float *curr, con
         er.y = s->x;
         er.ldy = D;
         er.lone = true;
+        er.frame = true;
         er.ws = s->part_o;
         er.ws_cap = s->part_o_floats;
         MA_TRY(launch_gemm(ly.sa_out, ao, N, EPI_RESID, er, st));

@@ -80,7 +80,7 @@ extern "C" int s3e_mul_mat_noalloc(s3e_ctx *ctx, const s3e_weight *w, const floa
     ea.lone = true;
     // a product split over K leaves its partial sums in the scratch array
     // too, behind the converted rows, where there is room for them
-    const int64_t parts = gemm_splitk_floats(W, M);
+    const int64_t parts = gemm_splitk_floats(W, M, false);
     auto split_at = [&](int64_t used) {
         if (parts > 0 && used + parts * 4 <= (int64_t)S3E_NOALLOC_SCRATCH_BYTES) {
             ea.ws = (float *)((uint8_t *)ctx->scratch + used);

@@ -533,7 +533,7 @@ bool sm_converts(const Weight &W, int64_t M) {
 // on another stream, beside calls that use the workspace.
 hipError_t run_tiles(s3e_ctx *ctx, const Weight &W, const Act &a, int64_t M, EpiArgs ea) {
     ea.lone = true;
-    if (gemm_splitk_floats(W, M) > 0) {
+    if (gemm_splitk_floats(W, M, false) > 0) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         hipError_t e = hipStreamIsCapturing(ctx->stream, &cap);
         if (e != hipSuccess) return e;

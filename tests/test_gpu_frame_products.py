@@ -1,0 +1,93 @@
+"""The products inside a Hiera block and a memory-attention layer, alone: the
+attention's projection and one MLP weight are zero, so what comes out is the
+product under test.
+"""
+import contextlib
+import os
+
+import numpy as np
+import pytest
+
+import s3e
+from model_patch import patched
+
+pytestmark = pytest.mark.gpu
+
+# Sums in fp32 that tell the K ranges they were formed in: 2^24 in the first
+# 512, 1 + 1 (in different stages) in the second, -2^24 in the third.  Ranges
+# of 512 added in order give (2^24 + 2) - 2^24 = 2; where the ones meet 2^24
+# one at a time both are lost (ties to even) and the sum is 0.
+BIG, ONES, BACK = 0, (512, 576), 1024
+
+
+def _hidden(n, off):
+    """fc1 biases (fc1's weight is zero) whose activations are 16384 at BIG and BACK, 16 at ONES, else 0."""
+    b = np.full(n, off, np.float32)
+    b[[BIG, BACK]] = 16384
+    b[list(ONES)] = 16
+    return b
+
+
+def _weights(n_out, n_hidden):
+    w = np.zeros((n_out, n_hidden), np.float32)
+    w[:, BIG], w[:, BACK], w[:, list(ONES)] = 1024, -1024, 1 / 16
+    return w
+
+
+@contextlib.contextmanager
+def _state(ctx, path):
+    gm = s3e.Model(ctx, path)
+    st = s3e.State(ctx, gm)
+    try:
+        yield st
+    finally:  # also where an assertion holds on to the frame: before the context goes
+        st.free()
+        gm.free()
+
+
+@pytest.fixture(scope="module")
+def hiera_file(tmpdir_session):
+    path = os.path.join(str(tmpdir_session), "products.ggml")
+    s3e.synth_write_sam2(path, "hiera_t", img_size=1024, ftype="f16", seed=4, stages=(1, 1, 2, 2), global_idx=())
+    return path
+
+
+@pytest.mark.parametrize("block,side,dim", [(3, 64, 384), (5, 32, 768)])
+def test_hiera_fc2_sums_in_ranges_of_512(ctx, hiera_file, tmpdir_session, block, side, dim):
+    # 192 tiles in 3 ranges, 96 tiles in 6
+    path, p = os.path.join(str(tmpdir_session), f"fc2_{block}.ggml"), f"hiera.blocks.{block}."
+    patched(hiera_file, path, {
+        p + "attn.proj.weight": 0, p + "attn.proj.bias": 0, p + "mlp.fc1.weight": 0, p + "mlp.fc1.bias": _hidden(4 * dim, -100),
+        p + "mlp.fc2.weight": _weights(dim, 4 * dim), p + "mlp.fc2.bias": 0})
+    T = side * side
+    x, y = ctx.to_device(np.zeros((T, dim), np.float32)), ctx.buffer(T * dim * 4)
+    print("hiera block", block, flush=True)
+    with _state(ctx, path) as st:
+        st.hiera_block(block, x, side, side, y)
+        ctx.sync()
+        assert (y.download(np.float32, (T, dim)) == 2).all()
+
+
+def test_memory_attention_linear2_sums_in_ranges_of_512(ctx, tmpdir_session):
+    # 4096 rows: 128 tiles in 4 ranges.  The norm at the end shows even channels (2, or 0) against odd ones (1)
+    src, path = (os.path.join(str(tmpdir_session), n) for n in ("ma.ggml", "ma_ranges.ggml"))
+    p = "mem_attn.layers.0."
+    s3e.synth_write_sam2(src, "hiera_t", img_size=64, ftype="f16", seed=13, mem_attn_layers=1, embed_dim=32, stages=(1, 1, 1, 1),
+                         global_idx=(), window_spec=(4, 4, 2, 2), bkg=(2, 2))
+    w = _weights(256, 2048)
+    w[1::2] = 0
+    w[1::2, ONES[0]] = 1 / 16
+    patched(src, path, {
+        p + "sa.out_proj.weight": 0, p + "sa.out_proj.bias": 0, p + "ca.out_proj.weight": 0, p + "ca.out_proj.bias": 0,
+        p + "linear1.weight": 0, p + "linear1.bias": _hidden(2048, 0), p + "linear2.weight": w, p + "linear2.bias": 0,
+        "mem_attn.norm.weight": 1, "mem_attn.norm.bias": 0})
+    N, M = 4096, 64
+    zero = ctx.to_device(np.zeros((N, 256), np.float32))
+    rope = ctx.to_device(np.ones((N, 128, 2), np.float32))
+    out = ctx.buffer(N * 256 * 4)
+    print("memory attention", flush=True)
+    with _state(ctx, path) as st:
+        st.mem_attn(zero, zero, N, zero, zero, M, M, rope, None, out)
+        ctx.sync()
+        y = out.download(np.float32, (N, 256))
+        assert (y[:, ::2] > 0.9).all() and (y[:, 1::2] < -0.9).all()
