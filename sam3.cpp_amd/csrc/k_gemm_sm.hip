@@ -122,14 +122,17 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
         if constexpr (XF) {
             // lane half lh holds 16 elements of each of the 4 blocks (quantized:
             // 16·lh ..; F16: the 8-element slabs 16·(j & 1) + 8·lh); blocks past
-            // K re-read the row's end, against zero weights
+            // K re-read the row's end (F16 its last 8 elements, as above), against
+            // zero weights and, quantized, zero scales and sums (convert)
 #pragma unroll
             for (int i = 0; i < MT; i++) {
                 const float *xr = p.x32 + (int64_t)rows[i] * G.ldx;
 #pragma unroll
                 for (int j = 0; j < 16; j++) {
-                    const int k = (b0 + j / 4) * 32 + (C::quant ? lh * 16 + 4 * (j & 3) : 16 * ((j >> 1) & 1) + 8 * lh + 4 * (j & 1));
-                    f.x[i][j] = *(const float4 *)(xr + min(k, G.K - 4));
+                    const int kb = (b0 + j / 4) * 32;
+                    const int k = C::quant ? min(kb + lh * 16 + 4 * (j & 3), G.K - 4)
+                                           : min(kb + 16 * ((j >> 1) & 1) + 8 * lh, G.K - 8) + 4 * (j & 1);
+                    f.x[i][j] = *(const float4 *)(xr + k);
                 }
             }
             return;
@@ -162,9 +165,11 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[i][r] = 0.f;
 
-    // the stage's rows in the product's format (ggml's from_float): the codes'
-    // operands, block scales and (Q4_1) sums
-    auto convert = [&](const Stage &f, uint4 (&fa)[MT][C::WL], uint2 (&fd)[MT], uint2 (&fs)[MT]) {
+    // the rows of stage s in the product's format (ggml's from_float): the codes'
+    // operands, block scales and (Q4_1) sums.  Scales and sums of blocks past K
+    // are zero, as the conversion pass writes them: what those blocks re-read
+    // may scale or sum to infinity, which a zero weight would turn into NaN
+    auto convert = [&](int s, const Stage &f, uint4 (&fa)[MT][C::WL], uint2 (&fd)[MT], uint2 (&fs)[MT]) {
 #pragma unroll
         for (int i = 0; i < MT; i++) {
             if constexpr (!XF) {
@@ -176,6 +181,7 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
                 uint32_t dw[2] = {0u, 0u}, sw[2] = {0u, 0u};
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
+                    const bool in = (4 * s + j) * QK < G.K;
                     const float *v = (const float *)&f.x[i][4 * j];
                     float amax = 0.f;
 #pragma unroll
@@ -192,8 +198,11 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
                         w[k / 4] |= ((uint32_t)(q & 0xff)) << (8 * (k & 3));
                     }
                     fa[i][j] = make_uint4(w[0], w[1], w[2], w[3]);
-                    dw[j >> 1] |= (uint32_t)half_bits(d) << (16 * (j & 1));
-                    if constexpr (C::q41) sw[j >> 1] |= (uint32_t)half_bits(d * (float)half_sum(sum)) << (16 * (j & 1));
+                    if (in) dw[j >> 1] |= (uint32_t)half_bits(d) << (16 * (j & 1));
+                    if constexpr (C::q41) {
+                        const uint32_t hs = half_bits(d * (float)half_sum(sum));
+                        if (in) sw[j >> 1] |= hs << (16 * (j & 1));
+                    }
                 }
                 fd[i] = make_uint2(dw[0], dw[1]);
                 fs[i] = make_uint2(sw[0], sw[1]);
@@ -209,10 +218,10 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
             }
         }
     };
-    auto compute = [&](const Stage &f) {
+    auto compute = [&](int s, const Stage &f) {
         uint4 fa[MT][C::WL];
         uint2 fd[MT], fs[MT];
-        convert(f, fa, fd, fs);
+        convert(s, f, fa, fd, fs);
         if constexpr (C::quant) {
             const v16i zi = {};
             const v16f zf = {};
@@ -275,7 +284,7 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
         for (int s = s0; s < s1; s++) {
             const bool more = s + 1 < s1;
             if (more) load(s + 1, nxt);
-            compute(cur);
+            compute(s, cur);
             if (more) cur = nxt;
         }
     }

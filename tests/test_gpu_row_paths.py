@@ -45,6 +45,29 @@ def test_rows_converted_in_the_product(ctx, t, M, N, K):
 
 
 @pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("M,N,K", [(1, 33, 32), (7, 130, 224), (16, 96, 1056), (33, 64, 160), (64, 40, 96)])
+@pytest.mark.parametrize("at,value", [(4, 2100.0), (1, 3e4), (8, 7e4), (16, 1e7)])
+def test_large_values_at_the_end_of_a_row(ctx, t, M, N, K, at, value):
+    # the last stage reaches past K: what it reads there must weigh nothing,
+    # also where a scale or a sum of the row's last values would be infinite
+    wb, X, _, w = _inputs(ctx, t, M, N, K, M + K)
+    X[:, -at:] = 0
+    X[:, K - at : K - at + 4] = value
+    Xd, Y0, Y = ctx.to_device(X), ctx.buffer(M * N * 4), ctx.buffer(M * N * 4)
+    planes = (K + 127) // 128 * 4 * ((M + 127) // 128 * 128) * 2
+    q, d, s = ctx.buffer(M * K * 2), ctx.buffer(planes), ctx.buffer(planes)
+    print(t, M, N, K, at, value, flush=True)
+    ctx.quantize_rows(VDT[t], Xd, M, K, q, d, s)
+    ctx.mul_mat_q(w, q, d, s, M, Y0)
+    ctx.mul_mat(w, Xd, M, Y)
+    ctx.sync()
+    got, want = Y.download(np.float32, (M, N)), Y0.download(np.float32, (M, N))
+    assert np.array_equal(got, want, equal_nan=True)
+    if value == 2100.0:
+        assert np.isfinite(got).all() and orc.rel_l2(got, orc.mul_mat(t, wb, N, K, X)) <= 1e-6
+
+
+@pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("M,N,K", [(65, 128, 512), (65, 96, 1024), (129, 1024, 4736), (1601, 1024, 4736),
                                    (200, 130, 2080), (2048, 1024, 448), (1984, 1024, 64), (2049, 1024, 1056)])
 def test_split_products(ctx, t, M, N, K):
