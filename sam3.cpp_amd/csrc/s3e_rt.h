@@ -23,9 +23,11 @@ struct s3e_ctx {
     std::vector<uint8_t> sm_last;
     // this device's copy of the allocation-free entry points' scratch array
     void *scratch = nullptr;
-    // partial sums of products split over K across work-groups
+    // partial sums of products of at most 64 rows split over K across work-groups
+    // (captured products hold its address), and of larger ones
     float *sk_part = nullptr;
     int64_t sk_part_cap = 0;
+    float *tile_part = nullptr;
     // s3e_flash_attn_ext_f16's operand copies and key-split partials
     void *attn_ws = nullptr;
     size_t attn_ws_cap = 0;

@@ -315,6 +315,7 @@ extern "C" void s3e_ctx_destroy(s3e_ctx *ctx) {
     (void)hipStreamDestroy(ctx->stream);
     if (ctx->sm_dev) (void)hipFree(ctx->sm_dev);
     if (ctx->sk_part) (void)hipFree(ctx->sk_part);
+    if (ctx->tile_part) (void)hipFree(ctx->tile_part);
     if (ctx->attn_ws) (void)hipFree(ctx->attn_ws);
     if (ctx->call_ws) (void)hipFree(ctx->call_ws);
     if (ctx->probe_sink) (void)hipFree(ctx->probe_sink);
@@ -474,15 +475,24 @@ int sm_kgroups(const Weight &W) {
     return std::max(1, std::min({SM_WG_GOAL / cgs, nst / (SM_KS * SM_MIN_STAGES), SM_KG_MAX}));
 }
 
-// The context's split workspace, made once at its largest (a split product has
-// fewer than 768 tile × range pairs, a small-M one a tenth of that) and never
-// moved: captured small-M products hold its address.
-constexpr int64_t SK_PARTS = 768LL * 64 * GEMM_BN;
+// The context's workspaces for partial sums, each made once at its largest and
+// never moved.  Small-M products (at most SM_WG_GOAL work-groups of 32 columns)
+// have one of their own: where captured, they hold its address, and a graph may
+// be replayed on another stream beside eager products of any size.
+constexpr int64_t SK_PARTS = SM_WG_GOAL * 32LL * 64;
 hipError_t sk_workspace(s3e_ctx *ctx) {
     if (ctx->sk_part) return hipSuccess;
     const hipError_t e = hipMalloc(&ctx->sk_part, (size_t)SK_PARTS * sizeof(float));
     if (e != hipSuccess) ctx->sk_part = nullptr;
     else ctx->sk_part_cap = SK_PARTS;
+    return e;
+}
+// (a split product has fewer than 768 tile × range pairs)
+constexpr int64_t TILE_PARTS = 768LL * 64 * GEMM_BN;
+hipError_t tile_workspace(s3e_ctx *ctx) {
+    if (ctx->tile_part) return hipSuccess;
+    const hipError_t e = hipMalloc(&ctx->tile_part, (size_t)TILE_PARTS * sizeof(float));
+    if (e != hipSuccess) ctx->tile_part = nullptr;
     return e;
 }
 
@@ -530,7 +540,7 @@ bool sm_converts(const Weight &W, int64_t M) {
 // ranges whose partial sums lie in the context's workspace (1601 × 1024 × 4736
 // Q8_0, 208 tiles: 45.6 µs on one range, 34.4 + 5.1 on three).  While the
 // stream is being captured the product runs unsplit: a graph may be replayed
-// on another stream, beside calls that use the workspace.
+// on another stream, beside calls that use that workspace.
 hipError_t run_tiles(s3e_ctx *ctx, const Weight &W, const Act &a, int64_t M, EpiArgs ea) {
     ea.lone = true;
     if (gemm_splitk_floats(W, M, false) > 0) {
@@ -538,9 +548,9 @@ hipError_t run_tiles(s3e_ctx *ctx, const Weight &W, const Act &a, int64_t M, Epi
         hipError_t e = hipStreamIsCapturing(ctx->stream, &cap);
         if (e != hipSuccess) return e;
         if (cap == hipStreamCaptureStatusNone) {
-            if ((e = sk_workspace(ctx)) != hipSuccess) return e;
-            ea.ws = ctx->sk_part;
-            ea.ws_cap = ctx->sk_part_cap;
+            if ((e = tile_workspace(ctx)) != hipSuccess) return e;
+            ea.ws = ctx->tile_part;
+            ea.ws_cap = TILE_PARTS;
         }
     }
     return launch_gemm(W, a, M, EPI_F32, ea, ctx->stream);

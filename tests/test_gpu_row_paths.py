@@ -6,6 +6,8 @@ and fp16 products then stage up to six stages at once: against the product in
 64 bits, where sums of K fp32 products in any order stay within 1e-6 relative
 L2 (2^-24 per sum, averaged over K ≤ 4736).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -112,3 +114,40 @@ def test_captured_product_sums_in_one_range(ctx, t):
     finally:
         gr.h.hipGraphExecDestroy(ex)
         gr.h.hipGraphDestroy(g)
+
+
+@pytest.mark.parametrize("t", [orc.Q4_0, orc.F16])
+def test_captured_small_product_beside_large_ones(ctx, t):
+    # a captured product of up to 64 rows keeps its partial sums where no larger product writes
+    gr = _Graphs()
+    gr.h.hipStreamCreateWithFlags.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_uint]
+    gr.h.hipStreamSynchronize.argtypes = gr.h.hipStreamDestroy.argtypes = [ctypes.c_void_p]
+    other = ctypes.c_void_p()
+    assert gr.h.hipStreamCreateWithFlags(ctypes.byref(other), 1) == 0  # hipStreamNonBlocking
+    ops = []
+    for M, N, K in ((32, 256, 2048), (300, 512, 2048)):  # 4 K ranges; 4 or 8
+        _, X, bias, w = _inputs(ctx, t, M, N, K, M)
+        Xd, Bd, Y = ctx.to_device(X), ctx.to_device(bias), ctx.buffer(M * N * 4)
+        planes = (K + 127) // 128 * 4 * ((M + 127) // 128 * 128) * 2
+        q, d, s = ctx.buffer(M * K * 2), ctx.buffer(planes), ctx.buffer(planes)
+        ctx.quantize_rows(VDT[t], Xd, M, K, q, d, s)
+        ctx.mul_mat_q(w, q, d, s, M, Y, Bd)
+        ctx.sync()
+        ops.append((M, N, Y, Y.download(np.float32, (M, N)), (w, q, d, s, M, Y, Bd)))
+    (M0, N0, Y0, want0, small), (M1, N1, Y1, want1, large) = ops
+    g, ex = gr.capture(ctx.stream, lambda: ctx.mul_mat_q(*small))
+    try:
+        for rep in range(10):
+            Y0.upload(np.full((M0, N0), np.nan, np.float32))
+            Y1.upload(np.full((M1, N1), np.nan, np.float32))
+            for _ in range(4):
+                ctx.mul_mat_q(*large)
+                assert gr.h.hipGraphLaunch(ex, other) == 0
+            ctx.sync()
+            assert gr.h.hipStreamSynchronize(other) == 0
+            assert np.array_equal(Y0.download(np.float32, (M0, N0)), want0), rep
+            assert np.array_equal(Y1.download(np.float32, (M1, N1)), want1), rep
+    finally:
+        gr.h.hipGraphExecDestroy(ex)
+        gr.h.hipGraphDestroy(g)
+        gr.h.hipStreamDestroy(other)
