@@ -109,10 +109,11 @@ int s3e_weight_info(const s3e_weight *w, int64_t out[4]);
  * The converted X lives in a workspace that the context keeps and shares
  * with s3e_flash_attn_ext, as large as the largest call so far (freed with the
  * context); a call that needs more than 1 GiB allocates for itself.  Calls
- * that convert wait for their result before they return.  Products with few
- * output tiles add up K in ranges whose partial sums take 25 MB of the context
- * (made once; not while its stream is being captured: a captured s3e_mul_mat_q
- * sums K in one range, equal up to fp32 summation order). */
+ * that convert wait for their result before they return.  Products above 64
+ * rows with few output tiles add up K in ranges whose partial sums take a 25 MB
+ * workspace made with the context (a context that found no memory for it, and
+ * a product captured into a graph, sum K in one range, equal up to fp32
+ * summation order). */
 int s3e_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const float *X, int64_t M,
                 const float *bias, float *Y);
 
@@ -134,11 +135,12 @@ int s3e_mul_mat_noalloc(s3e_ctx *ctx, const s3e_weight *w, const float *X, int64
 /* Same GEMM with X already in W's vec_dot type (ggml_mul_mat with src1 of
  * that type; ggml skips the conversion then): `xq`, `d`, `s` as written by
  * s3e_quantize_rows for K = W's ne0 (layout there).  Launches the GEMM kernel
- * only, so it is also the entry point to time the kernel alone.  Products of
+ * only (and, where K goes in ranges, the one that adds them up), so it is also
+ * the entry point to time the kernel alone.  Products of
  * at most 64 rows with Q4_0/Q4_1/Q8_0/F16 weights run on the weight-streaming
  * kernel.  s3e_weight_upload makes everything that kernel needs: the
- * block-interleaved copy of the weight and room in the uploading context's
- * workspace for the partial sums of a K-split product of up to 64 rows.  So
+ * block-interleaved copy of the weight and the uploading context's workspace
+ * for the partial sums of a K-split product of up to 64 rows.  So
  * s3e_mul_mat_q allocates nothing and does not synchronise; on a context
  * other than the upload's, a small product whose partial sums do not fit
  * that context's workspace runs with K unsplit (same kernel, results equal
@@ -150,7 +152,7 @@ int s3e_mul_mat_q(s3e_ctx *ctx, const s3e_weight *w, const void *xq, const uint1
  * s3e_mul_mat and the encoder run for Q4_0: each 32-block sum comes from the
  * fp6 MFMA, the same integers as the int8 path, so Y equals s3e_mul_mat_q's
  * bit for bit.  K must be a multiple of 128; any M (no small-M kernel).
- * Launches the GEMM kernel only. */
+ * Launches the GEMM kernel only (and the sum of its K ranges, as above). */
 int s3e_mul_mat_q_f6(s3e_ctx *ctx, const s3e_weight *w, const void *xq, const uint16_t *d, int64_t M,
                      const float *bias, float *Y);
 

@@ -278,6 +278,25 @@ std::vector<float> sinusoidal_pe_2d(int H, int W, int d) {
 // ---- end of shared host helpers ----
 
 // ---------------------------------------------------------------------------
+namespace {
+
+// The context's workspace for the partial sums of products above 64 rows (a
+// split product has fewer than 768 tile × range pairs), made with the context
+// so that no product allocates.  Without the memory for it they run unsplit.
+// (Relaxed capture mode: another stream's capture may be open.)
+constexpr int64_t TILE_PARTS = 768LL * 64 * GEMM_BN;
+void tile_workspace(s3e_ctx *ctx) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (hipMalloc(&ctx->tile_part, (size_t)TILE_PARTS * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->tile_part = nullptr;
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+}
+
+}  // namespace
+
 extern "C" const char *s3e_last_error(void) { return g_err.c_str(); }
 extern "C" int s3e_abi_version(void) { return S3E_ABI_VERSION; }
 
@@ -304,6 +323,7 @@ extern "C" int s3e_ctx_create(int device, s3e_ctx **out) try {
         set_error("hipStreamCreate: %s", hipGetErrorString(e));
         return S3E_ERR_HIP;
     }
+    tile_workspace(c);
     *out = c;
     return S3E_OK;
 } S3E_CATCH("s3e_ctx_create")
@@ -475,24 +495,16 @@ int sm_kgroups(const Weight &W) {
     return std::max(1, std::min({SM_WG_GOAL / cgs, nst / (SM_KS * SM_MIN_STAGES), SM_KG_MAX}));
 }
 
-// The context's workspaces for partial sums, each made once at its largest and
-// never moved.  Small-M products (at most SM_WG_GOAL work-groups of 32 columns)
-// have one of their own: where captured, they hold its address, and a graph may
-// be replayed on another stream beside eager products of any size.
+// The context's workspace for the partial sums of small-M products (at most
+// SM_WG_GOAL work-groups of 32 columns), made once at its largest and never moved.
+// No larger product writes there: captured small-M products hold its address,
+// and a graph may be replayed on another stream beside eager products.
 constexpr int64_t SK_PARTS = SM_WG_GOAL * 32LL * 64;
 hipError_t sk_workspace(s3e_ctx *ctx) {
     if (ctx->sk_part) return hipSuccess;
     const hipError_t e = hipMalloc(&ctx->sk_part, (size_t)SK_PARTS * sizeof(float));
     if (e != hipSuccess) ctx->sk_part = nullptr;
     else ctx->sk_part_cap = SK_PARTS;
-    return e;
-}
-// (a split product has fewer than 768 tile × range pairs)
-constexpr int64_t TILE_PARTS = 768LL * 64 * GEMM_BN;
-hipError_t tile_workspace(s3e_ctx *ctx) {
-    if (ctx->tile_part) return hipSuccess;
-    const hipError_t e = hipMalloc(&ctx->tile_part, (size_t)TILE_PARTS * sizeof(float));
-    if (e != hipSuccess) ctx->tile_part = nullptr;
     return e;
 }
 
@@ -543,12 +555,11 @@ bool sm_converts(const Weight &W, int64_t M) {
 // on another stream, beside calls that use that workspace.
 hipError_t run_tiles(s3e_ctx *ctx, const Weight &W, const Act &a, int64_t M, EpiArgs ea) {
     ea.lone = true;
-    if (gemm_splitk_floats(W, M, false) > 0) {
+    if (ctx->tile_part && gemm_splitk_floats(W, M, false) > 0) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        hipError_t e = hipStreamIsCapturing(ctx->stream, &cap);
+        const hipError_t e = hipStreamIsCapturing(ctx->stream, &cap);
         if (e != hipSuccess) return e;
         if (cap == hipStreamCaptureStatusNone) {
-            if ((e = tile_workspace(ctx)) != hipSuccess) return e;
             ea.ws = ctx->tile_part;
             ea.ws_cap = TILE_PARTS;
         }

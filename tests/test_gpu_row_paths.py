@@ -151,3 +151,32 @@ def test_captured_small_product_beside_large_ones(ctx, t):
         gr.h.hipGraphExecDestroy(ex)
         gr.h.hipGraphDestroy(g)
         gr.h.hipStreamDestroy(other)
+
+
+def test_first_large_product_allocates_nothing(ctx):
+    # a context's first split product, while another stream's capture (global mode) is open: an allocation would end it
+    M, N, K = 300, 96, 1024
+    c = s3e.Context(0)
+    rng = np.random.default_rng(8)
+    W, X = (rng.standard_normal(n).astype(np.float32) for n in ((N, K), (M, K)))
+    w, Xd, Y = c.weight(orc.F32, K, N, orc.to_weight_bytes(orc.F32, W)), c.to_device(X), c.buffer(M * N * 4)
+    x1, q1 = ctx.to_device(X), ctx.buffer(M * K * 2)
+    made = []
+
+    def calls():
+        c.mul_mat_q(w, Xd, None, None, M, Y)
+        ctx.quantize_rows(s3e.TYPE_F16, x1, M, K, q1, None, None)
+        made.append(s3e.Context(0))
+
+    gr = _Graphs()
+    try:
+        g, ex = gr.capture(ctx.stream, calls)
+        gr.h.hipGraphExecDestroy(ex)
+        gr.h.hipGraphDestroy(g)
+        c.sync()
+        assert orc.rel_l2(Y.download(np.float32, (M, N)), X.astype(np.float64) @ W.T.astype(np.float64)) <= 1e-6
+    finally:
+        for b in (w, Xd, Y):
+            b.free()
+        for x in (c, *made):
+            x.close()
