@@ -106,6 +106,7 @@ int s3e_weight_info(const s3e_weight *w, int64_t out[4]);
  * for F16, 4·K for F32, padded to 128-byte stages) and the repacked W must
  * each stay below 2 GiB; larger products return S3E_ERR_HIP.  M = 0 (an
  * empty batch) succeeds and writes nothing; M < 0 is S3E_ERR_INVALID.
+ * Y may overlap X where X is converted (every type but F32).
  * The converted X lives in a workspace that the context keeps and shares
  * with s3e_flash_attn_ext, as large as the largest call so far (freed with the
  * context); a call that needs more than 1 GiB allocates for itself.  Calls

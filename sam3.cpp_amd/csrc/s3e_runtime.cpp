@@ -538,12 +538,17 @@ hipError_t s3e::CallWs::get(size_t bytes, void **out) {
 
 namespace {
 
+bool overlap(const void *a, size_t an, const void *b, size_t bn) {
+    return (uintptr_t)a < (uintptr_t)b + bn && (uintptr_t)b < (uintptr_t)a + an;
+}
+
 // Whether a small-M product converts its rows inside the kernel.  Every
 // 32-column strip repeats the conversion of its K range, so few rows (little to
 // load and convert) or a small weight (few strips, short ranges) favour it: at
 // Q4_0, µs a call in two passes and in one, 7 × 1024 × 1024 21.2 → 19.3, 7 × 4736
 // × 1024 20.1 → 19.2, 64 × 1024 × 1024 21.7 → 20.5, but 64 × 4736 × 1024 22.5 →
 // 26.0 and 64 × 1024 × 4736 24.4 → 26.7.  fp16 rows cost less to convert.
+// (Not where Y overlaps X: work-groups would store before others have read.)
 bool sm_converts(const Weight &W, int64_t M) {
     return sm_eligible(W, M) && (M <= (W.kind == WK_F16 ? 32 : 16) || W.N * W.K <= (int64_t)1 << 21);
 }
@@ -670,7 +675,7 @@ extern "C" int s3e_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const float *X, in
     hipError_t e;
     Act a;
     a.ld = W.K;
-    if (sm_converts(W, M)) {
+    if (sm_converts(W, M) && !overlap(X, (size_t)(M * W.K) * 4, Y, (size_t)(M * W.N) * 4)) {
         e = run_mul_mat(ctx, w, a, M, ea, X);
     } else {
         // [values of X in the product's format][d][s (Q8_1)].  Rows past M of

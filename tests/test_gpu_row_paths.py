@@ -70,6 +70,24 @@ def test_large_values_at_the_end_of_a_row(ctx, t, M, N, K, at, value):
 
 
 @pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("M,N,K,shift", [(1, 256, 256, 0), (7, 256, 256, 0), (64, 256, 256, 0), (16, 96, 160, 0), (16, 160, 96, 0),
+                                         (33, 256, 256, 5000), (200, 256, 256, 0)])
+def test_output_over_input(ctx, t, M, N, K, shift):
+    # Y over X, or starting `shift` floats into it
+    _, X, bias, w = _inputs(ctx, t, M, N, K, M + N)
+    Xd, Bd, Y = ctx.to_device(X), ctx.to_device(bias), ctx.buffer(M * N * 4)
+    both = ctx.buffer((shift + M * max(N, K)) * 4)
+    over = s3e.DeviceView(both.ptr + 4 * shift, M * N * 4)
+    print(t, M, N, K, shift, flush=True)
+    ctx.mul_mat(w, Xd, M, Y, Bd)
+    both.upload(X)
+    ctx.mul_mat(w, both, M, over, Bd)
+    ctx.sync()
+    got = both.download(np.float32, shift + M * N)[shift:].reshape(M, N)
+    assert np.array_equal(got, Y.download(np.float32, (M, N)))
+
+
+@pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("M,N,K", [(65, 128, 512), (65, 96, 1024), (129, 1024, 4736), (1601, 1024, 4736),
                                    (200, 130, 2080), (2048, 1024, 448), (1984, 1024, 64), (2049, 1024, 1056)])
 def test_split_products(ctx, t, M, N, K):
