@@ -204,7 +204,8 @@ int s3e_layer_norm(s3e_ctx *ctx, const float *x, int64_t rows, int64_t n, float 
  * Tensors are f32 device memory addressed by ggml-style element strides:
  * Q(b,h,i,d) = q[b*q_nb[3] + h*q_nb[2] + i*q_nb[1] + d] (d contiguous), K and
  * V likewise (V may be the strided view of sam3.cpp:3762-3763).  O follows
- * ggml's output layout [D, nh, Nq, B]: o[((b*Nq + i)*nh + h)*D + d].
+ * ggml's output layout [D, nh, Nq, B]: o[((b*Nq + i)*nh + h)*D + d].  O may
+ * overlap Q, K and V.
  * D: any multiple of 4 up to 128 (the ViT's 64; Hiera's 96, 56, 72, 32 —
  * run zero-padded to 64 or 128 channels, sam3.cpp:4395), or 256 (the
  * memory attention, sam3.cpp:9267, :9312; S3E_PREC_DEFAULT only).  Nq and

@@ -862,6 +862,18 @@ struct AttnSplit {
     }
 };
 
+// Whether O's `bytes` overlap a tensor of [B][nh][N][D] elements of `size` bytes
+// by strides, which the attention kernel reads where it lies: O then goes
+// through the workspace, as work-groups would store before others have read.
+// (Not where the keys are split: the pass that adds the ranges up comes after.)
+bool over(const float *o, size_t bytes, const void *x, const int64_t nb[4], int64_t N, int64_t nh, int64_t B, int64_t D,
+          int64_t size) {
+    const int64_t step[3] = {(N - 1) * nb[1], (nh - 1) * nb[2], (B - 1) * nb[3]};
+    int64_t lo = 0, hi = D;
+    for (const int64_t s : step) (s < 0 ? lo : hi) += s;
+    return overlap(o, bytes, (const uint8_t *)x + lo * size, (size_t)((hi - lo) * size));
+}
+
 void set_strides(int64_t dst[3], const int64_t nb[4]) {
     for (int i = 0; i < 3; i++) dst[i] = nb[i + 1];
 }
@@ -912,10 +924,13 @@ extern "C" int s3e_flash_attn_ext(s3e_ctx *ctx, const float *q, const int64_t q_
     const int64_t ldv = vt_ld_for(Nkv);
     const size_t kn = (size_t)(BH * Nkv * hdp), vn = hdp == 256 ? (size_t)(BH * hdp * ldv) : kn;
     const AttnSplit sp(BH, Nq, Nkv, hdp);
-    // [K hi, lo][V hi, lo][partials]; every plane is a multiple of 128 bytes
+    const size_t ob = (size_t)(BH * Nq * D) * 4;
+    const bool via = sp.n == 1 && over(o, ob, q, q_nb, Nq, nh, B, D, 4);
+    // [K hi, lo][V hi, lo][partials, or O]; every plane is a multiple of 128 bytes
     CallWs ws(ctx);
     void *base = nullptr;
-    hipError_t e = ws.get((kn + vn) * 2 * np + sp.bytes(), &base);
+    hipError_t e = ws.get((kn + vn) * 2 * np + (via ? ob : sp.bytes()), &base);
+    uint8_t *const tail = (uint8_t *)base + (kn + vn) * 2 * np;
     AttnArgs a;
     if (e == hipSuccess) {
         _Float16 *k16 = (_Float16 *)base, *v16 = k16 + kn * np;
@@ -936,10 +951,11 @@ extern "C" int s3e_flash_attn_ext(s3e_ctx *ctx, const float *q, const int64_t q_
         if (e == hipSuccess && hdp == 256) e = launch_vt(v, v_nb, Nkv, nh, B, v16, ldv, ctx->stream);
     }
     if (e == hipSuccess) {
-        set_shape(a, D, hdp, Nq, Nkv, nh, BH, scale, o);
-        sp.set(a, (uint8_t *)base + (kn + vn) * 2 * np);
+        set_shape(a, D, hdp, Nq, Nkv, nh, BH, scale, via ? (float *)tail : o);
+        sp.set(a, tail);
         e = launch_attn(a, ctx->stream);
     }
+    if (e == hipSuccess && via) e = hipMemcpyAsync(o, tail, ob, hipMemcpyDeviceToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) { set_error("s3e_flash_attn_ext: %s", hipGetErrorString(e)); return S3E_ERR_HIP; }
     return S3E_OK;
@@ -978,10 +994,13 @@ extern "C" int s3e_flash_attn_ext_f16(s3e_ctx *ctx, const uint16_t *q, const int
     const bool k_in = in_place(k, k_nb), v_t = hdp == 256, v_in = !v_t && in_place(v, v_nb);
     const int64_t ldv = vt_ld_for(Nkv);
     const AttnSplit sp(BH, Nq, Nkv, hdp);
-    // workspace: [K copy][V copy or Vᵀ][partials]; a copy is a multiple of 128 bytes
+    const size_t ob = (size_t)(BH * Nq * D) * 4;
+    const bool via = sp.n == 1 && (over(o, ob, q, q_nb, Nq, nh, B, D, 2) || (k_in && over(o, ob, k, k_nb, Nkv, nh, B, D, 2)) ||
+                                   (v_in && over(o, ob, v, v_nb, Nkv, nh, B, D, 2)));
+    // workspace: [K copy][V copy or Vᵀ][partials, or O]; a copy is a multiple of 128 bytes
     const size_t kn = k_in ? 0 : (size_t)(BH * Nkv * hdp);
     const size_t vn = v_in ? 0 : (size_t)(BH * hdp * (v_t ? ldv : Nkv));
-    const size_t need = (kn + vn) * 2 + sp.bytes();
+    const size_t need = (kn + vn) * 2 + (via ? ob : sp.bytes());
     if (need > ctx->attn_ws_cap) {
         HIP_TRY(hipStreamSynchronize(ctx->stream));  // earlier calls may still read it
         if (ctx->attn_ws) (void)hipFree(ctx->attn_ws);
@@ -1012,9 +1031,11 @@ extern "C" int s3e_flash_attn_ext_f16(s3e_ctx *ctx, const uint16_t *q, const int
                                k_in ? nullptr : k16, v_in || v_t ? nullptr : v16, ctx->stream);
     if (e == hipSuccess && v_t) e = launch_vt((const _Float16 *)v, v_nb, Nkv, nh, B, v16, ldv, ctx->stream);
     if (e == hipSuccess) {
-        set_shape(a, D, hdp, Nq, Nkv, nh, BH, scale, o);
-        sp.set(a, (uint8_t *)ctx->attn_ws + (kn + vn) * 2);
+        uint8_t *const tail = (uint8_t *)ctx->attn_ws + (kn + vn) * 2;
+        set_shape(a, D, hdp, Nq, Nkv, nh, BH, scale, via ? (float *)tail : o);
+        sp.set(a, tail);
         e = launch_attn(a, ctx->stream);
+        if (e == hipSuccess && via) e = hipMemcpyAsync(o, tail, ob, hipMemcpyDeviceToDevice, ctx->stream);
     }
     if (e != hipSuccess) { set_error("s3e_flash_attn_ext_f16: %s", hipGetErrorString(e)); return S3E_ERR_HIP; }
     return S3E_OK;
