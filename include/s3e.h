@@ -128,7 +128,10 @@ int s3e_mul_mat(s3e_ctx *ctx, const s3e_weight *w, const float *X, int64_t M,
  * to fp32 summation order).  Calls no hipMalloc / hipFree and does not
  * synchronise.  A product whose conversion exceeds the array returns
  * S3E_ERR_INVALID.  All calls on one GPU share its array and leave their
- * contents in it: calls that overlap on one GPU race. */
+ * contents in it: calls that overlap on one GPU race (not F32 products, which
+ * convert nothing and leave the array alone).  Partial sums of K ranges lie
+ * behind the converted rows; where they do not fit, and for F32 under capture, K
+ * goes in one range (equal up to fp32 summation order). */
 #define S3E_NOALLOC_SCRATCH_BYTES (64ull << 20)
 int s3e_mul_mat_noalloc(s3e_ctx *ctx, const s3e_weight *w, const float *X, int64_t M, const float *bias,
                         float *Y);

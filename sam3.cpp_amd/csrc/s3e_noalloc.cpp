@@ -2,8 +2,8 @@
 // allocate device memory (code under HIP graph capture, serving loops that
 // forbid hipMalloc).  The activation conversion that s3e_mul_mat allocates per
 // call goes to `scratch`, one file-scope device array per GPU of a fixed
-// size, held until the process ends.  Every call on a GPU shares that GPU's
-// array and leaves its contents behind: calls that overlap on one GPU
+// size, held until the process ends.  Every call that converts shares its GPU's
+// array and leaves its contents behind: such calls that overlap on one GPU
 // (different streams, threads or contexts) race.
 #include <hip/hip_runtime.h>
 
@@ -77,21 +77,13 @@ extern "C" int s3e_mul_mat_noalloc(s3e_ctx *ctx, const s3e_weight *w, const floa
     a.kind = ak;
     a.ld = W.K;
     a.mp = round_up(M, ROW_PAD);
-    ea.lone = true;
-    // a product split over K leaves its partial sums in the scratch array
-    // too, behind the converted rows, where there is room for them
-    const int64_t parts = gemm_splitk_floats(W, M, false);
-    auto split_at = [&](int64_t used) {
-        if (parts > 0 && used + parts * 4 <= (int64_t)S3E_NOALLOC_SCRATCH_BYTES) {
-            ea.ws = (float *)((uint8_t *)ctx->scratch + used);
-            ea.ws_cap = parts;
-        }
-    };
     hipError_t e = hipSetDevice(ctx->device);
-    if (ak == A_F32) {  // f32 weights take the rows as they are
+    if (ak == A_F32) {
+        // f32 weights take the rows as they are and nothing of the scratch
+        // array: such calls may overlap on different contexts
         a.x = (void *)X;
-        split_at(0);
-        if (e == hipSuccess) e = launch_gemm(W, a, M, EPI_F32, ea, ctx->stream);
+        std::lock_guard<std::mutex> lock(ctx->call_mu);
+        if (e == hipSuccess) e = run_tiles(ctx, W, a, M, ea);
     } else {
         // [values M × K][d: (Kp/128) groups × mp rows × 4 fp16][s: same, Q8_1]
         const bool q8 = ak == A_Q8_0 || ak == A_Q8_1;
@@ -105,7 +97,14 @@ extern "C" int s3e_mul_mat_noalloc(s3e_ctx *ctx, const s3e_weight *w, const floa
         }
         uint8_t *base = (uint8_t *)ctx->scratch;
         a.x = base;
-        split_at(need);
+        ea.lone = true;
+        // a product split over K leaves its partial sums in the scratch array
+        // too, behind the converted rows, where there is room for them
+        const int64_t parts = gemm_splitk_floats(W, M, false);
+        if (parts > 0 && need + parts * 4 <= (int64_t)S3E_NOALLOC_SCRATCH_BYTES) {
+            ea.ws = (float *)(base + need);
+            ea.ws_cap = parts;
+        }
         if (q8) {
             a.d = (uint16_t *)(base + vbytes);
             if (ak == A_Q8_1) a.s = (uint16_t *)(base + vbytes + pbytes);

@@ -89,6 +89,10 @@ private:
     void *own_ = nullptr;
 };
 
+// A product of any M on the tiled kernels, on the context's stream; the caller
+// holds call_mu (s3e_runtime.cpp).
+hipError_t run_tiles(s3e_ctx *ctx, const Weight &W, const Act &a, int64_t M, EpiArgs ea);
+
 // A tensor record as read from a model file.
 struct RawTensor {
     int type = 0;

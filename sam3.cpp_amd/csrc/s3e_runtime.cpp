@@ -510,6 +510,25 @@ hipError_t sk_workspace(s3e_ctx *ctx) {
 
 }  // namespace
 
+// A product on the tiled kernels.  Where few tiles leave CUs idle, K goes in
+// ranges whose partial sums lie in the context's workspace (1601 × 1024 × 4736
+// Q8_0, 208 tiles: 45.6 µs on one range, 34.4 + 5.1 on three).  While the
+// stream is being captured the product runs unsplit: a graph may be replayed
+// on another stream, beside calls that use that workspace.
+hipError_t s3e::run_tiles(s3e_ctx *ctx, const Weight &W, const Act &a, int64_t M, EpiArgs ea) {
+    ea.lone = true;
+    if (ctx->tile_part && gemm_splitk_floats(W, M, false) > 0) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        const hipError_t e = hipStreamIsCapturing(ctx->stream, &cap);
+        if (e != hipSuccess) return e;
+        if (cap == hipStreamCaptureStatusNone) {
+            ea.ws = ctx->tile_part;
+            ea.ws_cap = TILE_PARTS;
+        }
+    }
+    return launch_gemm(W, a, M, EPI_F32, ea, ctx->stream);
+}
+
 hipError_t s3e::CallWs::get(size_t bytes, void **out) {
     *out = nullptr;
     if (bytes > CALL_WS_MAX) {
@@ -551,25 +570,6 @@ bool overlap(const void *a, size_t an, const void *b, size_t bn) {
 // (Not where Y overlaps X: work-groups would store before others have read.)
 bool sm_converts(const Weight &W, int64_t M) {
     return sm_eligible(W, M) && (M <= (W.kind == WK_F16 ? 32 : 16) || W.N * W.K <= (int64_t)1 << 21);
-}
-
-// A product on the tiled kernels.  Where few tiles leave CUs idle, K goes in
-// ranges whose partial sums lie in the context's workspace (1601 × 1024 × 4736
-// Q8_0, 208 tiles: 45.6 µs on one range, 34.4 + 5.1 on three).  While the
-// stream is being captured the product runs unsplit: a graph may be replayed
-// on another stream, beside calls that use that workspace.
-hipError_t run_tiles(s3e_ctx *ctx, const Weight &W, const Act &a, int64_t M, EpiArgs ea) {
-    ea.lone = true;
-    if (ctx->tile_part && gemm_splitk_floats(W, M, false) > 0) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        const hipError_t e = hipStreamIsCapturing(ctx->stream, &cap);
-        if (e != hipSuccess) return e;
-        if (cap == hipStreamCaptureStatusNone) {
-            ea.ws = ctx->tile_part;
-            ea.ws_cap = TILE_PARTS;
-        }
-    }
-    return launch_gemm(W, a, M, EPI_F32, ea, ctx->stream);
 }
 
 // x32: the rows of a product of at most 64 rows in f32 (a.x is then unused)

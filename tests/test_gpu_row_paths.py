@@ -198,3 +198,30 @@ def test_first_large_product_allocates_nothing(ctx):
             b.free()
         for x in (c, *made):
             x.close()
+
+
+def test_f32_noalloc_products_overlap(ctx):
+    # two contexts at once: F32 products convert nothing and keep their partial sums apart
+    c = s3e.Context(0)
+    calls = []
+    try:
+        for i, x in enumerate((ctx, c)):
+            M, N, K = 300 + i, 512, 1024
+            _, X, bias, w = _inputs(x, orc.F32, M, N, K, 20 + i)
+            Y = x.buffer(M * N * 4)
+            args = (w, x.to_device(X), M, Y, x.to_device(bias))
+            x.mul_mat_noalloc(*args)
+            x.sync()
+            calls.append((x, args, Y, Y.download(np.float32, (M, N))))
+        for rep in range(5):
+            for x, args, Y, want in calls:
+                Y.upload(np.full(want.shape, np.nan, np.float32))
+            for _ in range(8):
+                for x, args, Y, want in calls:
+                    x.mul_mat_noalloc(*args)
+            for x, args, Y, want in calls:
+                x.sync()
+                assert np.array_equal(Y.download(np.float32, want.shape), want), rep
+        calls[1][1][0].free()
+    finally:
+        c.close()
