@@ -1,8 +1,9 @@
 """The device's ggml_gelu computes x / (1 + e^(−2u)) and keeps the result only
 where fp16 rounds both ends of an error interval alike (gelu_tanh_half,
-csrc/s3e_internal.h).  Over every fp16 input: with the exponential and the
-reciprocal off by one unit in the last place either way, a kept result is the
-entry of ggml's table, and few inputs in use need the table.
+csrc/s3e_internal.h).  Restated here, over every fp16 input: with the
+exponential and the reciprocal off by one unit in the last place either way, a
+kept result is the entry of ggml's table, and few inputs in use need the table.
+The device's own results over every fp16 input: test_gpu_frame_products.py.
 """
 import numpy as np
 
@@ -31,7 +32,7 @@ def _kept(x, de, dr):
 def test_kept_results_are_the_table():
     bits = np.arange(65536, dtype=np.uint32).astype(np.uint16)
     x = bits.view(np.float16).astype(F)
-    use = np.abs(x) < 10
+    use = np.abs(x) <= 10  # (values just inside ±10 round to them)
     x, bits = x[use], bits[use]
     table = np.empty(65536, np.uint16)
     orc.LIB.orc_gelu_tanh_table(orc.ptr(table))

@@ -8,6 +8,7 @@ import os
 import numpy as np
 import pytest
 
+import oracle_lib as orc
 import s3e
 from model_patch import patched
 
@@ -91,3 +92,69 @@ def test_memory_attention_linear2_sums_in_ranges_of_512(ctx, tmpdir_session):
         ctx.sync()
         y = out.download(np.float32, (N, 256))
         assert (y[:, ::2] > 0.9).all() and (y[:, 1::2] < -0.9).all()
+
+
+def test_gelu_of_every_fp16_value(ctx, tmpdir_session):
+    """fc1 + ggml_gelu of an F16 file, bit for bit ggml's fp16 table: every fp16 value below 16 in size, and values that
+    round to ±10 from inside."""
+    src, path = (os.path.join(str(tmpdir_session), n) for n in ("gelu.ggml", "gelu_all.ggml"))
+    s3e.synth_write_sam2(src, "hiera_t", img_size=256, ftype="f16", seed=5, stages=(1, 1, 1, 1), global_idx=())
+    T, C, U, first = 4096, 96, 20, 2
+    # token t's first normalised channel is a[t]: each fp16 mantissa of [1, 2) and 0 .. 1023 / 1024, both signs
+    a = np.concatenate([1 + np.arange(1024) / 1024, np.arange(1024) / 1024])
+    a = np.concatenate([a, -a]).astype(np.float32)
+    x = np.zeros((T, C), np.float32)  # (mean 0 and variance 1; channels first .. first + U - 1 stay 0)
+    x[:, 0], x[:, 1] = a, -a
+    fill = C - first - U
+    x[:, first + U :] = np.sqrt((C - 2 * a.astype(np.float64) ** 2) / fill)[:, None] * np.where(np.arange(fill) % 2, 1, -1)
+    # hidden unit j is a·2^(3 - j) (exact), the last two a·8 ∓ 0.001; fc2 puts unit j into channel first + j
+    scale = np.float32(2.0) ** np.r_[3:-15:-1, 3, 3].astype(np.float32)
+    bias = np.zeros(4 * C, np.float32)
+    bias[U - 2 : U] = -0.001, 0.001
+    w1, w2 = np.zeros((4 * C, C), np.float32), np.zeros((C, 4 * C), np.float32)
+    w1[:U, 0] = scale
+    w2[first + np.arange(U), np.arange(U)] = 1
+    p = "hiera.blocks.0."
+    patched(src, path, {
+        p + "attn.proj.weight": 0, p + "attn.proj.bias": 0, p + "norm2.weight": 1, p + "norm2.bias": 0, p + "mlp.fc1.weight": w1,
+        p + "mlp.fc1.bias": bias, p + "mlp.fc2.weight": w2, p + "mlp.fc2.bias": 0})
+    normed = orc.layer_norm(x, 1e-6)[:, 0].astype(np.float16)
+    assert np.array_equal(normed, a.astype(np.float16))
+    pre = normed.astype(np.float32)[:, None] * scale + bias[:U]
+    seen = np.unique(np.abs(pre.astype(np.float16)).view(np.uint16))
+    assert np.array_equal(seen[seen < np.float16(15.99).view(np.uint16)], np.arange(np.float16(15.99).view(np.uint16)))
+    y = ctx.buffer(T * C * 4)
+    print("gelu", flush=True)
+    with _state(ctx, path) as st:
+        st.hiera_block(0, ctx.to_device(x), 64, 64, y)
+        ctx.sync()
+        got = y.download(np.float32, (T, C))[:, first : first + U]
+    want = orc.gelu_tanh(pre).astype(np.float16).astype(np.float32)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("img", [416, 1024])
+def test_fpn_products_on_split_fp16_weights(ctx, tmpdir_session, img):
+    """The F32 laterals of a quantized file, fp16 pairs on either side: few tiles (six stages in flight) and many, ragged
+    rows, K from 96 to 768.  2^-22 per operand and fp32 sums."""
+    path = os.path.join(str(tmpdir_session), "fpn.ggml")
+    s3e.synth_write_sam2(path, "hiera_t", img_size=1024, ftype="q8_0", seed=6, std=0.05, random_affine=True, stages=(1, 1, 1, 1),
+                         global_idx=(), scalp=0)
+    files = orc.read_model_file(path)
+    gm = s3e.Model(ctx, path)
+    st = s3e.State(ctx, gm, img)
+    try:
+        chw = np.random.default_rng(img).standard_normal((3, img, img)).astype(np.float32)
+        st.encode_chw(ctx.to_device(chw))
+        ctx.sync()
+        for i in (0, 1, 3):  # level 2 also takes level 3 from above
+            w, b = (files[f"fpn.convs.{3 - i}." + n][2].astype(np.float64) for n in ("weight", "bias"))
+            rows, K = (img // (4 << i)) ** 2, 96 << i
+            x, y = st.tensor(f"hiera_stage_{i}").reshape(rows, K), st.tensor(f"neck_trk_{i}").reshape(rows, 256)
+            ref = x.astype(np.float64) @ w.reshape(256, K).T + b
+            err = orc.rel_l2(y, ref)
+            print(img, i, rows, K, err, flush=True)
+            assert err <= 1e-6
+    finally:
+        st.free()
+        gm.free()

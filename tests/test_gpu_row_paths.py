@@ -87,7 +87,7 @@ def test_output_over_input(ctx, t, M, N, K, shift):
     assert np.array_equal(got, Y.download(np.float32, (M, N)))
 
 
-@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("t", TYPES + [orc.F32])
 @pytest.mark.parametrize("M,N,K", [(65, 128, 512), (65, 96, 1024), (129, 1024, 4736), (1601, 1024, 4736),
                                    (200, 130, 2080), (2048, 1024, 448), (1984, 1024, 64), (2049, 1024, 1056)])
 def test_split_products(ctx, t, M, N, K):
@@ -97,7 +97,10 @@ def test_split_products(ctx, t, M, N, K):
     ctx.mul_mat(w, ctx.to_device(X), M, Y, ctx.to_device(bias))
     ctx.sync()
     pick = np.unique(np.r_[0:3, M // 2 : M // 2 + 3, M - 3 : M])  # rows are independent: the oracle takes a few
-    ref = orc.mul_mat(t, wb, N, K, X[pick]).astype(np.float64) + bias
+    if t == orc.F32:
+        ref = X[pick].astype(np.float64) @ wb.view(np.float32).reshape(N, K).astype(np.float64).T + bias
+    else:
+        ref = orc.mul_mat(t, wb, N, K, X[pick]).astype(np.float64) + bias
     got = Y.download(np.float32, (M, N))
     assert np.isfinite(got).all()
     assert orc.rel_l2(got[pick], ref) <= 1e-6
