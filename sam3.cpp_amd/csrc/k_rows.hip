@@ -352,7 +352,7 @@ __global__ void k_im2col(const float *__restrict__ chw, int img, int P, int64_t 
     }
 }
 
-// Strided K (blockIdx.z 0) and V (1) rows, f32 or fp16 with head dim D, to fp16
+// Strided K and V rows (one of them per blockIdx.z), f32 or fp16 with head dim D, to fp16
 // [BH][N][hdp], channels D..hdp−1 zero; f32 with lo planes as pairs hi =
 // fp16(v), lo = fp16(v − hi).  Bound by its traffic: one thread moves 8
 // channels (two or one 16-byte loads when VEC, 16-byte stores), blockIdx.y is
@@ -368,7 +368,6 @@ struct PrepRows {
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void k_attn_prep(PrepRows p, int N, int nh, int D, int lg) {
     const int z = blockIdx.z, bh = blockIdx.y;
-    if (!p.hi[z]) return;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t row = idx >> lg;
     if (row >= N) return;
@@ -568,15 +567,21 @@ hipError_t attn_prep(PrepRows p, const int64_t *k_nb, const int64_t *v_nb, int64
     const int64_t *nb[2] = {k_nb, v_nb};
     constexpr int64_t E = 16 / (int64_t)sizeof(T);  // elements of a 16-byte load
     bool vec = true;
+    int n = 0;  // tensors to convert, moved to the front
     for (int z = 0; z < 2; z++) {
         if (!p.hi[z]) continue;
-        p.s1[z] = nb[z][1];
-        p.s2[z] = nb[z][2];
-        p.s3[z] = nb[z][3];
-        vec = vec && (uintptr_t)p.src[z] % 16 == 0 && nb[z][1] % E == 0 && nb[z][2] % E == 0 && nb[z][3] % E == 0;
+        p.src[n] = p.src[z];
+        p.hi[n] = p.hi[z];
+        p.lo[n] = p.lo[z];
+        p.s1[n] = nb[z][1];
+        p.s2[n] = nb[z][2];
+        p.s3[n] = nb[z][3];
+        vec = vec && (uintptr_t)p.src[n] % 16 == 0 && nb[z][1] % E == 0 && nb[z][2] % E == 0 && nb[z][3] % E == 0;
+        n++;
     }
+    if (n == 0) return hipSuccess;
     const int lg = hdp == 64 ? 3 : (hdp == 128 ? 4 : 5);
-    const dim3 grid((unsigned)(((N << lg) + 255) / 256), (unsigned)(B * nh), 2);
+    const dim3 grid((unsigned)(((N << lg) + 255) / 256), (unsigned)(B * nh), (unsigned)n);
     if (vec) hipLaunchKernelGGL((k_attn_prep<T, true>), grid, dim3(256), 0, st, p, (int)N, (int)nh, D, lg);
     else hipLaunchKernelGGL((k_attn_prep<T, false>), grid, dim3(256), 0, st, p, (int)N, (int)nh, D, lg);
     return hipGetLastError();
