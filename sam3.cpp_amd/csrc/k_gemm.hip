@@ -1394,16 +1394,21 @@ hipError_t dispatch_epi(Epi epi, const GemmParams &p, hipStream_t st) {
 // ViT frame (518 per band) and on short K (Hiera's first stages) the 64-row
 // tiles' three work-groups per CU measured as fast or faster.
 constexpr int64_t F16_WIDE_MIN_TILES = 1200;
-// A lone product overlaps nothing else: 5184 × 3072 × 1024 (984 such tiles) 67.8
-// → 63.4 µs a call.  From 480 tiles on every CU has nearly two work-groups.
-constexpr int64_t F16_WIDE_LONE_TILES = 480;
 constexpr int64_t F16_WIDE_MIN_K = 512;
+// A lone product overlaps nothing else, so its rounds of work-groups count: 512
+// wide tiles (two per CU) or 768 of 64 rows (three) at once.  Wide ones where
+// they need fewer rounds.  Kernel µs at N × K, by number of wide tiles, 64-row →
+// wide: 3072 × 1024 at 384 22.0 → 22.4, 432 29.9 → 23.3, 504 30.6 → 24.5, 528 30.9 →
+// 35.4, 648 36.5 → 36.1, 792 45.3 → 41.2, 1008 49.5 → 45.5, 1104 55.2 → 54.9; 768 ×
+// 512 at 510 20.1 → 17.6, 558 21.2 → 24.6, 798 29.7 → 29.3, 1098 35.6 → 37.5; 1024 ×
+// 4736 at 416 108 → 78, 528 118 → 124, 896 183 → 156.
+inline bool f16_wide_lone(int64_t tiles) { return (tiles + 511) / 512 < (2 * tiles + 767) / 768; }
 
 template <int WK>
 hipError_t dispatch_waves(Epi epi, GemmParams &p, hipStream_t st) {
     if constexpr (WK == WK_F16) {
         const int64_t t128 = (int64_t)(p.M + 127) / 128 * p.tiles_n;
-        if (p.ksplit == 1 && t128 >= (p.e.lone ? F16_WIDE_LONE_TILES : F16_WIDE_MIN_TILES) && p.a_kbytes >= 2 * F16_WIDE_MIN_K &&
+        if (p.ksplit == 1 && (t128 >= F16_WIDE_MIN_TILES || (p.e.lone && f16_wide_lone(t128))) && p.a_kbytes >= 2 * F16_WIDE_MIN_K &&
             (epi == EPI_F32 || epi == EPI_GELU || epi == EPI_QKV || epi == EPI_HQKV || epi == EPI_DECONV)) {
             p.tiles_m = (p.M + 127) / 128;
             p.ntiles = p.tiles_m * p.tiles_n;

@@ -106,6 +106,19 @@ def test_split_products(ctx, t, M, N, K):
     assert orc.rel_l2(got[pick], ref) <= 1e-6
 
 
+@pytest.mark.parametrize("M", [6144, 6145, 8064, 8193])
+def test_fp16_tiles_by_rounds(ctx, M):
+    # 384 tiles of 128 x 128 run in 64-row tiles, 392 to 512 wide, 520 in 64-row tiles
+    N, K = 1024, 512
+    wb, X, bias, w = _inputs(ctx, orc.F16, M, N, K, M)
+    Y = ctx.buffer(M * N * 4)
+    print(M, flush=True)
+    ctx.mul_mat(w, ctx.to_device(X), M, Y, ctx.to_device(bias))
+    ctx.sync()
+    ref = X.astype(np.float16).astype(np.float64) @ wb.view(np.float16).reshape(N, K).astype(np.float64).T + bias
+    assert orc.rel_l2(Y.download(np.float32, (M, N)), ref) <= 1e-6
+
+
 @pytest.mark.parametrize("t", [orc.Q8_0, orc.F16])
 def test_captured_product_sums_in_one_range(ctx, t):
     # a graph must not hold the context's workspace: its replays may run beside other calls
