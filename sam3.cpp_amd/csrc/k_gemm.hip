@@ -264,7 +264,7 @@ __device__ __forceinline__ void activate(const EpiArgs &e, const float *bias, fl
 // Epilogue from the fp32 tile Ct [BM][CLD] in LDS (scaled, complete), run by
 // the NT_ threads of the work-group.  tab: EPI_TAB<EPI, BM> bytes of LDS.
 template <int EPI, int BM>
-constexpr int EPI_TAB = EPI == EPI_HQKV || EPI == EPI_QKV ? 4 * (2 * BM + 2 * BN) : 0;
+constexpr int EPI_TAB = EPI == EPI_HQKV ? 4 * (2 * BM + 2 * BN) : 0;
 template <int EPI, int BM, int NT_, bool TABLE = true>
 __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, int *tab, int m0, int n0, int t) {
     const EpiArgs &e = p.e;
@@ -272,24 +272,10 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
         const int sel = n0 / e.E + e.sel0;  // 0 = Q, 1 = K, 2 = V (a tile never straddles)
         const int Nw = e.window * e.window;
         const int nwx = e.grid / e.window;
-        // (window, position) of the tile's tokens and (head, channel) of its
-        // columns, worked out once per tile as for EPI_HQKV below (5184 × 3072 ×
-        // 1024 Q4_0 in the encoder, with the loads before the stores, 59.5 →
-        // 58.2 µs)
-        int2 *const tok = (int2 *)tab;
-        int *const colw = tab + 2 * BM;
-        float *const colb = (float *)(colw + BN);  // the bias (see EPI_RESID on loads behind stores)
-        for (int i = t; i < BM + BN; i += NT_) {
-            if (i < BM) {
-                const int gm = m0 + i, py = gm / e.grid, px = gm - py * e.grid, wy = py / e.window, wx = px / e.window;
-                tok[i] = make_int2(wy * nwx + wx, (py - wy * e.window) * e.window + px - wx * e.window);
-            } else {
-                const int r2 = n0 + i - BM - (sel - e.sel0) * e.E, h = r2 / e.HD;
-                colw[i - BM] = h << 12 | (r2 - h * e.HD);
-                colb[i - BM] = e.bias[n0 + i - BM];
-            }
-        }
-        __syncthreads();
+        // (Positions from tables in LDS and all loads before the first store, as
+        // EPI_HQKV has them, measured slower here: in the banded ViT frame 36.0 →
+        // 38.5 µs for Q4_0, 43.1 → 44.1 Q8_0, 34.4 → 37.8 fp16; a memory-attention
+        // pass 1127 → 1131.)
         if (sel == 2) {
             // Vᵀ [b][h][d][slot]: a unit is one column d and 8 consecutive
             // tokens.  Window and image-row boundaries fall on multiples of 8
@@ -300,8 +286,13 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
                 const int col = u / (BM / 8), r0 = (u % (BM / 8)) * 8;
                 const int gm = m0 + r0;
                 if (gm >= p.M) continue;
-                const float bv = colb[col];
-                const int h = colw[col] >> 12, d = colw[col] & 0xfff, b = tok[r0].x, pp = tok[r0].y;
+                const int gn = n0 + col;
+                const float bv = e.bias[gn];
+                const int r2 = gn - (2 - e.sel0) * e.E;
+                const int h = r2 / e.HD, d = r2 % e.HD;
+                const int py = gm / e.grid, px = gm % e.grid;
+                const int b = (py / e.window) * nwx + px / e.window;
+                const int pp = (py % e.window) * e.window + px % e.window;
                 uint32_t w[4], wl[4];
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
@@ -322,24 +313,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
                 }
             }
         } else {
-            // Q, K [b][h][p][d] with RoPE: a unit is one token and 16 columns;
-            // the angles of all of a thread's units are loaded before the
-            // first store
-            constexpr int UP = BM * (BN / 16) / NT_;
-            float4 cs4[UP][4];
-            if (e.freqs) {
-#pragma unroll
-                for (int k = 0; k < UP; k++) {
-                    const int u = t + k * NT_, row = min(u / (BN / 16), p.M - 1 - m0), cc = u % (BN / 16);
-                    const float4 *f4 = (const float4 *)(e.freqs + ((int64_t)tok[row].y * (e.HD / 2) + (colw[cc * 16] & 0xfff) / 2) * 2);
-                    const bool on = e.rope_rows <= 0 || m0 + row < e.rope_rows;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) cs4[k][j] = on ? f4[j] : make_float4(1.f, 0.f, 1.f, 0.f);
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < UP; k++) {
-                const int u = t + k * NT_;
+            // Q, K [b][h][p][d] with RoPE: a unit is one token and 16 columns
+            for (int u = t; u < BM * (BN / 16); u += NT_) {
                 const int row = u / (BN / 16), cc = u % (BN / 16);
                 const int gm = m0 + row;
                 if (gm >= p.M) continue;
@@ -348,19 +323,24 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const float *Ct, i
 #pragma unroll
                 for (int j = 0; j < 16; j += 4) {
                     const float4 x = *(const float4 *)(Ct + row * CLD + cc * 16 + j);
-                    const float4 bb = *(const float4 *)(colb + cc * 16 + j);
+                    const float4 bb = *(const float4 *)(e.bias + gn0 + j);
                     v[j] = x.x + bb.x;
                     v[j + 1] = x.y + bb.y;
                     v[j + 2] = x.z + bb.z;
                     v[j + 3] = x.w + bb.w;
                 }
-                const int h = colw[cc * 16] >> 12, d0 = colw[cc * 16] & 0xfff, b = tok[row].x, pp = tok[row].y;
+                const int py = gm / e.grid, px = gm % e.grid;
+                const int b = (py / e.window) * nwx + px / e.window;
+                const int pp = (py % e.window) * e.window + px % e.window;
+                const int r2 = gn0 - (sel - e.sel0) * e.E;
+                const int h = r2 / e.HD, d0 = r2 % e.HD;
                 if (e.freqs && (e.rope_rows <= 0 || gm < e.rope_rows)) {
                     // sam3_apply_rope: out_re = re·cos − im·sin, out_im = re·sin + im·cos,
                     // each product rounded on its own (separate ggml ops).
+                    const float4 *f4 = (const float4 *)(e.freqs + ((int64_t)pp * (e.HD / 2) + d0 / 2) * 2);
 #pragma unroll
                     for (int j = 0; j < 16; j += 4) {
-                        const float4 cs = cs4[k][j / 4];  // cos, sin of pairs j/2 and j/2 + 1
+                        const float4 cs = f4[j / 4];  // cos, sin of pairs j/2 and j/2 + 1
                         const float c0 = cs.x, s0 = cs.y, c1 = cs.z, s1 = cs.w;
                         const float re0 = v[j], im0 = v[j + 1], re1 = v[j + 2], im1 = v[j + 3];
                         v[j] = __fsub_rn(__fmul_rn(re0, c0), __fmul_rn(im0, s0));
@@ -1160,7 +1140,7 @@ __global__ __launch_bounds__(256, 3) void k_gemm_f6(GemmParams p) {
     constexpr int OFF_A = 0, OFF_B = 12288, OFF_AD = 24576, OFF_BD = OFF_AD + BM * 8;
     constexpr int STAGE = OFF_BD + BN * 8;  // 26112
     constexpr int LDSZ = 2 * STAGE > BM * CLD * 4 ? 2 * STAGE : BM * CLD * 4;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[LDSZ + EPI_TAB<EPI, BM>];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[LDSZ];
 
     const int per = gridDim.x >> 3;
     const int logical0 = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -1326,7 +1306,7 @@ __global__ __launch_bounds__(256, 3) void k_gemm_f6(GemmParams p) {
             return;
         }
     }
-    epilogue<EPI, BM, NTH, false>(p, Ct, (int *)(lds + LDSZ), m0, n0, t);  // (no table: its registers would spill here)
+    epilogue<EPI, BM, NTH, false>(p, Ct, nullptr, m0, n0, t);  // (no table: its registers would spill here)
 }
 
 // y = Σ_k part[k] (+ bias) for EPI_F32, y += Σ_k part[k] (+ bias) for
