@@ -283,8 +283,8 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
     }
     __syncthreads();
     // (block, part, word) runs: 16 rows × 8 bytes at f6_act_word(.., r0, ..);
-    // 16-byte pieces of rows 2q, 2q + 1 (rows past M land in the padded rows
-    // of the 64-row tile, which no product stores)
+    // 16-byte pieces of rows 2q, 2q + 1, half of one where M ends between them
+    // (rows past M are not written)
     const int64_t nst = o.ld / 128;
     const int npieces = nblk * 6 * 8;
     for (int pc = threadIdx.x; pc < npieces; pc += 64 * LNW) {
@@ -292,13 +292,18 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
         const int blk = run / 6, pt = run % 6;
         if (r0 + 2 * q >= M) continue;
         const uint4 val = *(const uint4 *)(stg + blk * LNF6_BSTRIDE + pt * 16 + 2 * q);
-        *(uint4 *)((uint64_t *)o.x + f6_act_word(nst, r0, c0 / 32 + blk, pt / 3, pt % 3) + 2 * q) = val;
+        uint64_t *dst = (uint64_t *)o.x + f6_act_word(nst, r0, c0 / 32 + blk, pt / 3, pt % 3) + 2 * q;
+        if (r0 + 2 * q + 1 < M) *(uint4 *)dst = val;
+        else *(uint2 *)dst = make_uint2(val.x, val.y);
     }
     // block scales: per stage, 16 rows × 4 fp16 = 128 contiguous bytes
     for (int pc = threadIdx.x; pc < (nblk / 4) * 8; pc += 64 * LNW) {
         const int sg = pc >> 3, q = pc & 7;
         if (r0 + 2 * q >= M) continue;
-        *(uint4 *)(o.d + scale_index(o.mp, r0 + 2 * q, c0 / 32 + 4 * sg)) = *(const uint4 *)&stgd[sg][2 * q][0];
+        const uint4 val = *(const uint4 *)&stgd[sg][2 * q][0];
+        uint16_t *dst = o.d + scale_index(o.mp, r0 + 2 * q, c0 / 32 + 4 * sg);
+        if (r0 + 2 * q + 1 < M) *(uint4 *)dst = val;
+        else *(uint2 *)dst = make_uint2(val.x, val.y);
     }
 }
 

@@ -69,6 +69,23 @@ def test_large_values_at_the_end_of_a_row(ctx, t, M, N, K, at, value):
         assert np.isfinite(got).all() and orc.rel_l2(got, orc.mul_mat(t, wb, N, K, X)) <= 1e-6
 
 
+@pytest.mark.parametrize("M", [1, 15, 16, 63, 65])
+@pytest.mark.parametrize("K", [128, 1152])
+def test_fp6_conversion_leaves_rows_past_m(ctx, M, K):
+    X = np.random.default_rng(M + K).standard_normal((M, K)).astype(np.float32)
+    Mt, Mp, G = (M + 63) // 64 * 64, (M + 127) // 128 * 128, K // 128
+    q, d = np.full(3 * Mt * K // 2, 0xA5, np.uint8), np.full(G * Mp * 4, 0xA5A5, np.uint16)
+    qd, dd = ctx.to_device(q), ctx.to_device(d)
+    print(M, K, flush=True)
+    ctx.quantize_rows(s3e.TYPE_Q8_0_F6X2, ctx.to_device(X), M, K, qd, dd, None)
+    ctx.sync()
+    words = qd.download(np.uint64, (Mt // 64, G, 4, 2, 3, 64)).transpose(0, 5, 1, 2, 3, 4).reshape(Mt, -1)
+    scales = dd.download(np.uint16, (G, Mp, 4)).transpose(1, 0, 2).reshape(Mp, -1)
+    assert (words[M:] == 0xA5A5A5A5A5A5A5A5).all() and (scales[M:] == 0xA5A5).all()
+    want = np.abs(X.reshape(M, -1, 32)).max(-1) / np.float32(127)
+    assert np.array_equal(scales[:M].view(np.float16), want.astype(np.float16))
+
+
 @pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("M,N,K,shift", [(1, 256, 256, 0), (7, 256, 256, 0), (64, 256, 256, 0), (16, 96, 160, 0), (16, 160, 96, 0),
                                          (33, 256, 256, 5000), (200, 256, 256, 0)])
