@@ -111,7 +111,7 @@ int s3e_weight_info(const s3e_weight *w, int64_t out[4]);
  * with s3e_flash_attn_ext, as large as the largest call so far (freed with the
  * context); a call that needs more than 1 GiB allocates for itself.  Calls
  * that convert wait for their result before they return.  Products above 64
- * rows with few output tiles add up K in ranges whose partial sums take a 25 MB
+ * rows (F32: of any) with few output tiles add up K in ranges whose partial sums take a 25 MB
  * workspace made with the context (a context that found no memory for it, and
  * a product captured into a graph, sum K in one range, equal up to fp32
  * summation order). */

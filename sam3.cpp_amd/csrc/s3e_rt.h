@@ -24,7 +24,7 @@ struct s3e_ctx {
     // this device's copy of the allocation-free entry points' scratch array
     void *scratch = nullptr;
     // partial sums of products of at most 64 rows split over K across work-groups
-    // (captured products hold its address), and of larger ones
+    // (captured products hold its address), and of those on the tiled kernels
     float *sk_part = nullptr;
     int64_t sk_part_cap = 0;
     float *tile_part = nullptr;

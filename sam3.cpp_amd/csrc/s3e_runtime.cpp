@@ -280,7 +280,7 @@ std::vector<float> sinusoidal_pe_2d(int H, int W, int d) {
 // ---------------------------------------------------------------------------
 namespace {
 
-// The context's workspace for the partial sums of products above 64 rows (a
+// The context's workspace for the partial sums of products on the tiled kernels (a
 // split product has fewer than 768 tile × range pairs), made with the context
 // so that no product allocates.  Without the memory for it they run unsplit.
 // (Relaxed capture mode: another stream's capture may be open.)
