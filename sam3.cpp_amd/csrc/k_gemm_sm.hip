@@ -183,7 +183,7 @@ __global__ __launch_bounds__(64 * SM_WAVES, 2) void k_gemm_sm(SmArgs p) {
                 for (int j = 0; j < 4; j++) {
                     const bool in = (4 * s + j) * QK < G.K;
                     const float *v = (const float *)&f.x[i][4 * j];
-                    float amax = 0.f;
+                    float amax = __builtin_nanf("");  // (max passes over NaN: NaN where all of the block is)
 #pragma unroll
                     for (int k = 0; k < 16; k++) amax = fmaxf(amax, fabsf(v[k]));
                     amax = half_max(amax);

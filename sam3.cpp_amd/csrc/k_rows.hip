@@ -225,7 +225,8 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
             if (64 * it >= nseg) break;  // whole wave past the row
             // both lanes of a block are inside the row or both past it (nseg is even)
             if (seg >= nseg) continue;
-            float amax = 0.f;
+            // (max passes over NaN; a converted block that is all NaN has scale NaN, as in emit4)
+            float amax = NORM ? 0.f : __builtin_nanf("");
 #pragma unroll
             for (int j4 = 0; j4 < 4; j4++) {
                 float wv[4] = {1.f, 1.f, 1.f, 1.f}, bv[4] = {0.f, 0.f, 0.f, 0.f};

@@ -69,6 +69,26 @@ def test_large_values_at_the_end_of_a_row(ctx, t, M, N, K, at, value):
         assert np.isfinite(got).all() and orc.rel_l2(got, orc.mul_mat(t, wb, N, K, X)) <= 1e-6
 
 
+@pytest.mark.parametrize("t", [orc.Q4_0, orc.Q4_1, orc.Q8_0])
+@pytest.mark.parametrize("M,N,K", [(1, 33, 32), (16, 96, 224), (64, 64, 256), (65, 96, 256)])
+def test_blocks_of_nan_stay_nan(ctx, t, M, N, K):
+    # single values that are not numbers are passed over, as ggml's maximum does; a block of nothing else is not
+    _, X, _, w = _inputs(ctx, t, M, N, K, M + K)
+    X[0, K - 32 :] = np.nan
+    X[M // 2, 3] = np.nan
+    Xd, Y0, Y = ctx.to_device(X), ctx.buffer(M * N * 4), ctx.buffer(M * N * 4)
+    planes = (K + 127) // 128 * 4 * ((M + 127) // 128 * 128) * 2
+    q, d, s = ctx.buffer(M * K * 2), ctx.buffer(planes), ctx.buffer(planes)
+    print(t, M, N, K, flush=True)
+    ctx.quantize_rows(VDT[t], Xd, M, K, q, d, s)
+    ctx.mul_mat_q(w, q, d, s, M, Y0)
+    ctx.mul_mat(w, Xd, M, Y)
+    ctx.sync()
+    got, want = Y.download(np.float32, (M, N)), Y0.download(np.float32, (M, N))
+    assert np.isnan(got[0]).all() and np.isfinite(got[1:]).all()
+    assert np.array_equal(got, want, equal_nan=True)
+
+
 @pytest.mark.parametrize("M", [1, 15, 16, 63, 65])
 @pytest.mark.parametrize("K", [128, 1152])
 def test_fp6_conversion_leaves_rows_past_m(ctx, M, K):
