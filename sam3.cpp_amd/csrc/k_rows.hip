@@ -252,16 +252,20 @@ __global__ __launch_bounds__(64 * LNW) void k_layernorm_f6(const float *__restri
             // codes, slots 16-31 its l codes, so result dwords 0-2 are its 96
             // bits of the h string and dwords 3-5 its 96 bits of the l string
             f32x16 ev, od;
+            auto split = [&](auto big) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                float a, c, e, g;
-                f6_split<!NORM>(v[it][2 * i], id, a, c);
-                f6_split<!NORM>(v[it][2 * i + 1], id, e, g);
-                ev[i] = a;
-                od[i] = e;
-                ev[8 + i] = c;
-                od[8 + i] = g;
-            }
+                for (int i = 0; i < 8; i++) {
+                    float a, c, e, g;
+                    f6_split<!NORM, decltype(big)::value>(v[it][2 * i], id, a, c);
+                    f6_split<!NORM, decltype(big)::value>(v[it][2 * i + 1], id, e, g);
+                    ev[i] = a;
+                    od[i] = e;
+                    ev[8 + i] = c;
+                    od[8 + i] = g;
+                }
+            };
+            if (!NORM && __any(__builtin_isinf(id))) split(std::bool_constant<!NORM>{});
+            else split(std::false_type{});
             const u32x6 r6 = pack_bf6(ev, od);
             const int blk = seg >> 1;
             // LDS word of (block, part p, word t, row rr): blk·98 + (3p + t)·16 + rr

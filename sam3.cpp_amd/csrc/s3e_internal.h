@@ -488,14 +488,22 @@ __device__ __forceinline__ u32x6 pack_bf6(const f32x16 &even, const f32x16 &odd)
 
 // q = round-half-even(v·id) as a float, split q = 16·h + l with
 // h = ⌊(q + 8) / 16⌋, l = q − 16·h (f6_hi); every step is exact.
-// GUARD: a product that is not a number (v, or an infinite v against id = 0) is
-// code 0, as the integer conversion has it.
-template <bool GUARD = false>
+// GUARD: byte for byte what the integer conversion gives.  A product that is not
+// a number (v, or an infinite v against id = 0) is code 0, and so is −0; with
+// BIG, an infinite one (id, for a block whose maximum is below 127 / FLT_MAX) is
+// −1 or, below zero, 0: h = −0 and l that code.
+template <bool GUARD = false, bool BIG = false>
 __device__ __forceinline__ void f6_split(float v, float id, float &h, float &l) {
     float q = __builtin_rintf(v * id);
-    if constexpr (GUARD) q = q == q ? q : 0.f;
+    if constexpr (GUARD) q = (q == q ? q : 0.f) + 0.f;
     h = __builtin_floorf((q + 8.f) * 0.0625f);
     l = __builtin_fmaf(-16.f, h, q);
+    if constexpr (BIG) {
+        if (__builtin_isinf(q)) {
+            h = -0.f;
+            l = q > 0.f ? -1.f : 0.f;
+        }
+    }
 }
 
 // Write 4 consecutive values (columns col..col+3, col % 4 == 0) in the

@@ -69,6 +69,35 @@ def test_large_values_at_the_end_of_a_row(ctx, t, M, N, K, at, value):
         assert np.isfinite(got).all() and orc.rel_l2(got, orc.mul_mat(t, wb, N, K, X)) <= 1e-6
 
 
+@pytest.mark.parametrize("M,K", [(1, 128), (33, 640), (66, 2176)])
+def test_fp6_codes_are_the_int8_codes(ctx, M, K):
+    # E3M2 codes of q = 16·h + l, h = (q + 8) >> 4: no negative zeros, whatever the values
+    rng = np.random.default_rng(K)
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    X[0, 32:64] = np.where(np.arange(32) % 2, -1e-40, 1e-40)  # 127 / maximum is infinite: every code of it
+    X[-1, 5], X[-1, 70], X[-1, 96:] = np.nan, np.inf, 0
+    Mt, planes = (M + 63) // 64 * 64, (K + 127) // 128 * 4 * ((M + 127) // 128 * 128) * 2
+    q6, q8, d6, d8 = ctx.buffer(3 * Mt * K // 2), ctx.buffer(M * K), ctx.buffer(planes), ctx.buffer(planes)
+    Xd = ctx.to_device(X)
+    print(M, K, flush=True)
+    ctx.quantize_rows(s3e.TYPE_Q8_0_F6X2, Xd, M, K, q6, d6, None)
+    ctx.quantize_rows(s3e.TYPE_Q8_0, Xd, M, K, q8, d8, None)
+    ctx.sync()
+    words = q6.download(np.uint64, (Mt // 64, K // 128, 4, 2, 3, 64)).transpose(0, 5, 1, 2, 3, 4)  # row, stage, block, part, word
+    bits = np.unpackbits(np.ascontiguousarray(words).view(np.uint8).reshape(Mt, K // 32, 2, 24), axis=-1, bitorder="little")
+    code = (bits.reshape(Mt, K // 32, 2, 32, 6) << np.arange(6)).sum(-1)[:M]
+    value = np.array([0, 1, 2, 3, 4, 5, 6, 7, 8], np.int64)
+    table = np.full(64, 99, np.int64)
+    table[[0, 12, 16, 18, 20, 21, 22, 23, 24]] = value
+    table[[44, 48, 50, 52, 53, 54, 55, 56]] = -value[1:]
+    want = q8.download(np.int8, (M, K)).astype(np.int64).reshape(M, K // 32, 32)
+    tiny = np.zeros(want.shape, bool)
+    tiny[0, 1] = True
+    got = 16 * table[code[:, :, 0]] + table[code[:, :, 1]]
+    assert np.array_equal(got[~tiny], want[~tiny])
+    assert set(want[tiny]) == {-1, 0} and np.array_equal(table[code[:, :, 1]][tiny], want[tiny]) and (code[:, :, 0][tiny] == 32).all()
+
+
 @pytest.mark.parametrize("t", [orc.Q4_0, orc.Q4_1, orc.Q8_0])
 @pytest.mark.parametrize("M,N,K", [(1, 33, 32), (16, 96, 224), (64, 64, 256), (65, 96, 256)])
 def test_blocks_of_nan_stay_nan(ctx, t, M, N, K):
