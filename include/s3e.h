@@ -232,8 +232,8 @@ int s3e_flash_attn_ext(s3e_ctx *ctx,
  * shapes and output as s3e_flash_attn_ext, q/k/v as IEEE fp16 bits, computed
  * at S3E_PREC_DEFAULT (fp16 operands and probabilities, fp32 accumulation).
  * Q is read in place by its strides.  K and V are read in place when D and
- * their strides are multiples of 8 and they are 16-byte aligned, else copied to
- * [B][nh][N][64, 128 or 256], zero-padded; at D = 256 V is transposed into the
+ * their strides are multiples of 8 and they are 16-byte aligned (V's rows at
+ * least D apart), else copied to [B][nh][N][64, 128 or 256], zero-padded; at D = 256 V is transposed into the
  * engine's layout by one pass.  Asynchronous on the context's stream: O is complete after
  * s3e_ctx_sync.  The copies live in a context-owned workspace that a call
  * grows (synchronising the stream, then hipMalloc) only when it needs more

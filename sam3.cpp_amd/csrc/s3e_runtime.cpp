@@ -986,12 +986,14 @@ extern "C" int s3e_flash_attn_ext_f16(s3e_ctx *ctx, const uint16_t *q, const int
     // K and V are read where they lie when whole 16-byte chunks can be moved
     // (D and the strides multiples of 8, 16-byte aligned), else copied to
     // [BH][Nkv][hdp]; Q is read by strides of any kind, and head dim 256 takes
-    // V through the Vᵀ layout
+    // V through the Vᵀ layout.  V's rows must not overlap either: rows past the
+    // keys read as zeros because they lie behind the last one (an infinite value
+    // of a repeated row would meet their probability 0 and make NaN)
     auto in_place = [&](const void *x, const int64_t nb[4]) {
         return D % 8 == 0 && (uintptr_t)x % 16 == 0 && nb[1] % 8 == 0 && nb[2] % 8 == 0 && nb[3] % 8 == 0 &&
                nb[1] <= ATTN_MAX_ROW;
     };
-    const bool k_in = in_place(k, k_nb), v_t = hdp == 256, v_in = !v_t && in_place(v, v_nb);
+    const bool k_in = in_place(k, k_nb), v_t = hdp == 256, v_in = !v_t && in_place(v, v_nb) && v_nb[1] >= D;
     const int64_t ldv = vt_ld_for(Nkv);
     const AttnSplit sp(BH, Nq, Nkv, hdp);
     const size_t ob = (size_t)(BH * Nq * D) * 4;

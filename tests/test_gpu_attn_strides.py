@@ -99,6 +99,24 @@ def test_repeated_rows_by_zero_stride(ctx):
     assert np.linalg.norm(got - v.astype(np.float32)) <= 2e-3 * 3 * np.linalg.norm(v.astype(np.float32))
 
 
+@pytest.mark.parametrize("step", [0, 8])
+def test_infinite_value_in_overlapping_rows(ctx, step):
+    # rows of V closer than D: the padding keys of the last tile must not read one of them
+    rng = np.random.default_rng(3)
+    D, Nq, Nkv = 64, 5, 37
+    q, k = (rng.standard_normal((n, D)).astype(np.float16) for n in (Nq, Nkv))
+    v = rng.standard_normal(Nkv * step + D).astype(np.float16)
+    v[(Nkv - 1) * step + 9] = np.inf  # channel 9 of the last row, and of those before it
+    O = ctx.buffer(Nq * D * 4)
+    print(step, flush=True)
+    ctx.flash_attn_ext_f16(ctx.to_device(q), (1, D, 0, 0), ctx.to_device(k), (1, D, 0, 0), ctx.to_device(v), (1, step, 0, 0), D, Nq,
+                           Nkv, 1, 1, 0.125, O)
+    ctx.sync()
+    got = O.download(np.float32, (Nq, D))
+    inf = np.array([np.isinf(v[d : d + (Nkv - 1) * step + 1 : max(step, 1)]).any() for d in range(D)])
+    assert (got[:, inf] == np.inf).all() and np.isfinite(got[:, ~inf]).all()
+
+
 @pytest.mark.parametrize("prec", ["f16", "default", "f32"])
 @pytest.mark.parametrize("D,B,nh,Nq,Nkv", [(64, 2, 3, 200, 100), (72, 1, 4, 129, 100), (256, 1, 2, 130, 100), (64, 1, 2, 130, 1000)])
 @pytest.mark.parametrize("where", ["q", "k", "v"])
