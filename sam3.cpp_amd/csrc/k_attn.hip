@@ -697,8 +697,10 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
             }
         } else if (out.kind == A_Q8_0 || out.kind == A_Q8_1) {
             // ggml quantize_row_q8_0/q8_1 of the 32 values d = dt*32 .. dt*32+31,
-            // split 16/16 between lanes l and l^32
-            float amax = 0.f;
+            // split 16/16 between lanes l and l^32.  A block that is all NaN
+            // has scale NaN at head dim 256 (as in emit4, which the memory
+            // attention's split passes go through) and 0 in the encoders
+            float amax = HD == 256 ? __builtin_nanf("") : 0.f;
 #pragma unroll
             for (int r = 0; r < 16; r++) amax = fmaxf(amax, fabsf(o[dt][r]));
             amax = fmaxf(amax, __shfl_xor(amax, 32, 64));

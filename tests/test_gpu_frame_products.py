@@ -94,6 +94,29 @@ def test_memory_attention_linear2_sums_in_ranges_of_512(ctx, tmpdir_session):
         assert (y[:, ::2] > 0.9).all() and (y[:, 1::2] < -0.9).all()
 
 
+@pytest.mark.parametrize("ft", ["q8_0", "q4_1", "f16"])
+@pytest.mark.parametrize("M", [12, 1200])
+def test_nan_key_reaches_every_output(ctx, tmpdir_session, ft, M):
+    # one memory token is NaN: with few keys (one range) as with many, no output hides it
+    path = os.path.join(str(tmpdir_session), f"ma_nan_{ft}.ggml")
+    s3e.synth_write_sam2(path, "hiera_t", img_size=64, ftype=ft, seed=13, std=0.05, random_affine=True, mem_attn_layers=1, embed_dim=32,
+                         stages=(1, 1, 1, 1), global_idx=(), window_spec=(4, 4, 2, 2), bkg=(2, 2))
+    N, rng = 25, np.random.default_rng(M)
+    prompt = rng.standard_normal((M, 64)).astype(np.float32)
+    curr, zero = ctx.to_device(rng.standard_normal((N, 256)).astype(np.float32)), ctx.to_device(np.zeros((max(M, N), 256), np.float32))
+    rope = ctx.to_device(np.tile(np.float32([1, 0]), (N, 128, 1)))
+    print(ft, M, flush=True)
+    with _state(ctx, path) as st:
+        for bad in (False, True):
+            if bad:
+                prompt[M // 2] = np.nan
+            out = ctx.buffer(N * 256 * 4)
+            st.mem_attn(curr, zero, N, ctx.to_device(prompt), zero, M, M, rope, None, out)
+            ctx.sync()
+            y = out.download(np.float32, (N, 256))
+            assert np.isnan(y).all() if bad else np.isfinite(y).all()
+
+
 def test_gelu_of_every_fp16_value(ctx, tmpdir_session):
     """fc1 + ggml_gelu of an F16 file, bit for bit ggml's fp16 table: every fp16 value below 16 in size, and values that
     round to ±10 from inside."""
