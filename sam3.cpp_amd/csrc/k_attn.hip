@@ -175,7 +175,7 @@ __device__ __forceinline__ float sub_hi_half(float p, uint32_t h2) {
 
 // CROP: the windowed, cropped output mapping and narrower real heads
 // (a.wo, a.hd_out; the Hiera layouts), kept out of the plain variants.
-// STR: Q and K (and V, VN) by strides.
+// STR: Q and K (and V, VN) by strides; without, contiguous.
 // HR: channels that take part, the real head dim rounded up to whole MFMA
 // tiles (heads of 65 to 96 channels lie in rows of 128 and skip the last
 // quarter: its K chunks, Vᵀ rows, operand reads and MFMAs).
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
     // 10.9 ms), nor the cropped ones, whose few tiles do not repay the code.
     constexpr bool PAIRS = !SPLIT && ((HD == 64 && !CROP) || HD == 256);
     constexpr int NP = SPLIT ? 2 : 1;  // planes: hi (and lo)
-    static_assert(VN ? STR && HD <= 128 : !STR || HD == 256, "natural V at head dim 64 or 128, by strides");
+    static_assert(VN ? HD <= 128 && (STR || !SPLIT) : !STR || HD == 256, "natural V at head dim 64 or 128");
     constexpr int KPL = G::KPL, VPL = G::VPL;
     constexpr int KBUF = NP * KPL, VBUF = NP * VPL;
     // K ring (2 tiles) then Vᵀ ring (2 tiles)
@@ -208,10 +208,13 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         const int64_t off = (int64_t)(bh / a.NH) * a.qs[2] + (int64_t)(bh % a.NH) * a.qs[1] +
                             (int64_t)(qvalid ? qi : 0) * a.qs[0];
         const int dr = a.hd_out > 0 ? a.hd_out : HD;
+        // one loop per form, so that a work-group jumps over the others' code
+        // once and not once per step (fp16, 1024 work-groups of 12 queries × 12 keys at
+        // head dim 128: 10.5 → 9.8 µs a call)
+        if (a.q32) {
 #pragma unroll
-        for (int ds = 0; ds < DS; ds++) {
-            const int d0 = ds * 16 + lh * 8;
-            if (a.q32) {
+            for (int ds = 0; ds < DS; ds++) {
+                const int d0 = ds * 16 + lh * 8;
                 // (the head dim is a multiple of 4: four channels are all real or all padding)
                 float x[8];
 #pragma unroll
@@ -232,17 +235,25 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
                     qf[0][ds][i] = hv;
                     if constexpr (SPLIT) qf[NP - 1][ds][i] = (_Float16)(x[i] - (float)hv);
                 }
-            } else if constexpr (!SPLIT) {
-                const _Float16 *src = a.q + off + d0;
-                v8h z = {};
-                if (a.q_vec) {
-                    if (qvalid && d0 < dr) z = *(const v8h *)src;
-                } else {
+            }
+        } else if constexpr (!SPLIT) {
+            if (a.q_vec) {
+#pragma unroll
+                for (int ds = 0; ds < DS; ds++) {
+                    const int d0 = ds * 16 + lh * 8;
+                    const v8h z = {};
+                    qf[0][ds] = qvalid && d0 < dr ? *(const v8h *)(a.q + off + d0) : z;
+                }
+            } else {
+#pragma unroll
+                for (int ds = 0; ds < DS; ds++) {
+                    const int d0 = ds * 16 + lh * 8;
+                    v8h z = {};
 #pragma unroll
                     for (int i = 0; i < 8; i++)
-                        if (qvalid && d0 + i < dr) z[i] = src[i];
+                        if (qvalid && d0 + i < dr) z[i] = a.q[off + d0 + i];
+                    qf[0][ds] = z;
                 }
-                qf[0][ds] = z;
             }
         }
     } else {
@@ -265,7 +276,7 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
 #pragma unroll
         for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
 
-    int64_t koff = (int64_t)bh * a.Nkv * HD, voff = (int64_t)bh * HD * ldv;
+    int64_t koff = (int64_t)bh * a.Nkv * HD, voff = VN ? koff : (int64_t)bh * HD * ldv;
     // bytes from one K (V) row to the next, and of a row's real channels
     int k_rb = G::ROWK, v_rb = G::ROWK, real = 2 * HR;
     if constexpr (STR) {
@@ -835,7 +846,7 @@ hipError_t launch_attn(const AttnArgs &a, hipStream_t st) {
             if (st3[0] < 0 || st3[0] > ATTN_MAX_ROW || st3[0] % 8 || st3[1] % 8 || st3[2] % 8) return hipErrorInvalidValue;
         for (const void *ptr : {(const void *)a.k, (const void *)a.v, (const void *)a.k_lo, (const void *)a.v_lo})
             if ((uintptr_t)ptr % 16 != 0) return hipErrorInvalidValue;
-    } else if (a.v || a.q32) {
+    } else if (a.q32 || (a.v && (!a.q || a.k_lo || hd > 128 || crop))) {
         return hipErrorInvalidValue;
     }
     if (a.v) {
@@ -844,7 +855,13 @@ hipError_t launch_attn(const AttnArgs &a, hipStream_t st) {
             else if (hd == 64) hipLaunchKernelGGL((k_attn<true, 64, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
             else if (hd96) hipLaunchKernelGGL((k_attn<true, 128, true, true, true, 96>), grid, dim3(NTHR), 0, st, a, ldv);
             else hipLaunchKernelGGL((k_attn<true, 128, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
-        } else if (hd == 64 && !crop) hipLaunchKernelGGL((k_attn<false, 64, false, true>), grid, dim3(NTHR), 0, st, a, ldv);
+        }
+        // (contiguous fp16 tensors: the strides cost a work-group of few keys more
+        // than its tiles; 1024 of 18 × 35 8.0 → 7.3 µs a call, of 12 × 12 at head
+        // dim 128 9.8 → 9.0, 16 heads of 2000 × 2000 37.5 → 36.7)
+        else if (a.kv_d == 0 && hd == 64) hipLaunchKernelGGL((k_attn<false, 64, false, true, false>), grid, dim3(NTHR), 0, st, a, ldv);
+        else if (a.kv_d == 0) hipLaunchKernelGGL((k_attn<false, 128, true, true, false>), grid, dim3(NTHR), 0, st, a, ldv);
+        else if (hd == 64 && !crop) hipLaunchKernelGGL((k_attn<false, 64, false, true>), grid, dim3(NTHR), 0, st, a, ldv);
         else if (hd == 64) hipLaunchKernelGGL((k_attn<false, 64, true, true>), grid, dim3(NTHR), 0, st, a, ldv);
         else if (hd96) hipLaunchKernelGGL((k_attn<false, 128, true, true, true, 96>), grid, dim3(NTHR), 0, st, a, ldv);
         else hipLaunchKernelGGL((k_attn<false, 128, true, true>), grid, dim3(NTHR), 0, st, a, ldv);

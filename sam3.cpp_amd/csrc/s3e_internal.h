@@ -249,7 +249,8 @@ struct AttnArgs {
     // q32 (q_vec: its rows allow 16-byte loads), K and V fp16 rows of kv_d
     // channels (a multiple of 8; zeros from there to hd), 16-byte aligned,
     // strides multiples of 8, rows at most ATTN_MAX_ROW apart.  Head dim 256
-    // takes Q and K so, and vt.  kv_d = 0: plain layouts and vt
+    // takes Q and K so, and vt.  kv_d = 0: plain layouts, with vt, or with v as
+    // [BH][Nkv][hd] (fp16, whole heads)
     const _Float16 *v = nullptr, *v_lo = nullptr;
     const float *q32 = nullptr;
     int64_t qs[3] = {0, 0, 0}, ks[3] = {0, 0, 0}, vs[3] = {0, 0, 0};

@@ -1022,7 +1022,9 @@ extern "C" int s3e_flash_attn_ext_f16(s3e_ctx *ctx, const uint16_t *q, const int
     const auto contiguous = [&](const int64_t nb[4], int64_t N) {
         return nb[1] == hdp && nb[2] == N * hdp && nb[3] == nh * N * hdp;
     };
-    if (v_t && a.q_vec && k_in && contiguous(q_nb, Nq) && contiguous(k_nb, Nkv)) a.kv_d = 0;
+    // the plain layouts: no strides to work out
+    if (D == hdp && a.q_vec && k_in && (v_t || (v_in && contiguous(v_nb, Nkv))) && contiguous(q_nb, Nq) && contiguous(k_nb, Nkv))
+        a.kv_d = 0;
     a.k = k_in ? (const _Float16 *)k : k16;
     set_strides(a.ks, k_in ? k_nb : plain);
     if (v_t) a.vt = v16;

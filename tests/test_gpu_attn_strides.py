@@ -76,6 +76,16 @@ def test_layouts(ctx, prec, D, B, nh, Nq, Nkv):
         assert err <= (2e-6 if prec == "f32" else 2e-3), (layouts, offs, err)
 
 
+@pytest.mark.parametrize("D,B,nh,Nq,Nkv", [(64, 2, 3, 1, 1), (64, 1, 2, 129, 1025), (64, 64, 4, 13, 33), (128, 3, 2, 130, 65),
+                                           (128, 1, 1, 32, 2000)])
+def test_contiguous_is_the_strided_result(ctx, D, B, nh, Nq, Nkv):
+    # contiguous heads leave the strides out of the kernel, and change nothing else
+    rng = np.random.default_rng(D + Nkv)
+    q, k, v = (rng.standard_normal((B, nh, n, D)) for n in (Nq, Nkv, Nkv))
+    plain, wide = (_run(ctx, q, k, v, "f16", (layout,) * 3, (0, 0, 0)) for layout in ("heads", "wide"))
+    assert np.array_equal(plain, wide)
+
+
 def test_padding_reads_nothing_of_the_next_head(ctx):
     # heads of 72 channels side by side run padded to 128: head 1's NaN must stay out of head 0
     rng = np.random.default_rng(1)
