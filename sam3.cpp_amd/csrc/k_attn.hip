@@ -208,35 +208,38 @@ __global__ __launch_bounds__(NTHR, HD == 64 ? 3 : (HD == 128 ? 2 : 1)) void k_at
         const int64_t off = (int64_t)(bh / a.NH) * a.qs[2] + (int64_t)(bh % a.NH) * a.qs[1] +
                             (int64_t)(qvalid ? qi : 0) * a.qs[0];
         const int dr = a.hd_out > 0 ? a.hd_out : HD;
-        // one loop per form, so that a work-group jumps over the others' code
-        // once and not once per step (fp16, 1024 work-groups of 12 queries × 12 keys at
-        // head dim 128: 10.5 → 9.8 µs a call)
-        if (a.q32) {
+        // fp16: one loop per form, so that a work-group jumps over the others' code
+        // once and not once per step (1024 work-groups of 12 queries × 12 keys at
+        // head dim 128: 10.5 → 9.8 µs a call).  Split: a branch a step (9 × 16 heads
+        // of 576²: 81.6 → 79.0 µs a call)
+        if (SPLIT || a.q32) {
 #pragma unroll
             for (int ds = 0; ds < DS; ds++) {
                 const int d0 = ds * 16 + lh * 8;
-                // (the head dim is a multiple of 4: four channels are all real or all padding)
-                float x[8];
+                if (a.q32) {
+                    // (the head dim is a multiple of 4: four channels are all real or all padding)
+                    float x[8];
 #pragma unroll
-                for (int h4 = 0; h4 < 8; h4 += 4) {
-                    const float *src = a.q32 + off + d0 + h4;
-                    const bool in = qvalid && d0 + h4 < dr;
-                    if (a.q_vec) {
-                        const float4 f = in ? *(const float4 *)src : make_float4(0.f, 0.f, 0.f, 0.f);
-                        x[h4] = f.x; x[h4 + 1] = f.y; x[h4 + 2] = f.z; x[h4 + 3] = f.w;
-                    } else {
+                    for (int h4 = 0; h4 < 8; h4 += 4) {
+                        const float *src = a.q32 + off + d0 + h4;
+                        const bool in = qvalid && d0 + h4 < dr;
+                        if (a.q_vec) {
+                            const float4 f = in ? *(const float4 *)src : make_float4(0.f, 0.f, 0.f, 0.f);
+                            x[h4] = f.x; x[h4 + 1] = f.y; x[h4 + 2] = f.z; x[h4 + 3] = f.w;
+                        } else {
 #pragma unroll
-                        for (int i = 0; i < 4; i++) x[h4 + i] = in ? src[i] : 0.f;
+                            for (int i = 0; i < 4; i++) x[h4 + i] = in ? src[i] : 0.f;
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const _Float16 hv = to_half(x[i]);
+                        qf[0][ds][i] = hv;
+                        if constexpr (SPLIT) qf[NP - 1][ds][i] = (_Float16)(x[i] - (float)hv);
                     }
                 }
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const _Float16 hv = to_half(x[i]);
-                    qf[0][ds][i] = hv;
-                    if constexpr (SPLIT) qf[NP - 1][ds][i] = (_Float16)(x[i] - (float)hv);
-                }
             }
-        } else if constexpr (!SPLIT) {
+        } else {
             if (a.q_vec) {
 #pragma unroll
                 for (int ds = 0; ds < DS; ds++) {
